@@ -58,27 +58,23 @@ struct BvhObject
     DeviceBuffer codes;        // n u64, input order
     DeviceBuffer keysA, keysB; // n u64
     DeviceBuffer valsA, valsB; // n u32
-    DeviceBuffer hist;         // 256 * radix blocks u32
+    DeviceBuffer hist;         // 256 * (radix tiles + 1) u32
     DeviceBuffer scanScratch;
     DeviceBuffer boundsPartials; // 6 doubles per block + 6 final
     DeviceBuffer children;     // (n-1) * 2 u32
-    DeviceBuffer parents;      // (2n-1) u32
     DeviceBuffer rangeFirst;   // (n-1) u32
     DeviceBuffer rangeLast;    // (n-1) u32
     DeviceBuffer nodeBounds;   // (2n-1) * 6 f32
-    DeviceBuffer depthA, depthB, jumpA, jumpB; // (2n-1) u32: node depths by pointer jumping
-    DeviceBuffer levelHist;    // per-depth counts, then offsets and cursors
-    DeviceBuffer levelOrder;   // (n-1) internal nodes grouped by depth
-    DeviceBuffer expansion;    // max(1,n-1) * 8 u32
+    DeviceBuffer treeLists;    // subtrees that a run of the hierarchy leaves to the next launch
+    DeviceBuffer expansion;    // 8 u32 per node of the queue: its children, with open bits
     DeviceBuffer expandInfo;   // max(1,n-1) uint4: children with open bits, their half areas
     DeviceBuffer isNode8;      // max(1,n-1) u32
     DeviceBuffer node8Index;   // max(1,n-1) u32
-    DeviceBuffer frontier[ 2 ];
-    DeviceBuffer levelCounts;  // BVH_MAX_LEVELS + 2 u32 (last two: node count, error flag)
+    DeviceBuffer queue;        // max(1,n-1) u32: the binary nodes that became 8-wide ones, level by level
+    DeviceBuffer levelCounts;  // BVH_MAX_LEVELS + 1 u32 each: nodes per level, first node of each level
     DeviceBuffer nodes;        // nodeCount * stride
     DeviceBuffer nodes32;      // FP32 nodes an FP16 build converts from
     uint32_t*    hostCounts = nullptr; // pinned
-    uint32_t*    hostLevels = nullptr; // pinned per-depth node counts
     // batched build: per-scene offsets, binary and 8-wide roots, bounds
     uint32_t                sceneCount = 0;
     DeviceBuffer            sceneOffsets, sceneRoots, sceneRoots8, sceneBounds, scenePartials;
@@ -93,10 +89,6 @@ struct BvhObject
         if( hostCounts )
         {
             ( void )hipHostFree( hostCounts );
-        }
-        if( hostLevels )
-        {
-            ( void )hipHostFree( hostLevels );
         }
     }
 

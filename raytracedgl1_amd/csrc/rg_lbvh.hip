@@ -1,7 +1,6 @@
 // Linear BVH build for gfx950: FP64 bounds and Morton quantisation, stable
-// LSD radix sort with wave-ballot ranking, Karras (2012) hierarchy, bottom-up
-// refit with agent-scope acquire/release counters, and a deterministic
-// collapse into 8-wide nodes.
+// LSD radix sort with wave-ballot ranking, the Karras (2012) hierarchy joined
+// bottom-up with its boxes, and a deterministic collapse into 8-wide nodes.
 //
 // This replaces the driver-side acceleration-structure build of the reference
 // (ASBuilder::BuildBottomLevel / BuildTopLevel, Source/ASBuilder.cpp:141-206);
@@ -20,7 +19,7 @@ namespace
 {
 
 constexpr int      THREADS     = 256;
-constexpr int      RS_ITEMS    = 16;
+constexpr int      RS_ITEMS    = 8;
 constexpr int      RS_TILE     = THREADS * RS_ITEMS;
 constexpr uint32_t MORTON_BITS = 21;
 constexpr double   MORTON_CELLS = 2097152.0; // 2^21
@@ -364,16 +363,19 @@ __global__ void k_segment_boxes( const BvhNode8* nodes, const float4* sortedTris
 }
 
 // --------------------------------------------------------- radix sort
+// One pass = three launches: digit counts per tile, one block per digit that
+// scans its counts over the tiles, and the scatter.
 
 __global__ __launch_bounds__( THREADS ) void k_radix_hist( const uint64_t* keys, uint32_t n, int shift, uint32_t* hist, uint32_t numBlocks )
 {
     __shared__ uint32_t cnt[ 256 ];
     cnt[ threadIdx.x ] = 0;
     __syncthreads();
-    const uint64_t base = uint64_t( blockIdx.x ) * RS_TILE;
+    const uint32_t base = blockIdx.x * RS_TILE;
+#pragma unroll
     for( int k = 0; k < RS_ITEMS; k++ )
     {
-        uint64_t i = base + uint64_t( k ) * THREADS + threadIdx.x;
+        const uint32_t i = base + k * THREADS + threadIdx.x;
         if( i < n )
         {
             atomicAdd( &cnt[ uint32_t( keys[ i ] >> shift ) & 255u ], 1u );
@@ -383,8 +385,71 @@ __global__ __launch_bounds__( THREADS ) void k_radix_hist( const uint64_t* keys,
     hist[ threadIdx.x * numBlocks + blockIdx.x ] = cnt[ threadIdx.x ];
 }
 
-// Stable scatter: keys of a tile are ranked in (round, thread) order, which is
-// their input order; equal digits are ranked within a wave by ballot matching.
+// Inclusive sum over a wave.
+__device__ __forceinline__ uint32_t WaveInclusive( uint32_t v, int lane )
+{
+#pragma unroll
+    for( int off = 1; off < 64; off <<= 1 )
+    {
+        const uint32_t o = __shfl_up( v, off, 64 );
+        v += lane >= off ? o : 0u;
+    }
+    return v;
+}
+
+// Exclusive sum over a block of THREADS; *total is the block's sum.
+__device__ __forceinline__ uint32_t BlockExclusive( uint32_t v, uint32_t* s_wave, uint32_t* total )
+{
+    const int      lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t inc  = WaveInclusive( v, lane );
+    if( lane == 63 )
+    {
+        s_wave[ wave ] = inc;
+    }
+    __syncthreads();
+    uint32_t before = 0, sum = 0;
+#pragma unroll
+    for( int w = 0; w < THREADS / 64; w++ )
+    {
+        before += w < wave ? s_wave[ w ] : 0u;
+        sum += s_wave[ w ];
+    }
+    __syncthreads();
+    *total = sum;
+    return before + inc - v;
+}
+
+// Block d: the exclusive sums of digit d's counts over the tiles, in place,
+// and the digit's total.
+__global__ __launch_bounds__( THREADS ) void k_radix_scan( uint32_t* hist, uint32_t* totals, uint32_t numBlocks )
+{
+    __shared__ uint32_t s_wave[ THREADS / 64 ];
+    uint32_t*           h   = hist + size_t( blockIdx.x ) * numBlocks;
+    uint32_t            run = 0;
+    for( uint32_t base = 0; base < numBlocks; base += THREADS )
+    {
+        const uint32_t i = base + threadIdx.x;
+        const uint32_t v = i < numBlocks ? h[ i ] : 0u;
+        uint32_t       sum;
+        const uint32_t ex = BlockExclusive( v, s_wave, &sum );
+        if( i < numBlocks )
+        {
+            h[ i ] = run + ex;
+        }
+        run += sum;
+    }
+    if( threadIdx.x == 0 )
+    {
+        totals[ blockIdx.x ] = run;
+    }
+}
+
+// Stable scatter.  Each wave owns a run of the tile and ranks its keys item
+// by item (64 consecutive keys at a time, equal digits by ballot matching
+// over its own counters), so no barrier stands between items; the tile is
+// then ordered in LDS and written out digit by digit, in runs.  1M pairs:
+// 19 us with one barrier-separated round per 256 keys and scattered stores,
+// 11 us like this (24 MB moved).
 __global__ __launch_bounds__( THREADS ) void k_radix_scatter( const uint64_t* keysIn,
                                                               const uint32_t* valsIn,
                                                               uint64_t*       keysOut,
@@ -392,34 +457,46 @@ __global__ __launch_bounds__( THREADS ) void k_radix_scatter( const uint64_t* ke
                                                               uint32_t        n,
                                                               int             shift,
                                                               const uint32_t* offsets,
+                                                              const uint32_t* totals,
                                                               uint32_t        numBlocks )
 {
     constexpr int       WAVES = THREADS / 64;
-    __shared__ uint32_t s_base[ 256 ];
-    __shared__ uint32_t s_waveCnt[ WAVES ][ 256 ];
+    __shared__ uint32_t s_cnt[ WAVES ][ 256 ]; // per wave: counts, then first positions in the tile
+    __shared__ uint32_t s_out[ 256 ];          // global position of a digit's keys minus their position in the tile
+    __shared__ uint32_t s_wave[ WAVES ];
+    __shared__ uint64_t s_key[ RS_TILE ];
+    __shared__ uint32_t s_val[ RS_TILE ];
 
-    const int      tid  = threadIdx.x;
-    const int      lane = tid & 63;
-    const int      wave = tid >> 6;
+    const int      tid    = threadIdx.x;
+    const int      lane   = tid & 63;
+    const int      wave   = tid >> 6;
     const uint64_t ltMask = ( lane == 0 ) ? 0ull : ( ~0ull >> ( 64 - lane ) );
+    const uint32_t tile   = blockIdx.x * RS_TILE;
+    const uint32_t here   = n - tile < uint32_t( RS_TILE ) ? n - tile : uint32_t( RS_TILE );
 
-    s_base[ tid ] = offsets[ tid * numBlocks + blockIdx.x ];
+#pragma unroll
     for( int w = 0; w < WAVES; w++ )
     {
-        s_waveCnt[ w ][ tid ] = 0;
+        s_cnt[ w ][ tid ] = 0;
     }
     __syncthreads();
 
-    const uint64_t base = uint64_t( blockIdx.x ) * RS_TILE;
-    for( int round = 0; round < RS_ITEMS; round++ )
+    uint32_t* cnt = s_cnt[ wave ];
+    uint64_t           key[ RS_ITEMS ];
+    uint32_t           val[ RS_ITEMS ], rank[ RS_ITEMS ];
+#pragma unroll
+    for( int r = 0; r < RS_ITEMS; r++ )
     {
-        const uint64_t i     = base + uint64_t( round ) * THREADS + tid;
-        const bool     valid = i < n;
-        uint64_t       key   = valid ? keysIn[ i ] : 0ull;
-        uint32_t       val   = valid ? valsIn[ i ] : 0u;
-        uint32_t       digit = uint32_t( key >> shift ) & 255u;
-
-        uint64_t peers = __ballot( valid );
+        const uint32_t i = uint32_t( wave * RS_ITEMS + r ) * 64u + lane;
+        key[ r ]         = i < here ? keysIn[ tile + i ] : 0ull;
+        val[ r ]         = i < here ? valsIn[ tile + i ] : 0u;
+    }
+#pragma unroll
+    for( int r = 0; r < RS_ITEMS; r++ )
+    {
+        const bool     valid = uint32_t( wave * RS_ITEMS + r ) * 64u + lane < here;
+        const uint32_t digit = uint32_t( key[ r ] >> shift ) & 255u;
+        uint64_t       peers = __ballot( valid );
 #pragma unroll
         for( int b = 0; b < 8; b++ )
         {
@@ -427,258 +504,361 @@ __global__ __launch_bounds__( THREADS ) void k_radix_scatter( const uint64_t* ke
             const uint64_t m   = __ballot( bit );
             peers &= bit ? m : ~m;
         }
-        const uint32_t rank = __popcll( peers & ltMask );
-        if( valid && rank == 0 )
+        const uint32_t before = cnt[ digit ];
+        const uint32_t lower  = __popcll( peers & ltMask );
+        rank[ r ]             = before + lower;
+        // every lane has read before the first of its peers counts them
+        __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
+        __builtin_amdgcn_wave_barrier();
+        if( valid && lower == 0 )
         {
-            s_waveCnt[ wave ][ digit ] = __popcll( peers );
+            cnt[ digit ] = before + __popcll( peers );
         }
-        __syncthreads();
-        if( valid )
+        __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+
+    // thread d: digit d's first position in the tile, per wave, and in the output
+    uint32_t c[ WAVES ], sum = 0, all;
+#pragma unroll
+    for( int w = 0; w < WAVES; w++ )
+    {
+        c[ w ] = s_cnt[ w ][ tid ];
+        sum += c[ w ];
+    }
+    uint32_t       first = BlockExclusive( sum, s_wave, &all );
+    const uint32_t start = BlockExclusive( totals[ tid ], s_wave, &all );
+    s_out[ tid ]         = start + offsets[ size_t( tid ) * numBlocks + blockIdx.x ] - first;
+#pragma unroll
+    for( int w = 0; w < WAVES; w++ )
+    {
+        s_cnt[ w ][ tid ] = first;
+        first += c[ w ];
+    }
+    __syncthreads();
+#pragma unroll
+    for( int r = 0; r < RS_ITEMS; r++ )
+    {
+        if( uint32_t( wave * RS_ITEMS + r ) * 64u + lane < here )
         {
-            uint32_t pos = s_base[ digit ] + rank;
-            for( int w = 0; w < wave; w++ )
-            {
-                pos += s_waveCnt[ w ][ digit ];
-            }
-            keysOut[ pos ] = key;
-            valsOut[ pos ] = val;
+            const uint32_t pos = s_cnt[ wave ][ uint32_t( key[ r ] >> shift ) & 255u ] + rank[ r ];
+            s_key[ pos ]       = key[ r ];
+            s_val[ pos ]       = val[ r ];
         }
-        __syncthreads();
-        uint32_t add = 0;
-        for( int w = 0; w < WAVES; w++ )
+    }
+    __syncthreads();
+#pragma unroll
+    for( int r = 0; r < RS_ITEMS; r++ )
+    {
+        const uint32_t i = r * THREADS + tid;
+        if( i < here )
         {
-            add += s_waveCnt[ w ][ tid ];
-            s_waveCnt[ w ][ tid ] = 0;
+            const uint64_t k   = s_key[ i ];
+            const uint32_t out = s_out[ uint32_t( k >> shift ) & 255u ] + i;
+            keysOut[ out ]     = k;
+            valsOut[ out ]     = s_val[ i ];
         }
-        s_base[ tid ] += add;
-        __syncthreads();
     }
 }
 
-// ------------------------------------------------------------- Karras
+// ----------------------------------------------------------- hierarchy
+// The binary radix tree over the sorted keys (Karras 2012) with its boxes,
+// built bottom-up (Apetrei 2014): a subtree over the sorted range [l, r]
+// joins its left or its right neighbour, whichever shares the longer key
+// prefix with it, and of two siblings the one that is done last makes their
+// parent.  Node ids are Karras's: an internal node is the right end of its
+// range as a left child, the left end as a right child, 0 as the root;
+// leaf k is n - 1 + k.
+//
+// A block joins what lies within its own run of elements, with the meeting
+// points in LDS; the subtrees whose sibling lies outside go to a list, and
+// the next launch joins those of BUILD_LISTS lists.  Nothing is exchanged
+// between blocks of a launch, so no fence or atomic leaves the CU.  A run is
+// cut by at most two root paths, so its list holds at most two subtrees per
+// level of the tree (63 key bits and 28 index bits).
+// Bound by the latency of a run's climb and the 80 bytes written per node:
+// 135 us for 1M triangles in 5 launches, where separate kernels for the
+// topology, the depths by pointer jumping, a sort by depth and one union
+// launch per level took 345 us in 56.
+constexpr uint32_t BUILD_LIST_CAP = 192;
+constexpr uint32_t BUILD_LISTS    = 8;
 
-__device__ __forceinline__ int Delta( const uint64_t* keys, int64_t n, int64_t i, int64_t j )
+// Length of the prefix that sorted keys i and i + 1 share, equal keys by
+// their positions; -1 at the ends.
+__device__ __forceinline__ int PrefixAt( const uint64_t* keys, uint32_t n, int64_t i )
 {
-    if( j < 0 || j >= n )
+    if( i < 0 || i + 1 >= int64_t( n ) )
     {
         return -1;
     }
-    const uint64_t a = keys[ i ], b = keys[ j ];
-    if( a == b )
-    {
-        return 64 + __clz( uint32_t( i ) ^ uint32_t( j ) );
-    }
-    return __clzll( a ^ b );
+    const uint64_t x = keys[ i ] ^ keys[ i + 1 ];
+    return x ? __clzll( x ) : 64 + __clz( uint32_t( i ) ^ uint32_t( i + 1 ) );
 }
 
-// Internal node i of n-1; child ids >= n-1 denote leaves (sorted position id-(n-1)).
-__global__ __launch_bounds__( THREADS ) void k_karras( const uint64_t* keys,
-                                                       uint32_t        n,
-                                                       uint32_t*       children,
-                                                       uint32_t*       parents,
-                                                       uint32_t*       rangeFirst,
-                                                       uint32_t*       rangeLast )
-{
-    const int64_t i = int64_t( blockIdx.x ) * THREADS + threadIdx.x;
-    const int64_t N = n;
-    if( i >= N - 1 )
-    {
-        return;
-    }
-    const int d    = ( Delta( keys, N, i, i + 1 ) - Delta( keys, N, i, i - 1 ) ) >= 0 ? 1 : -1;
-    const int dmin = Delta( keys, N, i, i - d );
-
-    int64_t lmax = 2;
-    while( Delta( keys, N, i, i + lmax * d ) > dmin )
-    {
-        lmax <<= 1;
-    }
-    int64_t l = 0;
-    for( int64_t t = lmax >> 1; t >= 1; t >>= 1 )
-    {
-        if( Delta( keys, N, i, i + ( l + t ) * d ) > dmin )
-        {
-            l += t;
-        }
-    }
-    const int64_t j     = i + l * d;
-    const int     dnode = Delta( keys, N, i, j );
-
-    int64_t s = 0, t = l;
-    do
-    {
-        t = ( t + 1 ) >> 1;
-        if( Delta( keys, N, i, i + ( s + t ) * d ) > dnode )
-        {
-            s += t;
-        }
-    } while( t > 1 );
-
-    const int64_t gamma = i + s * d + ( d < 0 ? d : 0 );
-    const int64_t lo = i < j ? i : j, hi = i < j ? j : i;
-
-    const uint32_t left  = uint32_t( lo == gamma ? ( N - 1 ) + gamma : gamma );
-    const uint32_t right = uint32_t( hi == gamma + 1 ? ( N - 1 ) + gamma + 1 : gamma + 1 );
-
-    children[ i * 2 + 0 ] = left;
-    children[ i * 2 + 1 ] = right;
-    parents[ left ]       = uint32_t( i );
-    parents[ right ]      = uint32_t( i );
-    rangeFirst[ i ]       = uint32_t( lo );
-    rangeLast[ i ]        = uint32_t( hi );
-    if( i == 0 )
-    {
-        parents[ 0 ] = 0xFFFFFFFFu;
-    }
-}
-
-// --------------------------------------------------------------- refit
-
-__device__ __forceinline__ void StoreBox( float* b, v3 lo, v3 hi )
-{
-    b[ 0 ] = lo.x;
-    b[ 1 ] = lo.y;
-    b[ 2 ] = lo.z;
-    b[ 3 ] = hi.x;
-    b[ 4 ] = hi.y;
-    b[ 5 ] = hi.z;
-}
-
-// Level-synchronous refit: the depth of every binary node by pointer
-// jumping over the parent links (7 rounds reach depth 128), a counting sort
-// of the internal nodes by depth, then one launch per level from the deepest
-// up, each node the union of its two children.  No atomics on the boxes and
-// no cross-wave ordering: min/max unions give the same boxes in any order.
-constexpr int      REFIT_JUMP_ROUNDS = 7;
-constexpr uint32_t REFIT_MAX_DEPTH   = 128;
-
-__global__ __launch_bounds__( THREADS ) void k_leaf_boxes( const float* tris, const uint32_t* sortedIdx, uint32_t n, float* bounds )
-{
-    const uint32_t k = blockIdx.x * THREADS + threadIdx.x;
-    if( k >= n )
-    {
-        return;
-    }
-    v3 a, b, c;
-    LoadTri( tris, sortedIdx[ k ], a, b, c );
-    StoreBox( bounds + size_t( ( n - 1 ) + k ) * 6, vmin( vmin( a, b ), c ), vmax( vmax( a, b ), c ) );
-}
-
-// dist[i] = 1 and jump[i] = parent for every node but the root (0, itself)
-__global__ __launch_bounds__( THREADS ) void k_depth_init( const uint32_t* parents, uint32_t count, uint32_t* dist, uint32_t* jump )
-{
-    const uint32_t i = blockIdx.x * THREADS + threadIdx.x;
-    if( i >= count )
-    {
-        return;
-    }
-    const uint32_t p    = parents[ i ];
-    const bool     root = i == 0 || p == 0xFFFFFFFFu;
-    dist[ i ]           = root ? 0u : 1u;
-    jump[ i ]           = root ? 0u : p;
-}
-
-__global__ __launch_bounds__( THREADS ) void k_depth_jump( uint32_t count, const uint32_t* distIn, const uint32_t* jumpIn, uint32_t* distOut,
-                                                           uint32_t* jumpOut )
-{
-    const uint32_t i = blockIdx.x * THREADS + threadIdx.x;
-    if( i >= count )
-    {
-        return;
-    }
-    const uint32_t j = jumpIn[ i ];
-    distOut[ i ]     = distIn[ i ] + distIn[ j ];
-    jumpOut[ i ]     = jumpIn[ j ];
-}
-
-// Histogram of internal-node depths, privatised per block in LDS (one
-// global atomic per bin per block); counts[REFIT_MAX_DEPTH] flags a deeper
-// tree.  Also writes the (depth, node) pairs one radix pass groups by depth.
-__global__ __launch_bounds__( THREADS ) void k_depth_keys( uint32_t internal, const uint32_t* depth, uint32_t* counts, uint64_t* keys,
-                                                           uint32_t* vals )
-{
-    __shared__ uint32_t s[ REFIT_MAX_DEPTH + 1 ];
-    for( uint32_t b = threadIdx.x; b <= REFIT_MAX_DEPTH; b += THREADS )
-    {
-        s[ b ] = 0;
-    }
-    __syncthreads();
-    const uint32_t i = blockIdx.x * THREADS + threadIdx.x;
-    if( i < internal )
-    {
-        const uint32_t d = depth[ i ] < REFIT_MAX_DEPTH ? depth[ i ] : REFIT_MAX_DEPTH;
-        atomicAdd( &s[ d ], 1u );
-        keys[ i ] = d;
-        vals[ i ] = i;
-    }
-    __syncthreads();
-    for( uint32_t b = threadIdx.x; b <= REFIT_MAX_DEPTH; b += THREADS )
-    {
-        if( s[ b ] )
-        {
-            atomicAdd( &counts[ b ], s[ b ] );
-        }
-    }
-}
-
-__global__ __launch_bounds__( THREADS ) void k_refit_level( const uint32_t* order, uint32_t first, uint32_t count, const uint32_t* children,
-                                                            float* bounds )
-{
-    const uint32_t t = blockIdx.x * THREADS + threadIdx.x;
-    if( t >= count )
-    {
-        return;
-    }
-    const uint32_t node = order[ first + t ];
-    const float*   l    = bounds + size_t( children[ node * 2 + 0 ] ) * 6;
-    const float*   r    = bounds + size_t( children[ node * 2 + 1 ] ) * 6;
-    const v3       lo   = vmin( mk3( l[ 0 ], l[ 1 ], l[ 2 ] ), mk3( r[ 0 ], r[ 1 ], r[ 2 ] ) );
-    const v3       hi   = vmax( mk3( l[ 3 ], l[ 4 ], l[ 5 ] ), mk3( r[ 3 ], r[ 4 ], r[ 5 ] ) );
-    StoreBox( bounds + size_t( node ) * 6, lo, hi );
-}
-
-// ------------------------------------------------------------ collapse
-
-__device__ __forceinline__ float HalfArea( const float* b )
+__device__ __forceinline__ float HalfArea( const float b[ 6 ] )
 {
     const float dx = b[ 3 ] - b[ 0 ], dy = b[ 4 ] - b[ 1 ], dz = b[ 5 ] - b[ 2 ];
     return dx * dy + dy * dz + dz * dx;
 }
+
+constexpr uint32_t OPEN_BIT = 0x80000000u;
+
+struct TreeArgs
+{
+    const float*    tris;
+    const uint64_t* keys;      // sorted
+    const uint32_t* order;     // triangle of each sorted position
+    uint32_t        n;
+    uint32_t        leafMax;
+    uint2*          children;  // per internal node
+    uint32_t*       rangeFirst;
+    uint32_t*       rangeLast;
+    float*          bounds;    // 6 per node, internal then leaves
+    uint4*          info;      // per internal node: the collapse's record (below)
+    const uint2*    listIn;    // ranges of the subtrees of the launch before
+    const uint32_t* countIn;
+    uint32_t        lists;
+    uint2*          listOut;
+    uint32_t*       countOut;
+};
+
+// LEAVES: the elements are PER * THREADS sorted triangles, else the subtrees
+// of BUILD_LISTS lists.  The collapse's record of an internal node: its two
+// children, each with OPEN_BIT set when it may be opened (internal, more
+// than leafMax triangles), and their half areas (-1 for the others).
+template< bool LEAVES, int PER >
+__global__ __launch_bounds__( THREADS ) void k_tree( TreeArgs a )
+{
+    constexpr int       CAP = PER * THREADS;
+    static_assert( LEAVES || CAP >= int( BUILD_LISTS * BUILD_LIST_CAP ), "element capacity" );
+    __shared__ float    s_box[ 6 ][ CAP ];
+    __shared__ uint32_t s_first[ LEAVES ? 1 : CAP ], s_last[ LEAVES ? 1 : CAP ];
+    __shared__ uint32_t s_meet[ CAP ]; // between elements e and e + 1: 1 + the far end of the subtree that came first
+    __shared__ int8_t   s_prefix[ CAP + 1 ];
+    __shared__ uint32_t s_wave[ THREADS / 64 ];
+    constexpr uint32_t  TAKEN = 0xFFFFFFFFu;
+
+    const uint32_t tid = threadIdx.x, n = a.n, I = a.n - 1;
+    uint32_t       count = 0, base = 0;
+    if constexpr( LEAVES )
+    {
+        base  = blockIdx.x * CAP;
+        count = n - base < uint32_t( CAP ) ? n - base : uint32_t( CAP );
+    }
+    else
+    {
+        for( uint32_t k = 0; k < BUILD_LISTS; k++ )
+        {
+            const uint32_t list = blockIdx.x * BUILD_LISTS + k;
+            const uint32_t c    = list < a.lists ? a.countIn[ list ] : 0u;
+            if( tid < c )
+            {
+                const uint2 rng        = a.listIn[ size_t( list ) * BUILD_LIST_CAP + tid ];
+                s_first[ count + tid ] = rng.x;
+                s_last[ count + tid ]  = rng.y;
+            }
+            count += c;
+        }
+        __syncthreads();
+    }
+    auto first = [ & ]( uint32_t e ) { return LEAVES ? base + e : s_first[ LEAVES ? 0 : e ]; };
+    auto last  = [ & ]( uint32_t e ) { return LEAVES ? base + e : s_last[ LEAVES ? 0 : e ]; };
+    for( uint32_t e = tid; e < count; e += THREADS )
+    {
+        s_prefix[ e ] = int8_t( PrefixAt( a.keys, n, int64_t( first( e ) ) - 1 ) );
+        s_meet[ e ]   = 0u;
+    }
+    if( tid == 0 )
+    {
+        s_prefix[ count ] = int8_t( PrefixAt( a.keys, n, last( count - 1 ) ) );
+    }
+    __syncthreads();
+
+    // the subtrees at the run's ends (one at either at most): [endA, count) and [0, startB]
+    constexpr uint32_t NONE = 0xFFFFFFFFu;
+    uint32_t           endA = NONE, startB = NONE;
+    for( uint32_t e = tid; e < count; e += THREADS )
+    {
+        uint32_t A = e, B = e; // the subtree's elements
+        float    box[ 6 ];
+        if constexpr( LEAVES )
+        {
+            v3 p, q, r;
+            LoadTri( a.tris, a.order[ base + e ], p, q, r );
+            const v3 lo = vmin( vmin( p, q ), r ), hi = vmax( vmax( p, q ), r );
+            box[ 0 ] = lo.x, box[ 1 ] = lo.y, box[ 2 ] = lo.z, box[ 3 ] = hi.x, box[ 4 ] = hi.y, box[ 5 ] = hi.z;
+            float2* o = reinterpret_cast< float2* >( a.bounds + ( size_t( I ) + base + e ) * 6 );
+            o[ 0 ]    = make_float2( box[ 0 ], box[ 1 ] );
+            o[ 1 ]    = make_float2( box[ 2 ], box[ 3 ] );
+            o[ 2 ]    = make_float2( box[ 4 ], box[ 5 ] );
+        }
+        else
+        {
+            const uint32_t l = first( e ), r = last( e );
+            const uint32_t id = l == r ? I + l : ( s_prefix[ e + 1 ] > s_prefix[ e ] ? r : l );
+            const float2*  o  = reinterpret_cast< const float2* >( a.bounds + size_t( id ) * 6 );
+            const float2   x = o[ 0 ], y = o[ 1 ], z = o[ 2 ];
+            box[ 0 ] = x.x, box[ 1 ] = x.y, box[ 2 ] = y.x, box[ 3 ] = y.y, box[ 4 ] = z.x, box[ 5 ] = z.y;
+        }
+        while( true )
+        {
+            const int before = s_prefix[ A ], after = s_prefix[ B + 1 ];
+            if( before < 0 && after < 0 )
+            {
+                break; // the whole tree
+            }
+            const bool left = after > before;
+            if( left ? B + 1 == count : A == 0 )
+            {
+                if( left )
+                {
+                    endA = A;
+                }
+                else
+                {
+                    startB = B;
+                }
+                break; // its sibling is not in this run
+            }
+            const uint32_t at = left ? B : A; // where this subtree's box is kept; the sibling's is next to it
+#pragma unroll
+            for( int k = 0; k < 6; k++ )
+            {
+                s_box[ k ][ at ] = box[ k ];
+            }
+            __builtin_amdgcn_fence( __ATOMIC_RELEASE, "workgroup" );
+            const uint32_t meet = left ? B : A - 1;
+            const uint32_t far  = __hip_atomic_exchange( &s_meet[ meet ], 1u + ( left ? A : B ), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP );
+            if( far == 0u )
+            {
+                break; // the sibling goes on from here
+            }
+            __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "workgroup" );
+            s_meet[ meet ]    = TAKEN;
+            const uint32_t sA = left ? B + 1 : far - 1, sB = left ? far - 1 : A - 1;
+            const uint32_t sat = left ? sA : sB;
+            float          sib[ 6 ];
+#pragma unroll
+            for( int k = 0; k < 6; k++ )
+            {
+                sib[ k ] = s_box[ k ][ sat ];
+            }
+            // the children in order
+            const uint32_t lA = left ? A : sA, lB = left ? B : sB, rA = left ? sA : A, rB = left ? sB : B;
+            const uint32_t lf = first( lA ), ll = last( lB ), rf = first( rA ), rl = last( rB );
+            const uint32_t lid = lf == ll ? I + lf : ll, rid = rf == rl ? I + rf : rf;
+            const bool     lo = lf != ll && ll - lf + 1u > a.leafMax, ro = rf != rl && rl - rf + 1u > a.leafMax;
+            const float    areaOwn = HalfArea( box ), areaSib = HalfArea( sib );
+            const float    la = lo ? ( left ? areaOwn : areaSib ) : -1.0f, ra = ro ? ( left ? areaSib : areaOwn ) : -1.0f;
+#pragma unroll
+            for( int k = 0; k < 3; k++ )
+            {
+                const float x = left ? box[ k ] : sib[ k ], y = left ? sib[ k ] : box[ k ];
+                const float z = left ? box[ 3 + k ] : sib[ 3 + k ], w = left ? sib[ 3 + k ] : box[ 3 + k ];
+                box[ k ]      = fminf( x, y );
+                box[ 3 + k ]  = fmaxf( z, w );
+            }
+            A = lA;
+            B = rB;
+            const int      pb = s_prefix[ A ], pa = s_prefix[ B + 1 ];
+            const uint32_t id = pb < 0 && pa < 0 ? 0u : ( pa > pb ? rl : lf );
+            a.children[ id ]   = make_uint2( lid, rid );
+            a.rangeFirst[ id ] = lf;
+            a.rangeLast[ id ]  = rl;
+            float2* o          = reinterpret_cast< float2* >( a.bounds + size_t( id ) * 6 );
+            o[ 0 ]             = make_float2( box[ 0 ], box[ 1 ] );
+            o[ 1 ]             = make_float2( box[ 2 ], box[ 3 ] );
+            o[ 2 ]             = make_float2( box[ 4 ], box[ 5 ] );
+            a.info[ id ] = make_uint4( lid | ( lo ? OPEN_BIT : 0u ), rid | ( ro ? OPEN_BIT : 0u ), __float_as_uint( la ), __float_as_uint( ra ) );
+        }
+    }
+    __syncthreads();
+    if( gridDim.x == 1 )
+    {
+        return; // one run: the tree is whole
+    }
+
+    // The list of this run's subtrees, in order: s_meet becomes, per element,
+    // 1 + the last element of the subtree that starts there (0: none).
+    uint32_t seen[ PER ];
+#pragma unroll
+    for( int k = 0; k < PER; k++ )
+    {
+        const uint32_t e = k * THREADS + tid;
+        seen[ k ]        = e < count ? s_meet[ e ] : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for( int k = 0; k < PER; k++ )
+    {
+        s_meet[ k * THREADS + tid ] = 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for( int k = 0; k < PER; k++ )
+    {
+        const uint32_t e = k * THREADS + tid;
+        if( seen[ k ] != 0u && seen[ k ] != TAKEN )
+        {
+            // nobody came to meet it: a left child [far, e] or a right child [e + 1, far]
+            const uint32_t far                    = seen[ k ] - 1u;
+            s_meet[ far <= e ? far : e + 1u ] = 1u + ( far <= e ? e : far );
+        }
+    }
+    if( endA != NONE )
+    {
+        s_meet[ endA ] = count;
+    }
+    if( startB != NONE )
+    {
+        s_meet[ 0 ] = 1u + startB;
+    }
+    __syncthreads();
+    uint32_t mine = 0;
+#pragma unroll
+    for( int k = 0; k < PER; k++ )
+    {
+        mine += s_meet[ tid * PER + k ] != 0u ? 1u : 0u;
+    }
+    uint32_t total;
+    uint32_t pos = BlockExclusive( mine, s_wave, &total );
+#pragma unroll
+    for( int k = 0; k < PER; k++ )
+    {
+        const uint32_t e = tid * PER + k, end = s_meet[ e ];
+        if( end != 0u )
+        {
+            if( pos < BUILD_LIST_CAP )
+            {
+                a.listOut[ size_t( blockIdx.x ) * BUILD_LIST_CAP + pos ] = make_uint2( first( e ), last( end - 1u ) );
+            }
+            pos++;
+        }
+    }
+    if( tid == 0 )
+    {
+        a.countOut[ blockIdx.x ] = total < BUILD_LIST_CAP ? total : BUILD_LIST_CAP;
+    }
+}
+
+// ------------------------------------------------------------ collapse
 
 __device__ __forceinline__ uint32_t NodeCount( uint32_t id, uint32_t n, const uint32_t* rf, const uint32_t* rl )
 {
     return id >= n - 1 ? 1u : rl[ id ] - rf[ id ] + 1u;
 }
 
-constexpr uint32_t OPEN_BIT = 0x80000000u;
-
-// Per internal binary node: its two children, each with OPEN_BIT set when it
-// may be opened (internal, more than leafMax triangles), and their half
-// areas (-1 for the others).  The collapse then reads one 16-byte record per
-// opening instead of a chain of child, range and box loads.
-__global__ __launch_bounds__( THREADS ) void k_expand_info( uint32_t internal, uint32_t n, uint32_t leafMax, const uint32_t* children,
-                                                            const uint32_t* rf, const uint32_t* rl, const float* bounds, uint4* info )
-{
-    const uint32_t b = blockIdx.x * THREADS + threadIdx.x;
-    if( b >= internal )
-    {
-        return;
-    }
-    const uint32_t l  = children[ b * 2 + 0 ], r = children[ b * 2 + 1 ];
-    const bool     el = l < n - 1 && NodeCount( l, n, rf, rl ) > leafMax;
-    const bool     er = r < n - 1 && NodeCount( r, n, rf, rl ) > leafMax;
-    const float    al = el ? HalfArea( bounds + size_t( l ) * 6 ) : -1.0f;
-    const float    ar = er ? HalfArea( bounds + size_t( r ) * 6 ) : -1.0f;
-    info[ b ]         = make_uint4( l | ( el ? OPEN_BIT : 0u ), r | ( er ? OPEN_BIT : 0u ), __float_as_uint( al ), __float_as_uint( ar ) );
-}
-
 // Expands binary node b into up to 8 children by repeatedly opening the
 // child with the largest surface area (first one on ties) among those that
-// are internal and hold more than leafMax triangles.
-__global__ __launch_bounds__( THREADS ) void k_collapse_level( const uint32_t* frontierIn,
-                                                               const uint32_t* countIn,
-                                                               uint32_t*       frontierOut,
-                                                               uint32_t*       countOut,
+// are internal and hold more than leafMax triangles.  Level by level: the
+// nodes of this level are queue[levelBase[0] ..  + levelCount[0]), the next
+// level's follow them, each wave taking room for its nodes with one atomic
+// (one per child on a single address took 131 and 197 us for the two widest
+// levels of a 1M-triangle build).
+__global__ __launch_bounds__( THREADS ) void k_collapse_level( uint32_t*       queue,
+                                                               uint32_t*       levelBase,
+                                                               uint32_t*       levelCount,
                                                                uint32_t        n,
                                                                uint32_t        leafMax,
                                                                const uint4*    info,
@@ -687,10 +867,18 @@ __global__ __launch_bounds__( THREADS ) void k_collapse_level( const uint32_t* f
                                                                uint32_t*       expansion,
                                                                uint32_t*       isNode8 )
 {
-    const uint32_t count = *countIn;
-    for( uint32_t t = blockIdx.x * THREADS + threadIdx.x; t < count; t += gridDim.x * THREADS )
+    const uint32_t count = levelCount[ 0 ], first = levelBase[ 0 ];
+    const int      lane  = threadIdx.x & 63;
+    if( blockIdx.x == 0 && threadIdx.x == 0 )
     {
-        const uint32_t b = frontierIn[ t ];
+        levelBase[ 1 ] = first + count;
+    }
+    // whole waves stay in the loop, for the sums over their lanes
+    for( uint32_t w = ( blockIdx.x * THREADS + threadIdx.x ) & ~63u; w < count; w += gridDim.x * THREADS )
+    {
+        const uint32_t t    = w + lane;
+        const bool     have = t < count;
+        const uint32_t b    = have ? queue[ first + t ] : 0u;
         // The node's children so far, each with whether it may be opened
         // (internal, more than leafMax triangles) and its half area.  Every
         // index into these arrays is a compile-time constant (the loops are
@@ -706,7 +894,10 @@ __global__ __launch_bounds__( THREADS ) void k_collapse_level( const uint32_t* f
             ex[ k ] = false;
         }
         int nch = 0;
-        if( b >= n - 1 || NodeCount( b, n, rf, rl ) <= leafMax )
+        if( !have )
+        {
+        }
+        else if( b >= n - 1 || NodeCount( b, n, rf, rl ) <= leafMax )
         {
             ch[ 0 ] = b; // a root that is small enough is a single leaf
             nch     = 1;
@@ -780,22 +971,38 @@ __global__ __launch_bounds__( THREADS ) void k_collapse_level( const uint32_t* f
                 nch++;
             }
         }
-        const uint32_t slot = b < n - 1 ? b : 0;
-#pragma unroll
-        for( int k = 0; k < 8; k++ )
+        if( have )
         {
-            expansion[ size_t( slot ) * 8 + k ] = k < nch ? ch[ k ] : 0xFFFFFFFFu;
-        }
-        isNode8[ slot ] = 1u;
-        if( nch > 1 )
-        {
+            uint32_t out[ 8 ];
 #pragma unroll
             for( int k = 0; k < 8; k++ )
             {
-                if( k < nch && ex[ k ] )
-                {
-                    frontierOut[ atomicAdd( countOut, 1u ) ] = ch[ k ];
-                }
+                out[ k ] = k < nch ? ( ch[ k ] | ( ex[ k ] ? OPEN_BIT : 0u ) ) : 0xFFFFFFFFu;
+            }
+            uint4* e = reinterpret_cast< uint4* >( expansion ) + size_t( first + t ) * 2;
+            e[ 0 ]   = make_uint4( out[ 0 ], out[ 1 ], out[ 2 ], out[ 3 ] );
+            e[ 1 ]   = make_uint4( out[ 4 ], out[ 5 ], out[ 6 ], out[ 7 ] );
+            isNode8[ b < n - 1 ? b : 0 ] = 1u;
+        }
+        uint32_t kids = 0;
+#pragma unroll
+        for( int k = 0; k < 8; k++ )
+        {
+            kids += k < nch && ex[ k ] ? 1u : 0u;
+        }
+        const uint32_t inc  = WaveInclusive( kids, lane );
+        uint32_t       base = 0;
+        if( lane == 63 && inc != 0u )
+        {
+            base = atomicAdd( levelCount + 1, inc );
+        }
+        uint32_t pos = first + count + __shfl( base, 63, 64 ) + inc - kids;
+#pragma unroll
+        for( int k = 0; k < 8; k++ )
+        {
+            if( k < nch && ex[ k ] )
+            {
+                queue[ pos++ ] = ch[ k ];
             }
         }
     }
@@ -806,10 +1013,9 @@ __device__ __forceinline__ uint32_t LeafRef( uint32_t first, uint32_t count )
     return RG_EXT_BVH_CHILD_LEAF_BIT | ( first << 3 ) | ( count - 1u );
 }
 
-__global__ __launch_bounds__( THREADS ) void k_write_nodes( uint32_t        slots,
+__global__ __launch_bounds__( THREADS ) void k_write_nodes( uint32_t        count,
                                                             uint32_t        n,
-                                                            uint32_t        leafMax,
-                                                            const uint32_t* isNode8,
+                                                            const uint32_t* queue,
                                                             const uint32_t* node8Index,
                                                             const uint32_t* expansion,
                                                             const uint32_t* rf,
@@ -817,47 +1023,37 @@ __global__ __launch_bounds__( THREADS ) void k_write_nodes( uint32_t        slot
                                                             const float*    bounds,
                                                             BvhNode8*       nodes )
 {
-    // one thread per (slot, child): the 8 threads of a node write its SoA
-    // arrays as contiguous 32-byte runs
+    // one thread per (node of the collapse's queue, child): the 8 threads of
+    // a node write its SoA arrays as contiguous 32-byte runs
     const uint64_t t = uint64_t( blockIdx.x ) * THREADS + threadIdx.x;
-    const uint32_t b = uint32_t( t >> 3 );
+    const uint32_t q = uint32_t( t >> 3 );
     const int      k = int( t & 7u );
-    if( b >= slots || !isNode8[ b ] )
+    if( q >= count )
     {
         return;
     }
-    BvhNode8& node = nodes[ node8Index[ b ] ];
+    const uint32_t b    = queue[ q ];
+    BvhNode8&      node = nodes[ node8Index[ b < n - 1 ? b : 0 ] ];
+    const uint32_t e    = expansion[ t ];
+    if( e == 0xFFFFFFFFu )
     {
-        const uint32_t c = expansion[ size_t( b ) * 8 + k ];
-        if( c == 0xFFFFFFFFu )
-        {
-            node.lo_x[ k ] = node.lo_y[ k ] = node.lo_z[ k ] = INFINITY;
-            node.hi_x[ k ] = node.hi_y[ k ] = node.hi_z[ k ] = -INFINITY;
-            node.child[ k ] = RG_EXT_BVH_CHILD_EMPTY;
-            node.pad[ k ]   = 0;
-            return;
-        }
-        const float* bb = bounds + size_t( c ) * 6;
-        node.lo_x[ k ]  = bb[ 0 ];
-        node.lo_y[ k ]  = bb[ 1 ];
-        node.lo_z[ k ]  = bb[ 2 ];
-        node.hi_x[ k ]  = bb[ 3 ];
-        node.hi_y[ k ]  = bb[ 4 ];
-        node.hi_z[ k ]  = bb[ 5 ];
+        node.lo_x[ k ] = node.lo_y[ k ] = node.lo_z[ k ] = INFINITY;
+        node.hi_x[ k ] = node.hi_y[ k ] = node.hi_z[ k ] = -INFINITY;
+        node.child[ k ] = RG_EXT_BVH_CHILD_EMPTY;
         node.pad[ k ]   = 0;
-        if( c >= n - 1 )
-        {
-            node.child[ k ] = LeafRef( c - ( n - 1 ), 1 );
-        }
-        else if( NodeCount( c, n, rf, rl ) <= leafMax || isNode8[ c ] == 0u || c == b )
-        {
-            node.child[ k ] = LeafRef( rf[ c ], rl[ c ] - rf[ c ] + 1u );
-        }
-        else
-        {
-            node.child[ k ] = node8Index[ c ];
-        }
+        return;
     }
+    const uint32_t c  = e & ~OPEN_BIT;
+    const float2*  bb = reinterpret_cast< const float2* >( bounds + size_t( c ) * 6 );
+    const float2   x = bb[ 0 ], y = bb[ 1 ], z = bb[ 2 ];
+    node.lo_x[ k ]  = x.x;
+    node.lo_y[ k ]  = x.y;
+    node.lo_z[ k ]  = y.x;
+    node.hi_x[ k ]  = y.y;
+    node.hi_y[ k ]  = z.x;
+    node.hi_z[ k ]  = z.y;
+    node.pad[ k ]   = 0;
+    node.child[ k ] = e & OPEN_BIT ? node8Index[ c ] : ( c >= n - 1 ? LeafRef( c - ( n - 1 ), 1 ) : LeafRef( rf[ c ], rl[ c ] - rf[ c ] + 1u ) );
 }
 
 // Outward rounding to half: the half nearest to v - origin, stepped down
@@ -961,16 +1157,84 @@ __global__ __launch_bounds__( THREADS ) void k_sorted_tris( const float* tris, c
     out[ size_t( k ) * 3 + 2 ] = make_float4( c.x, c.y, c.z, 0.0f );
 }
 
-__global__ void k_seed_frontier( uint32_t* frontier, uint32_t* counts )
+__global__ void k_seed_frontier( uint32_t* queue, uint32_t* counts )
 {
-    frontier[ 0 ] = 0;
-    counts[ 0 ]   = 1;
+    queue[ 0 ]  = 0;
+    counts[ 0 ] = 1;
 }
 
 } // namespace
 
 namespace
 {
+// Stable sort of n (key, value) pairs by key bits [lo, hi); on return *kin and
+// *vin hold the result.  hist: 256 words per tile and 256 more.
+void RadixSort( uint64_t** kin, uint64_t** kout, uint32_t** vin, uint32_t** vout, uint32_t n, int lo, int hi, uint32_t* hist, hipStream_t stream )
+{
+    const uint32_t blocks = DivUp( n, RS_TILE );
+    uint32_t*      totals = hist + size_t( 256 ) * blocks;
+    for( int shift = lo; shift < hi; shift += 8 )
+    {
+        k_radix_hist<<< blocks, THREADS, 0, stream >>>( *kin, n, shift, hist, blocks );
+        CheckLaunch( "k_radix_hist" );
+        k_radix_scan<<< 256, THREADS, 0, stream >>>( hist, totals, blocks );
+        CheckLaunch( "k_radix_scan" );
+        k_radix_scatter<<< blocks, THREADS, 0, stream >>>( *kin, *vin, *kout, *vout, n, shift, hist, totals, blocks );
+        CheckLaunch( "k_radix_scatter" );
+        std::swap( *kin, *kout );
+        std::swap( *vin, *vout );
+    }
+}
+
+// Runs of the hierarchy's first launch: 256 triangles while that fills the
+// chip with blocks, 1024 (and a quarter of the subtrees left over) beyond.
+constexpr uint32_t TREE_RUN_SMALL = THREADS, TREE_RUN = 4 * THREADS;
+constexpr uint32_t TREE_SMALL     = 128 * TREE_RUN_SMALL;
+
+uint32_t TreeRuns( uint32_t n )
+{
+    return n <= TREE_SMALL ? DivUp( n, TREE_RUN_SMALL ) : DivUp( n, TREE_RUN );
+}
+
+// Two sets of lists (the first launch's and the second's) and their counts.
+size_t TreeListBytes( uint32_t n )
+{
+    const size_t runs = TreeRuns( n ), next = DivUp( runs, BUILD_LISTS );
+    return ( runs + next ) * ( BUILD_LIST_CAP * sizeof( uint2 ) + sizeof( uint32_t ) );
+}
+
+void BuildTree( TreeArgs a, uint2* lists, hipStream_t stream )
+{
+    uint32_t  runs = TreeRuns( a.n );
+    const uint32_t next = DivUp( runs, BUILD_LISTS );
+    uint2*    listA = lists;
+    uint2*    listB = listA + size_t( runs ) * BUILD_LIST_CAP;
+    uint32_t* cntA = reinterpret_cast< uint32_t* >( listB + size_t( next ) * BUILD_LIST_CAP );
+    uint32_t* cntB = cntA + runs;
+    a.listOut  = listA;
+    a.countOut = cntA;
+    if( a.n <= TREE_SMALL )
+    {
+        k_tree< true, 1 ><<< runs, THREADS, 0, stream >>>( a );
+    }
+    else
+    {
+        k_tree< true, 4 ><<< runs, THREADS, 0, stream >>>( a );
+    }
+    CheckLaunch( "k_tree" );
+    while( runs > 1 )
+    {
+        a.listIn   = a.listOut;
+        a.countIn  = a.countOut;
+        a.lists    = runs;
+        a.listOut  = a.listOut == listA ? listB : listA;
+        a.countOut = a.countOut == cntA ? cntB : cntA;
+        runs       = DivUp( runs, BUILD_LISTS );
+        k_tree< false, int( BUILD_LISTS * BUILD_LIST_CAP / THREADS ) ><<< runs, THREADS, 0, stream >>>( a );
+        CheckLaunch( "k_tree" );
+    }
+}
+
 // Shared by the single-scene and the batched build; `batch` (host offsets,
 // S + 1 of them) switches steps 1-2 to per-scene bounds and keys and seeds
 // the collapse with every scene's root.
@@ -991,8 +1255,6 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
     const uint32_t slots      = internal > 0 ? internal : 1;
     const uint32_t rsBlocks   = DivUp( n, RS_TILE );
     const uint32_t bndBlocks  = DivUp( n, THREADS ) < 1024 ? DivUp( n, THREADS ) : 1024;
-    const uint32_t histCount  = 256 * rsBlocks;
-    const uint32_t scanElems  = histCount > slots ? histCount : slots;
 
     bvh.sortedTris.Reserve( size_t( n ) * 48 );
     bvh.codes.Reserve( size_t( n ) * 8 );
@@ -1000,33 +1262,23 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
     bvh.keysB.Reserve( size_t( n ) * 8 );
     bvh.valsA.Reserve( size_t( n ) * 4 );
     bvh.valsB.Reserve( size_t( n ) * 4 );
-    bvh.hist.Reserve( size_t( histCount ) * 4 );
-    bvh.scanScratch.Reserve( ScanScratchBytes( scanElems ) );
+    bvh.hist.Reserve( size_t( 256 ) * ( rsBlocks + 1 ) * 4 );
+    bvh.scanScratch.Reserve( ScanScratchBytes( slots ) );
     bvh.boundsPartials.Reserve( size_t( bndBlocks + 1 ) * 6 * 8 );
     bvh.children.Reserve( size_t( slots ) * 8 );
-    bvh.parents.Reserve( size_t( 2 * n - 1 ) * 4 );
     bvh.rangeFirst.Reserve( size_t( slots ) * 4 );
     bvh.rangeLast.Reserve( size_t( slots ) * 4 );
     bvh.nodeBounds.Reserve( size_t( 2 * n - 1 ) * 24 );
-    bvh.depthA.Reserve( size_t( 2 * n - 1 ) * 4 );
-    bvh.depthB.Reserve( size_t( 2 * n - 1 ) * 4 );
-    bvh.jumpA.Reserve( size_t( 2 * n - 1 ) * 4 );
-    bvh.jumpB.Reserve( size_t( 2 * n - 1 ) * 4 );
-    bvh.levelHist.Reserve( size_t( REFIT_MAX_DEPTH + 1 ) * 4 );
-    bvh.levelOrder.Reserve( size_t( slots ) * 4 );
-    if( !bvh.hostLevels )
-    {
-        RG_HIP_CHECK( hipHostMalloc( reinterpret_cast< void** >( &bvh.hostLevels ), ( REFIT_MAX_DEPTH + 1 ) * 4, hipHostMallocDefault ) );
-    }
+    bvh.expandInfo.Reserve( size_t( slots ) * sizeof( uint4 ) );
+    bvh.treeLists.Reserve( TreeListBytes( n ) );
     bvh.expansion.Reserve( size_t( slots ) * 32 );
     bvh.isNode8.Reserve( size_t( slots ) * 4 );
     bvh.node8Index.Reserve( size_t( slots ) * 4 );
-    bvh.frontier[ 0 ].Reserve( size_t( slots ) * 4 );
-    bvh.frontier[ 1 ].Reserve( size_t( slots ) * 4 );
-    bvh.levelCounts.Reserve( ( BVH_MAX_LEVELS + 2 ) * 4 );
+    bvh.queue.Reserve( size_t( slots ) * 4 );
+    bvh.levelCounts.Reserve( ( BVH_MAX_LEVELS + 1 ) * 2 * 4 );
     if( !bvh.hostCounts )
     {
-        RG_HIP_CHECK( hipHostMalloc( reinterpret_cast< void** >( &bvh.hostCounts ), ( BVH_MAX_LEVELS + 2 ) * 4, hipHostMallocDefault ) );
+        RG_HIP_CHECK( hipHostMalloc( reinterpret_cast< void** >( &bvh.hostCounts ), 2 * 4, hipHostMallocDefault ) );
     }
 
     double* partials    = bvh.boundsPartials.as< double >();
@@ -1078,101 +1330,37 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
     uint64_t* kout = bvh.keysB.as< uint64_t >();
     uint32_t* vin  = bvh.valsA.as< uint32_t >();
     uint32_t* vout = bvh.valsB.as< uint32_t >();
-    for( int pass = 0; pass < 8; pass++ )
-    {
-        const int shift = pass * 8;
-        k_radix_hist<<< rsBlocks, THREADS, 0, stream >>>( kin, n, shift, bvh.hist.as< uint32_t >(), rsBlocks );
-        CheckLaunch( "k_radix_hist" );
-        ExclusiveScan( bvh.hist.as< uint32_t >(), histCount, bvh.hist.as< uint32_t >(), nullptr, bvh.scanScratch.as< uint32_t >(), stream );
-        k_radix_scatter<<< rsBlocks, THREADS, 0, stream >>>( kin, vin, kout, vout, n, shift, bvh.hist.as< uint32_t >(), rsBlocks );
-        CheckLaunch( "k_radix_scatter" );
-        std::swap( kin, kout );
-        std::swap( vin, vout );
-    }
+    RadixSort( &kin, &kout, &vin, &vout, n, 0, 64, bvh.hist.as< uint32_t >(), stream );
     bvh.sortedKeys = kin;
     bvh.sortedIdx  = vin;
 
-    // 4. Karras hierarchy.
+    // 4. The binary hierarchy with its boxes.
     uint32_t* children = bvh.children.as< uint32_t >();
-    uint32_t* parents  = bvh.parents.as< uint32_t >();
     uint32_t* rf       = bvh.rangeFirst.as< uint32_t >();
     uint32_t* rl       = bvh.rangeLast.as< uint32_t >();
-    if( internal > 0 )
-    {
-        k_karras<<< DivUp( internal, THREADS ), THREADS, 0, stream >>>( kin, n, children, parents, rf, rl );
-        CheckLaunch( "k_karras" );
-    }
+    float*    bounds   = bvh.nodeBounds.as< float >();
+    TreeArgs  ta{};
+    ta.tris       = d_tris;
+    ta.keys       = kin;
+    ta.order      = vin;
+    ta.n          = n;
+    ta.leafMax    = bvh.leafMax;
+    ta.children   = bvh.children.as< uint2 >();
+    ta.rangeFirst = rf;
+    ta.rangeLast  = rl;
+    ta.bounds     = bounds;
+    ta.info       = bvh.expandInfo.as< uint4 >();
+    BuildTree( ta, bvh.treeLists.as< uint2 >(), stream );
 
-    // 5. Refit.
-    float* bounds = bvh.nodeBounds.as< float >();
-    k_leaf_boxes<<< DivUp( n, THREADS ), THREADS, 0, stream >>>( d_tris, vin, n, bounds );
-    CheckLaunch( "k_leaf_boxes" );
-    if( internal > 0 )
-    {
-        const uint32_t all  = 2 * n - 1;
-        uint32_t*      dA   = bvh.depthA.as< uint32_t >();
-        uint32_t*      dB   = bvh.depthB.as< uint32_t >();
-        uint32_t*      jA   = bvh.jumpA.as< uint32_t >();
-        uint32_t*      jB   = bvh.jumpB.as< uint32_t >();
-        k_depth_init<<< DivUp( all, THREADS ), THREADS, 0, stream >>>( parents, all, dA, jA );
-        CheckLaunch( "k_depth_init" );
-        for( int r = 0; r < REFIT_JUMP_ROUNDS; r++ )
-        {
-            k_depth_jump<<< DivUp( all, THREADS ), THREADS, 0, stream >>>( all, dA, jA, dB, jB );
-            CheckLaunch( "k_depth_jump" );
-            std::swap( dA, dB );
-            std::swap( jA, jB );
-        }
-        uint32_t* hist = bvh.levelHist.as< uint32_t >();
-        RG_HIP_CHECK( hipMemsetAsync( hist, 0, ( REFIT_MAX_DEPTH + 1 ) * 4, stream ) );
-        // (depth, node) pairs into the free key buffer and dB, then one
-        // stable 8-bit radix pass groups the nodes by depth into levelOrder
-        k_depth_keys<<< DivUp( internal, THREADS ), THREADS, 0, stream >>>( internal, dA, hist, kout, dB );
-        CheckLaunch( "k_depth_keys" );
-        RG_HIP_CHECK( hipMemcpyAsync( bvh.hostLevels, hist, ( REFIT_MAX_DEPTH + 1 ) * 4, hipMemcpyDeviceToHost, stream ) );
-        const uint32_t lvBlocks = DivUp( internal, RS_TILE );
-        k_radix_hist<<< lvBlocks, THREADS, 0, stream >>>( kout, internal, 0, bvh.hist.as< uint32_t >(), lvBlocks );
-        CheckLaunch( "k_radix_hist" );
-        ExclusiveScan( bvh.hist.as< uint32_t >(), 256 * lvBlocks, bvh.hist.as< uint32_t >(), nullptr, bvh.scanScratch.as< uint32_t >(), stream );
-        k_radix_scatter<<< lvBlocks, THREADS, 0, stream >>>( kout, dB, kin, bvh.levelOrder.as< uint32_t >(), internal, 0, bvh.hist.as< uint32_t >(),
-                                                             lvBlocks );
-        CheckLaunch( "k_radix_scatter" );
-        bvh.sortedKeys = nullptr; // the sorted Morton keys were overwritten
-        RG_HIP_CHECK( hipStreamSynchronize( stream ) );
-        RG_REQUIRE( bvh.hostLevels[ REFIT_MAX_DEPTH ] == 0, RG_RESULT_INTERNAL_ERROR, "BVH deeper than the refit level limit" );
-        uint32_t first[ REFIT_MAX_DEPTH ], sum = 0;
-        int      deepest = 0;
-        for( uint32_t d = 0; d < REFIT_MAX_DEPTH; d++ )
-        {
-            first[ d ] = sum;
-            sum += bvh.hostLevels[ d ];
-            deepest = bvh.hostLevels[ d ] ? int( d ) : deepest;
-        }
-        for( int d = deepest; d >= 0; d-- )
-        {
-            const uint32_t c = bvh.hostLevels[ d ];
-            if( c )
-            {
-                k_refit_level<<< DivUp( c, THREADS ), THREADS, 0, stream >>>( bvh.levelOrder.as< uint32_t >(), first[ d ], c, children, bounds );
-                CheckLaunch( "k_refit_level" );
-            }
-        }
-    }
-
-    // 6. Collapse to 8-wide nodes, level by level.
-    bvh.expandInfo.Reserve( size_t( internal > 0 ? internal : 1 ) * sizeof( uint4 ) );
-    if( internal > 0 )
-    {
-        k_expand_info<<< DivUp( internal, THREADS ), THREADS, 0, stream >>>( internal, n, bvh.leafMax, children, rf, rl, bounds,
-                                                                            bvh.expandInfo.as< uint4 >() );
-        CheckLaunch( "k_expand_info" );
-    }
-    uint32_t* counts = bvh.levelCounts.as< uint32_t >();
-    RG_HIP_CHECK( hipMemsetAsync( counts, 0, ( BVH_MAX_LEVELS + 2 ) * 4, stream ) );
+    // 5. Collapse to 8-wide nodes, level by level.
+    uint32_t* queue  = bvh.queue.as< uint32_t >();
+    uint32_t* counts = bvh.levelCounts.as< uint32_t >();  // nodes of each level
+    uint32_t* bases  = counts + BVH_MAX_LEVELS + 1;       // its first node in the queue
+    RG_HIP_CHECK( hipMemsetAsync( counts, 0, ( BVH_MAX_LEVELS + 1 ) * 2 * 4, stream ) );
     RG_HIP_CHECK( hipMemsetAsync( bvh.isNode8.ptr, 0, size_t( slots ) * 4, stream ) );
     if( !batched )
     {
-        k_seed_frontier<<< 1, 1, 0, stream >>>( bvh.frontier[ 0 ].as< uint32_t >(), counts );
+        k_seed_frontier<<< 1, 1, 0, stream >>>( queue, counts );
         CheckLaunch( "k_seed_frontier" );
     }
     else
@@ -1181,51 +1369,49 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
         k_scene_roots<<< DivUp( internal, THREADS ), THREADS, 0, stream >>>( internal, rf, rl, bvh.sceneOffsets.as< uint32_t >(), sceneCount,
                                                                            bvh.sceneRoots.as< uint32_t >() );
         CheckLaunch( "k_scene_roots" );
-        k_seed_frontier_seg<<< 1, 256, 0, stream >>>( bvh.sceneRoots.as< uint32_t >(), sceneCount, bvh.frontier[ 0 ].as< uint32_t >(), counts );
+        k_seed_frontier_seg<<< 1, 256, 0, stream >>>( bvh.sceneRoots.as< uint32_t >(), sceneCount, queue, counts );
         CheckLaunch( "k_seed_frontier_seg" );
     }
 
-    const uint32_t maxFrontier   = n / ( bvh.leafMax + 1 ) + 1;
-    const uint32_t collapseGrid  = DivUp( maxFrontier, THREADS ) < 4096 ? DivUp( maxFrontier, THREADS ) : 4096;
-    uint32_t       level         = 0;
-    bool           done          = false;
-    while( !done )
+    const uint32_t maxFrontier  = n / ( bvh.leafMax + 1 ) + 1;
+    const uint32_t collapseGrid = DivUp( maxFrontier, THREADS ) < 4096 ? DivUp( maxFrontier, THREADS ) : 4096;
+    // levels before the first look at how many nodes are left: an 8-wide
+    // node stands for about 1.75 binary levels
+    uint32_t bits = 1;
+    while( bits < 28 && ( n >> bits ) != 0 )
     {
-        constexpr uint32_t BATCH = 8;
-        for( uint32_t k = 0; k < BATCH; k++, level++ )
+        bits++;
+    }
+    uint32_t level = 0, batch = bits * 4 / 7 + 2;
+    do
+    {
+        for( uint32_t k = 0; k < batch; k++, level++ )
         {
             RG_REQUIRE( level + 1 < BVH_MAX_LEVELS, RG_RESULT_INTERNAL_ERROR, "BVH deeper than the level limit" );
-            k_collapse_level<<< collapseGrid, THREADS, 0, stream >>>( bvh.frontier[ level & 1 ].as< uint32_t >(),
-                                                                      counts + level,
-                                                                      bvh.frontier[ ( level + 1 ) & 1 ].as< uint32_t >(),
-                                                                      counts + level + 1,
-                                                                      n,
-                                                                      bvh.leafMax,
-                                                                      bvh.expandInfo.as< uint4 >(),
-                                                                      rf,
-                                                                      rl,
-                                                                      bvh.expansion.as< uint32_t >(),
+            k_collapse_level<<< collapseGrid, THREADS, 0, stream >>>( queue, bases + level, counts + level, n, bvh.leafMax,
+                                                                      bvh.expandInfo.as< uint4 >(), rf, rl, bvh.expansion.as< uint32_t >(),
                                                                       bvh.isNode8.as< uint32_t >() );
             CheckLaunch( "k_collapse_level" );
         }
         RG_HIP_CHECK( hipMemcpyAsync( bvh.hostCounts, counts + level, 4, hipMemcpyDeviceToHost, stream ) );
+        RG_HIP_CHECK( hipMemcpyAsync( bvh.hostCounts + 1, bases + level, 4, hipMemcpyDeviceToHost, stream ) );
         RG_HIP_CHECK( hipStreamSynchronize( stream ) );
-        done = bvh.hostCounts[ 0 ] == 0;
-    }
-
-    uint32_t* nodeTotal = counts + BVH_MAX_LEVELS;
-    ExclusiveScan( bvh.isNode8.as< uint32_t >(), slots, bvh.node8Index.as< uint32_t >(), nodeTotal, bvh.scanScratch.as< uint32_t >(), stream );
-    RG_HIP_CHECK( hipMemcpyAsync( bvh.hostCounts, nodeTotal, 4, hipMemcpyDeviceToHost, stream ) );
-    RG_HIP_CHECK( hipStreamSynchronize( stream ) );
-    bvh.nodeCount = bvh.hostCounts[ 0 ];
+        batch = 4;
+    } while( bvh.hostCounts[ 0 ] != 0 );
+    bvh.nodeCount = bvh.hostCounts[ 1 ];
     // a batch of one-triangle frame segments has leaves for roots and no node
     RG_REQUIRE( bvh.nodeCount >= 1 || segmentBoxes, RG_RESULT_INTERNAL_ERROR, "BVH collapse produced no nodes" );
+    ExclusiveScan( bvh.isNode8.as< uint32_t >(), slots, bvh.node8Index.as< uint32_t >(), nullptr, bvh.scanScratch.as< uint32_t >(), stream );
 
     const bool    half    = params.nodeFormat == RG_EXT_BVH_NODE_FP16;
     DeviceBuffer& fp32Out = half ? bvh.nodes32 : bvh.nodes;
     fp32Out.Reserve( size_t( bvh.nodeCount ) * sizeof( BvhNode8 ) );
-    k_write_nodes<<< DivUp( slots * 8u, THREADS ), THREADS, 0, stream >>>( slots, n, bvh.leafMax, bvh.isNode8.as< uint32_t >(), bvh.node8Index.as< uint32_t >(), bvh.expansion.as< uint32_t >(), rf, rl, bounds, fp32Out.as< BvhNode8 >() );
-    CheckLaunch( "k_write_nodes" );
+    if( bvh.nodeCount > 0 )
+    {
+        k_write_nodes<<< DivUp( uint64_t( bvh.nodeCount ) * 8u, THREADS ), THREADS, 0, stream >>>(
+            bvh.nodeCount, n, queue, bvh.node8Index.as< uint32_t >(), bvh.expansion.as< uint32_t >(), rf, rl, bounds, fp32Out.as< BvhNode8 >() );
+        CheckLaunch( "k_write_nodes" );
+    }
     k_sorted_tris<<< DivUp( n, THREADS ), THREADS, 0, stream >>>( d_tris, vin, n, bvh.sortedTris.as< float4 >() );
     CheckLaunch( "k_sorted_tris" );
     if( batched )

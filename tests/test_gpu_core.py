@@ -59,6 +59,24 @@ def test_lbvh_bit_exact_duplicates(gpu, oracle):
     _assert_same_bvh(b.download(), oracle.bvh(tris, 3).download())
 
 
+@pytest.mark.parametrize("kind", ["even", "nested"])
+@pytest.mark.parametrize("n", [255, 257, 1024, 2049, 32768, 32769, 50001])
+def test_lbvh_bit_exact_at_run_and_tile_edges(gpu, oracle, n, kind):
+    """Sizes about the hierarchy's runs (256 and 1024 triangles), the sort's
+    tiles (2048) and the change between the runs (32768); "nested" halves the
+    distances again and again towards one place with thousands of equal
+    triangles, which makes the longest root paths across runs."""
+    tris = _random_tris(n, seed=n)
+    if kind == "nested":
+        r = np.random.default_rng(n)
+        k = np.minimum(r.integers(0, 40, n), 22)  # 45% of them at the last distance
+        tris = np.broadcast_to(np.float32([0, 0, 0, 1e-3, 0, 0, 0, 1e-3, 0]), (n, 9)) + np.repeat(np.float32(2.0) ** -k[:, None], 9, 1)
+        tris = np.ascontiguousarray(tris, np.float32)
+    for leaf in (1, 3):
+        b, _ = _gpu_bvh(tris, leaf)
+        _assert_same_bvh(b.download(), oracle.bvh(tris, leaf).download())
+
+
 def test_lbvh_bit_exact_terrain_boxes(gpu, oracle):
     s = scenes.terrain_boxes_scene()
     b, _ = _gpu_bvh(s.tris, 3)
