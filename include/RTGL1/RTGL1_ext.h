@@ -71,6 +71,9 @@ RGAPI RgResult RGCONV rgExtTimerElapsedMs( RgExtTimer timer, float* pMs );
  * gives the same nodes bit for bit. */
 typedef struct RgExtBvh_T* RgExtBvh;
 
+/* Format of the published nodes (rgExtBvhGetView), which traces with
+ * RG_EXT_TRACE_COLLECT_STATS walk; other traces walk nodes of the
+ * library's own. */
 #define RG_EXT_BVH_NODE_FP32 0u /* 256-byte nodes with FP32 child boxes     */
 #define RG_EXT_BVH_NODE_FP16 1u /* 144-byte nodes: FP32 origin, child boxes as FP16
                                    offsets from it rounded outward */
@@ -143,7 +146,8 @@ typedef struct RgExtHit
 #define RG_EXT_TRACE_CLOSEST         0u
 #define RG_EXT_TRACE_ANY_HIT         1u /* stop at the first hit (occlusion) */
 #define RG_EXT_TRACE_CULL_FRONT_FACE 2u /* gl_RayFlagsCullFrontFacingTrianglesEXT, CCW = front */
-#define RG_EXT_TRACE_COLLECT_STATS   4u /* count node visits and triangle tests */
+#define RG_EXT_TRACE_COLLECT_STATS   4u /* walk the published nodes near to far, counting node
+                                          visits and triangle tests: the same hits, slower */
 
 RGAPI RgResult RGCONV rgExtTraceRays( RgExtBvh        bvh,
                                       const RgExtRay* d_rays,
@@ -158,7 +162,7 @@ RGAPI RgResult RGCONV rgExtTraceRays( RgExtBvh        bvh,
  * scratch is one fixed device array per GPU of 40 MiB + 8.25 KiB, held
  * until the process ends: the ray-chunk counters, the error word, the
  * statistics and the global traversal stacks of a persistent grid of at
- * most 1024 blocks (64 stack entries per ray, 24 of them in LDS; a deeper
+ * most 1024 blocks (64 stack words per ray, 24 of them in LDS; a deeper
  * stack sets RG_EXT_TRACE_ERROR_STACK_OVERFLOW).  Every call on a GPU
  * shares that array, so calls that overlap on one GPU race.  After a call,
  * rgExtBvhGetTraceErrors / rgExtBvhGetTraceStats of the BVH report that
@@ -203,7 +207,7 @@ RGAPI RgResult RGCONV rgExtTraceRaysBatch( RgExtBvh        bvh,
 /* Traversal tuning chosen by rgExtTraceAutotune. */
 typedef struct RgExtTraceTuning
 {
-    uint32_t stackLdsEntries; /* LDS part of the 128-entry per-lane stack: 16, 24, 32 */
+    uint32_t stackLdsEntries; /* words of the per-lane stack in LDS: 16, 24, 32 (two per node visited) */
     uint32_t rayChunk;        /* rays a wave takes per counter atomic: 32, 64, 128   */
     float    msPerLaunch;     /* best time on the tuning rays                         */
     float    msDefault;       /* time with the defaults (24, 64)                      */
@@ -507,8 +511,10 @@ typedef struct RgExtDrawFramePathParams
 } RgExtDrawFramePathParams;
 
 /* FP16 precision form: FP16 storage of the denoiser's temporal and a-trous
- * planes (RG_EXT_STORAGE_FP16) and FP16 BVH nodes (RG_EXT_BVH_NODE_FP16);
- * camera matrices stay FP64 on the host and ray-triangle tests FP32. */
+ * planes (RG_EXT_STORAGE_FP16); camera matrices stay FP64 on the host and
+ * ray-triangle tests FP32.  RG_EXT_PRECISION_FP16_NODES is accepted and
+ * changes nothing: frames trace through nodes smaller than FP16 ones, with
+ * the same hits. */
 #define RG_EXT_PRECISION_FP16_STORAGE 1u
 #define RG_EXT_PRECISION_FP16_NODES   2u
 

@@ -43,17 +43,41 @@ struct alignas( 16 ) BvhNode8H
 };
 static_assert( sizeof( BvhNode8H ) == 144, "node size" );
 
+// The traversal's node, 80 bytes: eight child boxes as bytes on a grid of the
+// node's own (origin + q * 2^k per axis, rounded outward), child nodes in
+// the first slots (slot s is node childBase + s), then leaves of one
+// triangle each (slot s is triangle triBase + s), so that neither a sort key
+// nor the stack needs a child reference.
+struct alignas( 16 ) BvhNodeQ
+{
+    float    origin[ 3 ];
+    uint32_t meta;          // three biased exponents, child nodes << 24, leaves << 28
+    uint8_t  lo[ 3 ][ 8 ];
+    uint8_t  hi[ 3 ][ 8 ];
+    uint32_t childBase;
+    uint32_t triBase;
+    uint32_t pad[ 2 ];
+};
+static_assert( sizeof( BvhNodeQ ) == 80, "node size" );
+
 constexpr uint32_t BVH_MAX_LEVELS = 128;
 
 struct BvhObject
 {
     uint32_t n          = 0;
-    uint32_t nodeCount  = 0;
+    uint32_t nodeCount  = 0; // published nodes; without them the traversal's
+    uint32_t nodeCountQ = 0; // traversal nodes
     uint32_t nodeFormat = RG_EXT_BVH_NODE_FP32;
     uint32_t leafMax    = 3;
     double   sceneMin[ 3 ] = { 0, 0, 0 };
     double   sceneMax[ 3 ] = { 0, 0, 0 };
 
+    // what rays are traced through
+    DeviceBuffer nodesQ;       // nodeCountQ BvhNodeQ, each scene's or segment's root first
+    DeviceBuffer nodeTris;     // n * 3 float4: (v0, primId bits) (v1, 0) (v2, 0), a node's leaves side by side
+    DeviceBuffer scratch;      // of that tree's build
+
+    // the published LBVH (rgExtBvhBuild, rgExtBvhBuildBatch)
     DeviceBuffer sortedTris;   // n * 3 float4
     DeviceBuffer codes;        // n u64, input order
     DeviceBuffer keysA, keysB; // n u64
@@ -71,24 +95,21 @@ struct BvhObject
     DeviceBuffer isNode8;      // max(1,n-1) u32
     DeviceBuffer node8Index;   // max(1,n-1) u32
     DeviceBuffer queue;        // max(1,n-1) u32: the binary nodes that became 8-wide ones, level by level
-    DeviceBuffer levelCounts;  // BVH_MAX_LEVELS + 1 u32 each: nodes per level, first node of each level
     DeviceBuffer nodes;        // nodeCount * stride
     DeviceBuffer nodes32;      // FP32 nodes an FP16 build converts from
-    uint32_t*    hostCounts = nullptr; // pinned
+    uint32_t*    hostLevels = nullptr; // pinned: per tree, nodes of each level and its first node
     // batched build: per-scene offsets, binary and 8-wide roots, bounds
     uint32_t                sceneCount = 0;
     DeviceBuffer            sceneOffsets, sceneRoots, sceneRoots8, sceneBounds, scenePartials;
     std::vector< uint32_t > hostSceneOffsets, hostSceneRoots;
 
-    // Index of the sorted-order permutation after the sort (keysA/valsA or B).
-    const uint32_t* sortedIdx = nullptr;
-    const uint64_t* sortedKeys = nullptr;
+    const uint32_t* sortedIdx = nullptr; // the published sorted order
 
     ~BvhObject()
     {
-        if( hostCounts )
+        if( hostLevels )
         {
-            ( void )hipHostFree( hostCounts );
+            ( void )hipHostFree( hostLevels );
         }
     }
 
@@ -101,11 +122,10 @@ struct BvhObject
     struct FrameSegment
     {
         uint32_t cls  = 0;       // the class (index into BuildFrameBvh's counts)
-        uint32_t root = 0;       // 8-wide node, or the leaf of a one-triangle segment
+        uint32_t root = 0;       // traversal node
         float    box[ 6 ] = {};  // lo x, y, z, hi x, y, z (infinite for a single segment)
     };
     std::vector< FrameSegment > frameSegs;
-    DeviceBuffer                segBoxes;     // 8 floats per segment
     std::vector< float >        hostSegBoxes;
 };
 
@@ -113,8 +133,9 @@ void BuildBvh( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtBvhBu
 // Several scenes in one BVH object: triangles of scene s are
 // [offsets[s], offsets[s+1]) of d_tris (host offsets); each scene gets its
 // own root (hostSceneRoots) and never shares a node with another scene.
+// Without view, only what rays are traced through is built.
 void BuildBvhBatch( BvhObject& bvh, const float* d_tris, const uint32_t* offsets, uint32_t sceneCount, const RgExtBvhBuildParams& params,
-                    hipStream_t stream );
+                    hipStream_t stream, bool view = true );
 
 // The frame's BVH over the triangles of classTris[c] triangles per class,
 // classes in order.  One class: a single-scene build.  Several: one batched
@@ -135,7 +156,7 @@ struct TraceContext
     DeviceBuffer            segRays; // ray offsets of a batched launch
     std::vector< uint32_t > segHost;
     uint32_t     gridBlocks = 0;                        // the largest grid (sizes the overflow stacks)
-    uint32_t     grid[ 2 ][ TRACE_STACK_VARIANTS ] = {}; // resident blocks per node format and stack variant
+    uint32_t     grid[ TRACE_STACK_VARIANTS + 1 ] = {}; // resident blocks per stack variant, and of the counting walk
     uint32_t     stackVariant = 1;                      // LDS stack depth 16, 24 (default) or 32
     uint32_t     rayChunk     = 64;                     // rays per counter atomic
 };

@@ -143,7 +143,36 @@ __device__ __forceinline__ uint32_t Quantize21( double c, double lo, double hi )
     return f >= MORTON_CELLS - 1.0 ? ( 1u << MORTON_BITS ) - 1u : ( f <= 0.0 ? 0u : uint32_t( f ) );
 }
 
-__global__ __launch_bounds__( THREADS ) void k_morton( const float* tris, uint32_t n, const double* bounds, uint64_t* codes, uint64_t* keys, uint32_t* vals )
+// Key of the traversal's tree: the axes share one cell size, a 2^21st of the
+// longest extent.  Cells of the per-axis quantisation are as flat as the
+// scene, and so were the boxes: rays over a 256 x 256 terrain with 10 units
+// of height visited 13.5 (camera), 19.9 (bounce) and 20.8 (shadow) nodes,
+// and 8.3, 11.5 and 16.7 with cubic cells.
+__device__ __forceinline__ uint64_t CubicCode( const double c[ 3 ], const double* bounds )
+{
+    const double e = fmax( bounds[ 3 ] - bounds[ 0 ], fmax( bounds[ 4 ] - bounds[ 1 ], bounds[ 5 ] - bounds[ 2 ] ) );
+    return ( ExpandBits21( Quantize21( c[ 0 ], bounds[ 0 ], bounds[ 0 ] + e ) ) << 2 ) |
+           ( ExpandBits21( Quantize21( c[ 1 ], bounds[ 1 ], bounds[ 1 ] + e ) ) << 1 ) | ExpandBits21( Quantize21( c[ 2 ], bounds[ 2 ], bounds[ 2 ] + e ) );
+}
+
+__device__ __forceinline__ uint64_t AxisCode( const double c[ 3 ], const double* bounds )
+{
+    return ( ExpandBits21( Quantize21( c[ 0 ], bounds[ 0 ], bounds[ 3 ] ) ) << 2 ) | ( ExpandBits21( Quantize21( c[ 1 ], bounds[ 1 ], bounds[ 4 ] ) ) << 1 ) |
+           ExpandBits21( Quantize21( c[ 2 ], bounds[ 2 ], bounds[ 5 ] ) );
+}
+
+// Where a build's keys go: the traversal's tree, and the published one (null
+// codes: not asked for).
+struct KeyOut
+{
+    uint64_t* codes;
+    uint64_t* viewKeys;
+    uint32_t* viewVals;
+    uint64_t* keys;
+    uint32_t* vals;
+};
+
+__global__ __launch_bounds__( THREADS ) void k_morton( const float* tris, uint32_t n, const double* bounds, KeyOut o )
 {
     uint32_t i = blockIdx.x * THREADS + threadIdx.x;
     if( i >= n )
@@ -152,15 +181,15 @@ __global__ __launch_bounds__( THREADS ) void k_morton( const float* tris, uint32
     }
     double c[ 3 ];
     Centroid( tris, i, c );
-    uint32_t q[ 3 ];
-    for( int k = 0; k < 3; k++ )
+    o.keys[ i ] = CubicCode( c, bounds );
+    o.vals[ i ] = i;
+    if( o.codes )
     {
-        q[ k ] = Quantize21( c[ k ], bounds[ k ], bounds[ 3 + k ] );
+        const uint64_t code = AxisCode( c, bounds );
+        o.codes[ i ]        = code;
+        o.viewKeys[ i ]     = code;
+        o.viewVals[ i ]     = i;
     }
-    uint64_t code = ( ExpandBits21( q[ 0 ] ) << 2 ) | ( ExpandBits21( q[ 1 ] ) << 1 ) | ExpandBits21( q[ 2 ] );
-    codes[ i ]    = code;
-    keys[ i ]     = code;
-    vals[ i ]     = i;
 }
 
 // ------------------------------------------------------ batched scenes
@@ -247,30 +276,30 @@ __global__ void k_bounds_final_seg( const double* partials, uint32_t B, double* 
 // groups the scenes and orders each by its Morton curve, and the Karras
 // hierarchy over the keys splits at scene boundaries first.
 __global__ __launch_bounds__( THREADS ) void k_morton_seg( const float* tris, uint32_t n, const uint32_t* offsets, uint32_t S,
-                                                           const double* bounds, uint64_t* codes, uint64_t* keys, uint32_t* vals )
+                                                           const double* bounds, KeyOut o )
 {
     uint32_t i = blockIdx.x * THREADS + threadIdx.x;
     if( i >= n )
     {
         return;
     }
-    const uint32_t scene = SceneOf( offsets, S, i );
-    const double*  bb    = bounds + size_t( scene ) * 6;
+    const uint64_t scene = SceneOf( offsets, S, i );
+    const double*  bb    = bounds + scene * 6;
     double         c[ 3 ];
     Centroid( tris, i, c );
-    uint32_t q[ 3 ];
-    for( int k = 0; k < 3; k++ )
+    o.keys[ i ] = ( scene << 57 ) | ( CubicCode( c, bb ) >> 6 );
+    o.vals[ i ] = i;
+    if( o.codes )
     {
-        q[ k ] = Quantize21( c[ k ], bb[ k ], bb[ 3 + k ] );
+        const uint64_t code = AxisCode( c, bb );
+        o.codes[ i ]        = code;
+        o.viewKeys[ i ]     = ( scene << 57 ) | ( code >> 6 );
+        o.viewVals[ i ]     = i;
     }
-    const uint64_t code = ( ExpandBits21( q[ 0 ] ) << 2 ) | ( ExpandBits21( q[ 1 ] ) << 1 ) | ExpandBits21( q[ 2 ] );
-    codes[ i ]          = code;
-    keys[ i ]           = ( uint64_t( scene ) << 57 ) | ( code >> 6 );
-    vals[ i ]           = i;
 }
 
-// The internal node whose range is exactly scene s (each scene has >= 2
-// triangles, and its keys differ from its neighbours' in the scene bits).
+// The internal node whose range is exactly scene s (its keys differ from its
+// neighbours' in the scene bits); none for a one-triangle scene.
 __global__ __launch_bounds__( THREADS ) void k_scene_roots( uint32_t internal, const uint32_t* rf, const uint32_t* rl, const uint32_t* offsets,
                                                             uint32_t S, uint32_t* roots )
 {
@@ -286,9 +315,12 @@ __global__ __launch_bounds__( THREADS ) void k_scene_roots( uint32_t internal, c
     }
 }
 
-// Seeds the collapse with every scene root; a one-triangle scene (frame
-// segments only) has no internal node and is left out.
-__global__ void k_seed_frontier_seg( const uint32_t* roots, uint32_t S, uint32_t* frontier, uint32_t* counts )
+// Seeds a collapse with every scene root.  A one-triangle scene (frame
+// segments only) has no internal node: the published tree leaves it out, the
+// traversal's tree gives it a node of one leaf, so that scene s's root is
+// its node s.  With boxes: each root's box (lo xyz, hi xyz, 2 unused).
+__global__ void k_seed_frontier_seg( const uint32_t* roots, uint32_t S, const uint32_t* offsets, uint32_t internal, bool leaves, uint32_t* queue,
+                                     uint32_t* counts, const float* bounds, float* boxes )
 {
     if( threadIdx.x == 0 )
     {
@@ -297,77 +329,57 @@ __global__ void k_seed_frontier_seg( const uint32_t* roots, uint32_t S, uint32_t
         {
             if( roots[ s ] != 0xFFFFFFFFu )
             {
-                frontier[ k++ ] = roots[ s ];
+                queue[ k++ ] = roots[ s ];
+            }
+            else if( leaves )
+            {
+                queue[ k++ ] = internal + offsets[ s ];
             }
         }
         counts[ 0 ] = k;
     }
+    if( boxes && threadIdx.x < S )
+    {
+        const uint32_t s  = threadIdx.x;
+        const uint32_t id = roots[ s ] != 0xFFFFFFFFu ? roots[ s ] : internal + offsets[ s ];
+        for( int k = 0; k < 6; k++ )
+        {
+            boxes[ s * 8 + k ] = bounds[ size_t( id ) * 6 + k ];
+        }
+        boxes[ s * 8 + 6 ] = boxes[ s * 8 + 7 ] = 0.0f;
+    }
 }
 
-// 8-wide root of each scene; a one-triangle scene's root is the leaf of its
-// triangle, which the sort left at the scene's first position.
-__global__ void k_gather_roots8( const uint32_t* roots, const uint32_t* offsets, uint32_t S, const uint32_t* node8Index, uint32_t* roots8 )
+// 8-wide root of each scene of the published tree.
+__global__ void k_gather_roots8( const uint32_t* roots, uint32_t S, const uint32_t* node8Index, uint32_t* roots8 )
 {
     for( uint32_t s = threadIdx.x; s < S; s += blockDim.x )
     {
-        roots8[ s ] = roots[ s ] != 0xFFFFFFFFu ? node8Index[ roots[ s ] ] : ( RG_EXT_BVH_CHILD_LEAF_BIT | ( offsets[ s ] << 3 ) );
+        roots8[ s ] = roots[ s ] != 0xFFFFFFFFu ? node8Index[ roots[ s ] ] : 0xFFFFFFFFu;
     }
-}
-
-// Box of each frame segment's root: the union of an 8-wide root's child
-// boxes, or a one-triangle root's triangle box.  Out: 8 floats per segment
-// (lo xyz, hi xyz, 2 unused).
-__global__ void k_segment_boxes( const BvhNode8* nodes, const float4* sortedTris, const uint32_t* roots8, uint32_t S, float* out )
-{
-    const uint32_t s = threadIdx.x;
-    if( s >= S )
-    {
-        return;
-    }
-    float          lo[ 3 ] = { INFINITY, INFINITY, INFINITY }, hi[ 3 ] = { -INFINITY, -INFINITY, -INFINITY };
-    const uint32_t r       = roots8[ s ];
-    if( r & RG_EXT_BVH_CHILD_LEAF_BIT )
-    {
-        const uint32_t first = ( r >> 3 ) & 0x0FFFFFFFu;
-        for( uint32_t k = 0; k <= ( r & 7u ); k++ )
-        {
-            for( int v = 0; v < 3; v++ )
-            {
-                const float4 q = sortedTris[ size_t( first + k ) * 3 + v ];
-                lo[ 0 ] = fminf( lo[ 0 ], q.x ), hi[ 0 ] = fmaxf( hi[ 0 ], q.x );
-                lo[ 1 ] = fminf( lo[ 1 ], q.y ), hi[ 1 ] = fmaxf( hi[ 1 ], q.y );
-                lo[ 2 ] = fminf( lo[ 2 ], q.z ), hi[ 2 ] = fmaxf( hi[ 2 ], q.z );
-            }
-        }
-    }
-    else
-    {
-        const BvhNode8& nd = nodes[ r ];
-        for( int j = 0; j < 8; j++ )
-        {
-            if( nd.child[ j ] != RG_EXT_BVH_CHILD_EMPTY )
-            {
-                lo[ 0 ] = fminf( lo[ 0 ], nd.lo_x[ j ] ), hi[ 0 ] = fmaxf( hi[ 0 ], nd.hi_x[ j ] );
-                lo[ 1 ] = fminf( lo[ 1 ], nd.lo_y[ j ] ), hi[ 1 ] = fmaxf( hi[ 1 ], nd.hi_y[ j ] );
-                lo[ 2 ] = fminf( lo[ 2 ], nd.lo_z[ j ] ), hi[ 2 ] = fmaxf( hi[ 2 ], nd.hi_z[ j ] );
-            }
-        }
-    }
-    for( int k = 0; k < 3; k++ )
-    {
-        out[ s * 8 + k ]     = lo[ k ];
-        out[ s * 8 + 3 + k ] = hi[ k ];
-    }
-    out[ s * 8 + 6 ] = 0.0f;
-    out[ s * 8 + 7 ] = 0.0f;
 }
 
 // --------------------------------------------------------- radix sort
 // One pass = three launches: digit counts per tile, one block per digit that
-// scans its counts over the tiles, and the scatter.
-
-__global__ __launch_bounds__( THREADS ) void k_radix_hist( const uint64_t* keys, uint32_t n, int shift, uint32_t* hist, uint32_t numBlocks )
+// scans its counts over the tiles, and the scatter.  The two trees of a
+// build go through every launch together (blockIdx.y): the launches are
+// bound by their latency far more than by the keys they move.
+struct SortSet
 {
+    uint64_t* keys[ 2 ];
+    uint32_t* vals[ 2 ];
+    uint32_t* hist;   // 256 x tiles
+    uint32_t* totals; // 256
+};
+struct SortSets
+{
+    SortSet s[ 2 ];
+};
+
+__global__ __launch_bounds__( THREADS ) void k_radix_hist( SortSets sets, int from, uint32_t n, int shift, uint32_t numBlocks )
+{
+    const uint64_t* keys = sets.s[ blockIdx.y ].keys[ from ];
+    uint32_t*       hist = sets.s[ blockIdx.y ].hist;
     __shared__ uint32_t cnt[ 256 ];
     cnt[ threadIdx.x ] = 0;
     __syncthreads();
@@ -421,10 +433,10 @@ __device__ __forceinline__ uint32_t BlockExclusive( uint32_t v, uint32_t* s_wave
 
 // Block d: the exclusive sums of digit d's counts over the tiles, in place,
 // and the digit's total.
-__global__ __launch_bounds__( THREADS ) void k_radix_scan( uint32_t* hist, uint32_t* totals, uint32_t numBlocks )
+__global__ __launch_bounds__( THREADS ) void k_radix_scan( SortSets sets, uint32_t numBlocks )
 {
     __shared__ uint32_t s_wave[ THREADS / 64 ];
-    uint32_t*           h   = hist + size_t( blockIdx.x ) * numBlocks;
+    uint32_t*           h   = sets.s[ blockIdx.y ].hist + size_t( blockIdx.x ) * numBlocks;
     uint32_t            run = 0;
     for( uint32_t base = 0; base < numBlocks; base += THREADS )
     {
@@ -440,7 +452,7 @@ __global__ __launch_bounds__( THREADS ) void k_radix_scan( uint32_t* hist, uint3
     }
     if( threadIdx.x == 0 )
     {
-        totals[ blockIdx.x ] = run;
+        sets.s[ blockIdx.y ].totals[ blockIdx.x ] = run;
     }
 }
 
@@ -450,16 +462,15 @@ __global__ __launch_bounds__( THREADS ) void k_radix_scan( uint32_t* hist, uint3
 // then ordered in LDS and written out digit by digit, in runs.  1M pairs:
 // 19 us with one barrier-separated round per 256 keys and scattered stores,
 // 11 us like this (24 MB moved).
-__global__ __launch_bounds__( THREADS ) void k_radix_scatter( const uint64_t* keysIn,
-                                                              const uint32_t* valsIn,
-                                                              uint64_t*       keysOut,
-                                                              uint32_t*       valsOut,
-                                                              uint32_t        n,
-                                                              int             shift,
-                                                              const uint32_t* offsets,
-                                                              const uint32_t* totals,
-                                                              uint32_t        numBlocks )
+__global__ __launch_bounds__( THREADS ) void k_radix_scatter( SortSets sets, int from, uint32_t n, int shift, uint32_t numBlocks )
 {
+    const SortSet&      set     = sets.s[ blockIdx.y ];
+    const uint64_t*     keysIn  = set.keys[ from ];
+    const uint32_t*     valsIn  = set.vals[ from ];
+    uint64_t*           keysOut = set.keys[ from ^ 1 ];
+    uint32_t*           valsOut = set.vals[ from ^ 1 ];
+    const uint32_t*     offsets = set.hist;
+    const uint32_t*     totals  = set.totals;
     constexpr int       WAVES = THREADS / 64;
     __shared__ uint32_t s_cnt[ WAVES ][ 256 ]; // per wave: counts, then first positions in the tile
     __shared__ uint32_t s_out[ 256 ];          // global position of a digit's keys minus their position in the tile
@@ -627,9 +638,14 @@ struct TreeArgs
 // of BUILD_LISTS lists.  The collapse's record of an internal node: its two
 // children, each with OPEN_BIT set when it may be opened (internal, more
 // than leafMax triangles), and their half areas (-1 for the others).
-template< bool LEAVES, int PER >
-__global__ __launch_bounds__( THREADS ) void k_tree( TreeArgs a )
+struct TreeSets
 {
+    TreeArgs s[ 2 ];
+};
+template< bool LEAVES, int PER >
+__global__ __launch_bounds__( THREADS ) void k_tree( TreeSets sets )
+{
+    const TreeArgs&     a = sets.s[ blockIdx.y ];
     constexpr int       CAP = PER * THREADS;
     static_assert( LEAVES || CAP >= int( BUILD_LISTS * BUILD_LIST_CAP ), "element capacity" );
     __shared__ float    s_box[ 6 ][ CAP ];
@@ -856,17 +872,34 @@ __device__ __forceinline__ uint32_t NodeCount( uint32_t id, uint32_t n, const ui
 // level's follow them, each wave taking room for its nodes with one atomic
 // (one per child on a single address took 131 and 197 us for the two widest
 // levels of a 1M-triangle build).
-__global__ __launch_bounds__( THREADS ) void k_collapse_level( uint32_t*       queue,
-                                                               uint32_t*       levelBase,
-                                                               uint32_t*       levelCount,
-                                                               uint32_t        n,
-                                                               uint32_t        leafMax,
-                                                               const uint4*    info,
-                                                               const uint32_t* rf,
-                                                               const uint32_t* rl,
-                                                               uint32_t*       expansion,
-                                                               uint32_t*       isNode8 )
+struct CollapseArgs
 {
+    uint32_t*       queue;
+    uint32_t*       levelBase;
+    uint32_t*       levelCount;
+    uint32_t        n;
+    uint32_t        leafMax;
+    const uint4*    info;
+    const uint32_t* rf;
+    const uint32_t* rl;
+    uint32_t*       expansion;
+    uint32_t*       isNode8;   // published tree: marks, by binary node
+    uint2*          nodeBase;  // traversal's tree: first child node and first triangle of each node
+    uint32_t*       triCount;
+};
+struct CollapseSets
+{
+    CollapseArgs s[ 2 ];
+};
+
+__global__ __launch_bounds__( THREADS ) void k_collapse_level( CollapseSets sets, uint32_t level )
+{
+    const CollapseArgs& a          = sets.s[ blockIdx.y ];
+    uint32_t* const     queue      = a.queue;
+    uint32_t* const     levelBase  = a.levelBase + level;
+    uint32_t* const     levelCount = a.levelCount + level;
+    const uint32_t      n = a.n, leafMax = a.leafMax;
+    const uint4* const  info = a.info;
     const uint32_t count = levelCount[ 0 ], first = levelBase[ 0 ];
     const int      lane  = threadIdx.x & 63;
     if( blockIdx.x == 0 && threadIdx.x == 0 )
@@ -897,7 +930,7 @@ __global__ __launch_bounds__( THREADS ) void k_collapse_level( uint32_t*       q
         if( !have )
         {
         }
-        else if( b >= n - 1 || NodeCount( b, n, rf, rl ) <= leafMax )
+        else if( b >= n - 1 || NodeCount( b, n, a.rf, a.rl ) <= leafMax )
         {
             ch[ 0 ] = b; // a root that is small enough is a single leaf
             nch     = 1;
@@ -979,10 +1012,13 @@ __global__ __launch_bounds__( THREADS ) void k_collapse_level( uint32_t*       q
             {
                 out[ k ] = k < nch ? ( ch[ k ] | ( ex[ k ] ? OPEN_BIT : 0u ) ) : 0xFFFFFFFFu;
             }
-            uint4* e = reinterpret_cast< uint4* >( expansion ) + size_t( first + t ) * 2;
+            uint4* e = reinterpret_cast< uint4* >( a.expansion ) + size_t( first + t ) * 2;
             e[ 0 ]   = make_uint4( out[ 0 ], out[ 1 ], out[ 2 ], out[ 3 ] );
             e[ 1 ]   = make_uint4( out[ 4 ], out[ 5 ], out[ 6 ], out[ 7 ] );
-            isNode8[ b < n - 1 ? b : 0 ] = 1u;
+            if( a.isNode8 )
+            {
+                a.isNode8[ b < n - 1 ? b : 0 ] = 1u;
+            }
         }
         uint32_t kids = 0;
 #pragma unroll
@@ -990,13 +1026,30 @@ __global__ __launch_bounds__( THREADS ) void k_collapse_level( uint32_t*       q
         {
             kids += k < nch && ex[ k ] ? 1u : 0u;
         }
-        const uint32_t inc  = WaveInclusive( kids, lane );
-        uint32_t       base = 0;
-        if( lane == 63 && inc != 0u )
+        // child nodes in the low half, leaf children in the high half
+        const uint32_t own  = kids | ( uint32_t( nch ) - kids ) << 16;
+        const uint32_t inc  = WaveInclusive( own, lane );
+        uint32_t       base = 0, tri = 0;
+        if( lane == 63 )
         {
-            base = atomicAdd( levelCount + 1, inc );
+            if( ( inc & 0xFFFFu ) != 0u )
+            {
+                base = atomicAdd( levelCount + 1, inc & 0xFFFFu );
+            }
+            if( a.nodeBase && ( inc >> 16 ) != 0u )
+            {
+                tri = atomicAdd( a.triCount, inc >> 16 );
+            }
         }
-        uint32_t pos = first + count + __shfl( base, 63, 64 ) + inc - kids;
+        uint32_t pos = first + count + __shfl( base, 63, 64 ) + ( ( inc - own ) & 0xFFFFu );
+        if( a.nodeBase )
+        {
+            tri = __shfl( tri, 63, 64 ) + ( ( inc - own ) >> 16 );
+            if( have )
+            {
+                a.nodeBase[ first + t ] = make_uint2( pos, tri );
+            }
+        }
 #pragma unroll
         for( int k = 0; k < 8; k++ )
         {
@@ -1157,32 +1210,162 @@ __global__ __launch_bounds__( THREADS ) void k_sorted_tris( const float* tris, c
     out[ size_t( k ) * 3 + 2 ] = make_float4( c.x, c.y, c.z, 0.0f );
 }
 
-__global__ void k_seed_frontier( uint32_t* queue, uint32_t* counts )
+// ----------------------------------------------------- traversal nodes
+
+// Box planes of an axis as bytes: scale 2^k and origin such that
+// origin + q * 2^k, q in 0..254, covers [lo, hi] with room to spare; 2^k is
+// no finer than four units in the last place of the coordinates, so that the
+// origin, half a step below lo and rounded to float, stays below it.  An axis whose
+// box is not finite gets an infinite scale and zero bytes: the traversal's
+// distances are then NaN, which its min / max leave out.
+struct AxisGrid
 {
-    queue[ 0 ]  = 0;
-    counts[ 0 ] = 1;
+    float    origin;
+    uint32_t exponent; // of the scale, biased as in a float
+};
+__device__ __forceinline__ AxisGrid MakeGrid( float lo, float hi )
+{
+    AxisGrid     g;
+    const double ext = double( hi ) - double( lo ), big = fmax( fabs( double( lo ) ), fabs( double( hi ) ) );
+    if( !( ext >= 0.0 && big < 1e36 ) )
+    {
+        g.origin   = 0.0f;
+        g.exponent = 255u;
+        return g;
+    }
+    int k = ext > 0.0 ? ilogb( ext / 252.0 ) : -126;
+    k     = ext > 0.0 && ldexp( 252.0, k ) < ext ? k + 1 : k;
+    const int fine = big > 0.0 ? ilogb( big ) - 21 : -126;
+    k              = k < fine ? fine : k;
+    k              = k < -126 ? -126 : k;
+    g.origin       = float( double( lo ) - ldexp( 0.5, k ) );
+    g.exponent     = uint32_t( k + 127 );
+    return g;
+}
+// The byte plane below lo or above hi.  The traversal evaluates
+// fma(q, 2^k / d, (origin - o) / d) with about 3e-5 steps of rounding error
+// beyond a relative one of a few units in the last place; 2^-10 steps of
+// margin cover it.
+__device__ __forceinline__ uint32_t GridLo( const AxisGrid& g, float v )
+{
+    if( g.exponent == 255u )
+    {
+        return 0u;
+    }
+    const double q = floor( ldexp( double( v ) - double( g.origin ), 127 - int( g.exponent ) ) - 0x1p-10 );
+    return q > 0.0 ? uint32_t( fmin( q, 255.0 ) ) : 0u; // NaN: 0
+}
+__device__ __forceinline__ uint32_t GridHi( const AxisGrid& g, float v )
+{
+    if( g.exponent == 255u )
+    {
+        return 0u;
+    }
+    const double q = ceil( ldexp( double( v ) - double( g.origin ), 127 - int( g.exponent ) ) + 0x1p-10 );
+    return q < 255.0 ? uint32_t( fmax( q, 0.0 ) ) : 255u; // NaN: 255
+}
+
+// One traversal node per node of the collapse's queue, eight lanes a node
+// (one per child), and its leaves' triangles side by side.
+__global__ __launch_bounds__( THREADS ) void k_pack_nodes( uint32_t count, uint32_t n, const uint32_t* expansion, const uint2* nodeBase,
+                                                           const float* bounds, const uint32_t* order, const float* tris, BvhNodeQ* nodes,
+                                                           float4* nodeTris )
+{
+    const uint64_t t    = uint64_t( blockIdx.x ) * THREADS + threadIdx.x;
+    const uint32_t q    = uint32_t( t >> 3 );
+    const bool     have = q < count;
+    const uint32_t e    = have ? expansion[ t ] : 0xFFFFFFFFu;
+    const bool     full = e != 0xFFFFFFFFu, inner = full && ( e & OPEN_BIT ) != 0u;
+    const uint32_t c    = e & ~OPEN_BIT;
+    const int      lane = threadIdx.x & 63, first = lane & ~7;
+
+    float lo[ 3 ] = { INFINITY, INFINITY, INFINITY }, hi[ 3 ] = { -INFINITY, -INFINITY, -INFINITY };
+    if( full )
+    {
+        const float2* bb = reinterpret_cast< const float2* >( bounds + size_t( c ) * 6 );
+        const float2  x = bb[ 0 ], y = bb[ 1 ], z = bb[ 2 ];
+        lo[ 0 ] = x.x, lo[ 1 ] = x.y, lo[ 2 ] = y.x, hi[ 0 ] = y.y, hi[ 1 ] = z.x, hi[ 2 ] = z.y;
+    }
+    const uint32_t inMask   = uint32_t( __ballot( inner ) >> first ) & 0xFFu;
+    const uint32_t leafMask = uint32_t( __ballot( full && !inner ) >> first ) & 0xFFu;
+    const uint32_t below    = ( 1u << ( lane & 7 ) ) - 1u;
+    const uint32_t inner8 = __popc( inMask ), leaf8 = __popc( leafMask );
+    // child nodes take the first slots, leaves the next ones
+    const uint32_t slot = inner ? __popc( inMask & below ) : ( full ? inner8 + __popc( leafMask & below ) : inner8 + leaf8 + __popc( ~( inMask | leafMask ) & below ) );
+    AxisGrid       g[ 3 ];
+#pragma unroll
+    for( int ax = 0; ax < 3; ax++ )
+    {
+        float l = lo[ ax ], h = hi[ ax ];
+#pragma unroll
+        for( int m = 1; m < 8; m <<= 1 )
+        {
+            l = fminf( l, __shfl_xor( l, m, 64 ) );
+            h = fmaxf( h, __shfl_xor( h, m, 64 ) );
+        }
+        g[ ax ] = MakeGrid( l, h );
+    }
+    if( !have )
+    {
+        return;
+    }
+    BvhNodeQ&   node = nodes[ q ];
+    const uint2 base = nodeBase[ q ];
+#pragma unroll
+    for( int ax = 0; ax < 3; ax++ )
+    {
+        node.lo[ ax ][ slot ] = uint8_t( full ? GridLo( g[ ax ], lo[ ax ] ) : 255u );
+        node.hi[ ax ][ slot ] = uint8_t( full ? GridHi( g[ ax ], hi[ ax ] ) : 0u );
+    }
+    if( ( lane & 7 ) == 0 )
+    {
+        node.origin[ 0 ] = g[ 0 ].origin;
+        node.origin[ 1 ] = g[ 1 ].origin;
+        node.origin[ 2 ] = g[ 2 ].origin;
+        node.meta        = g[ 0 ].exponent | g[ 1 ].exponent << 8 | g[ 2 ].exponent << 16 | inner8 << 24 | leaf8 << 28;
+        node.childBase   = base.x;
+        node.triBase     = base.y - inner8; // leaf slot s holds triangle triBase + s
+        node.pad[ 0 ] = node.pad[ 1 ] = 0u;
+    }
+    if( full && !inner )
+    {
+        const uint32_t id = order[ c - ( n - 1 ) ];
+        v3             v0, v1, v2;
+        LoadTri( tris, id, v0, v1, v2 );
+        float4* o = nodeTris + size_t( base.y + slot - inner8 ) * 3;
+        o[ 0 ]    = make_float4( v0.x, v0.y, v0.z, __uint_as_float( id ) );
+        o[ 1 ]    = make_float4( v1.x, v1.y, v1.z, 0.0f );
+        o[ 2 ]    = make_float4( v2.x, v2.y, v2.z, 0.0f );
+    }
+}
+
+__global__ void k_seed_frontier( CollapseSets sets, uint32_t count )
+{
+    if( threadIdx.x < count )
+    {
+        sets.s[ threadIdx.x ].queue[ 0 ]      = 0;
+        sets.s[ threadIdx.x ].levelCount[ 0 ] = 1;
+    }
 }
 
 } // namespace
 
 namespace
 {
-// Stable sort of n (key, value) pairs by key bits [lo, hi); on return *kin and
-// *vin hold the result.  hist: 256 words per tile and 256 more.
-void RadixSort( uint64_t** kin, uint64_t** kout, uint32_t** vin, uint32_t** vout, uint32_t n, int lo, int hi, uint32_t* hist, hipStream_t stream )
+// Stable sort of n (key, value) pairs of `count` sets by key bits [0, 64):
+// an even number of passes, so the result is where the input was.
+void RadixSort( const SortSets& sets, uint32_t count, uint32_t n, hipStream_t stream )
 {
     const uint32_t blocks = DivUp( n, RS_TILE );
-    uint32_t*      totals = hist + size_t( 256 ) * blocks;
-    for( int shift = lo; shift < hi; shift += 8 )
+    for( int pass = 0; pass < 8; pass++ )
     {
-        k_radix_hist<<< blocks, THREADS, 0, stream >>>( *kin, n, shift, hist, blocks );
+        const int from = pass & 1, shift = pass * 8;
+        k_radix_hist<<< dim3( blocks, count ), THREADS, 0, stream >>>( sets, from, n, shift, blocks );
         CheckLaunch( "k_radix_hist" );
-        k_radix_scan<<< 256, THREADS, 0, stream >>>( hist, totals, blocks );
+        k_radix_scan<<< dim3( 256, count ), THREADS, 0, stream >>>( sets, blocks );
         CheckLaunch( "k_radix_scan" );
-        k_radix_scatter<<< blocks, THREADS, 0, stream >>>( *kin, *vin, *kout, *vout, n, shift, hist, totals, blocks );
+        k_radix_scatter<<< dim3( blocks, count ), THREADS, 0, stream >>>( sets, from, n, shift, blocks );
         CheckLaunch( "k_radix_scatter" );
-        std::swap( *kin, *kout );
-        std::swap( *vin, *vout );
     }
 }
 
@@ -1203,43 +1386,120 @@ size_t TreeListBytes( uint32_t n )
     return ( runs + next ) * ( BUILD_LIST_CAP * sizeof( uint2 ) + sizeof( uint32_t ) );
 }
 
-void BuildTree( TreeArgs a, uint2* lists, hipStream_t stream )
+void BuildTree( TreeSets a, uint2* const lists[ 2 ], uint32_t count, hipStream_t stream )
 {
-    uint32_t  runs = TreeRuns( a.n );
-    const uint32_t next = DivUp( runs, BUILD_LISTS );
-    uint2*    listA = lists;
-    uint2*    listB = listA + size_t( runs ) * BUILD_LIST_CAP;
-    uint32_t* cntA = reinterpret_cast< uint32_t* >( listB + size_t( next ) * BUILD_LIST_CAP );
-    uint32_t* cntB = cntA + runs;
-    a.listOut  = listA;
-    a.countOut = cntA;
-    if( a.n <= TREE_SMALL )
+    const uint32_t n    = a.s[ 0 ].n;
+    uint32_t       runs = TreeRuns( n );
+    const uint32_t first = runs, next = DivUp( runs, BUILD_LISTS );
+    auto           point = [ & ]( bool flip, bool in ) {
+        for( uint32_t k = 0; k < count; k++ )
+        {
+            uint2*    listA = lists[ k ];
+            uint2*    listB = listA + size_t( first ) * BUILD_LIST_CAP;
+            uint32_t* cntA  = reinterpret_cast< uint32_t* >( listB + size_t( next ) * BUILD_LIST_CAP );
+            uint32_t* cntB  = cntA + first;
+            if( in )
+            {
+                a.s[ k ].listIn  = flip ? listB : listA;
+                a.s[ k ].countIn = flip ? cntB : cntA;
+            }
+            else
+            {
+                a.s[ k ].listOut  = flip ? listB : listA;
+                a.s[ k ].countOut = flip ? cntB : cntA;
+            }
+        }
+    };
+    bool flip = false;
+    point( flip, false );
+    if( n <= TREE_SMALL )
     {
-        k_tree< true, 1 ><<< runs, THREADS, 0, stream >>>( a );
+        k_tree< true, 1 ><<< dim3( runs, count ), THREADS, 0, stream >>>( a );
     }
     else
     {
-        k_tree< true, 4 ><<< runs, THREADS, 0, stream >>>( a );
+        k_tree< true, 4 ><<< dim3( runs, count ), THREADS, 0, stream >>>( a );
     }
     CheckLaunch( "k_tree" );
     while( runs > 1 )
     {
-        a.listIn   = a.listOut;
-        a.countIn  = a.countOut;
-        a.lists    = runs;
-        a.listOut  = a.listOut == listA ? listB : listA;
-        a.countOut = a.countOut == cntA ? cntB : cntA;
-        runs       = DivUp( runs, BUILD_LISTS );
-        k_tree< false, int( BUILD_LISTS * BUILD_LIST_CAP / THREADS ) ><<< runs, THREADS, 0, stream >>>( a );
+        point( flip, true );
+        flip = !flip;
+        point( flip, false );
+        for( uint32_t k = 0; k < count; k++ )
+        {
+            a.s[ k ].lists = runs;
+        }
+        runs = DivUp( runs, BUILD_LISTS );
+        k_tree< false, int( BUILD_LISTS * BUILD_LIST_CAP / THREADS ) ><<< dim3( runs, count ), THREADS, 0, stream >>>( a );
         CheckLaunch( "k_tree" );
     }
 }
 
-// Shared by the single-scene and the batched build; `batch` (host offsets,
-// S + 1 of them) switches steps 1-2 to per-scene bounds and keys and seeds
-// the collapse with every scene's root.
+// Carves aligned arrays out of one allocation.
+struct Carver
+{
+    char*  base = nullptr;
+    size_t used = 0;
+    template< typename T >
+    T* Take( size_t count )
+    {
+        T* p = base ? reinterpret_cast< T* >( base + used ) : nullptr;
+        used += ( count * sizeof( T ) + 255 ) & ~size_t( 255 );
+        return p;
+    }
+};
+
+// Scratch of the traversal's tree.
+struct TreeScratch
+{
+    uint64_t *keys0, *keys1;
+    uint32_t *vals0, *vals1, *hist;
+    uint2*    children;
+    uint32_t *rf, *rl;
+    float*    bounds;
+    uint4*    info;
+    uint2*    lists;
+    uint32_t *expansion, *queue;
+    uint2*    nodeBase;
+    uint32_t* roots;
+    float*    boxes;
+    uint32_t* levels; // per set: nodes of each level, then its first node; one more word for the triangle count
+    size_t    bytes;
+
+    TreeScratch( char* base, uint32_t n, uint32_t sceneCount )
+    {
+        Carver       c{ base };
+        const size_t slots = n > 1 ? n - 1 : 1;
+        keys0     = c.Take< uint64_t >( n );
+        keys1     = c.Take< uint64_t >( n );
+        vals0     = c.Take< uint32_t >( n );
+        vals1     = c.Take< uint32_t >( n );
+        hist      = c.Take< uint32_t >( size_t( 256 ) * ( DivUp( n, RS_TILE ) + 1 ) );
+        children  = c.Take< uint2 >( slots );
+        rf        = c.Take< uint32_t >( slots );
+        rl        = c.Take< uint32_t >( slots );
+        bounds    = c.Take< float >( ( 2 * size_t( n ) - 1 ) * 6 );
+        info      = c.Take< uint4 >( slots );
+        lists     = c.Take< uint2 >( TreeListBytes( n ) / sizeof( uint2 ) + 1 );
+        expansion = c.Take< uint32_t >( ( slots + sceneCount ) * 8 ); // one-triangle scenes have nodes of their own
+        queue     = c.Take< uint32_t >( slots + sceneCount );
+        nodeBase  = c.Take< uint2 >( slots + sceneCount );
+        roots     = c.Take< uint32_t >( sceneCount + 1 );
+        boxes     = c.Take< float >( size_t( sceneCount + 1 ) * 8 );
+        levels    = c.Take< uint32_t >( LEVEL_WORDS * 2 + 1 );
+        bytes     = c.used;
+    }
+    static constexpr uint32_t LEVEL_WORDS = ( BVH_MAX_LEVELS + 1 ) * 2;
+};
+
+// Builds the traversal's tree (nodesQ, nodeTris) over the cubic keys and,
+// with `view`, the published LBVH (codes, order, binary tree, nodes) over
+// the per-axis ones, the two side by side through the same launches.
+// batchOffsets (host, S + 1 of them) switches to per-scene bounds and keys
+// and seeds the collapse with every scene's root.
 void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtBvhBuildParams& params, const uint32_t* batchOffsets,
-                   uint32_t sceneCount, hipStream_t stream, bool segmentBoxes = false )
+                   uint32_t sceneCount, hipStream_t stream, bool view )
 {
     RG_REQUIRE( n > 0, RG_RESULT_WRONG_FUNCTION_ARGUMENT, "triangle count must be > 0" );
     RG_REQUIRE( n < ( 1u << 28 ), RG_RESULT_WRONG_FUNCTION_ARGUMENT, "triangle count must be < 2^28" );
@@ -1247,61 +1507,78 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
     RG_REQUIRE( params.nodeFormat == RG_EXT_BVH_NODE_FP32 || params.nodeFormat == RG_EXT_BVH_NODE_FP16, RG_RESULT_WRONG_FUNCTION_ARGUMENT,
                 "unknown node format" );
 
-    bvh.n          = n;
-    bvh.leafMax    = params.maxLeafSize;
-    bvh.nodeFormat = params.nodeFormat;
+    const bool batched = batchOffsets != nullptr;
+    bvh.n              = n;
+    bvh.leafMax        = params.maxLeafSize;
+    bvh.nodeFormat     = params.nodeFormat;
+    bvh.nodeCount      = 0; // until the build is done
+    bvh.nodeCountQ     = 0;
+    bvh.sceneCount     = batched ? sceneCount : 0u;
 
-    const uint32_t internal   = n - 1;
-    const uint32_t slots      = internal > 0 ? internal : 1;
-    const uint32_t rsBlocks   = DivUp( n, RS_TILE );
-    const uint32_t bndBlocks  = DivUp( n, THREADS ) < 1024 ? DivUp( n, THREADS ) : 1024;
+    const uint32_t internal  = n - 1;
+    const uint32_t slots     = internal > 0 ? internal : 1;
+    const uint32_t rsBlocks  = DivUp( n, RS_TILE );
+    const uint32_t bndBlocks = DivUp( n, THREADS ) < 1024 ? DivUp( n, THREADS ) : 1024;
+    const uint32_t sets      = view ? 2 : 1; // set 0: the traversal's tree, set 1: the published one
+    const uint32_t S         = batched ? sceneCount : 0u;
 
-    bvh.sortedTris.Reserve( size_t( n ) * 48 );
-    bvh.codes.Reserve( size_t( n ) * 8 );
-    bvh.keysA.Reserve( size_t( n ) * 8 );
-    bvh.keysB.Reserve( size_t( n ) * 8 );
-    bvh.valsA.Reserve( size_t( n ) * 4 );
-    bvh.valsB.Reserve( size_t( n ) * 4 );
-    bvh.hist.Reserve( size_t( 256 ) * ( rsBlocks + 1 ) * 4 );
-    bvh.scanScratch.Reserve( ScanScratchBytes( slots ) );
+    bvh.scratch.Reserve( TreeScratch( nullptr, n, S ).bytes );
+    const TreeScratch ts( bvh.scratch.as< char >(), n, S );
+    bvh.nodeTris.Reserve( size_t( n ) * 48 );
     bvh.boundsPartials.Reserve( size_t( bndBlocks + 1 ) * 6 * 8 );
-    bvh.children.Reserve( size_t( slots ) * 8 );
-    bvh.rangeFirst.Reserve( size_t( slots ) * 4 );
-    bvh.rangeLast.Reserve( size_t( slots ) * 4 );
-    bvh.nodeBounds.Reserve( size_t( 2 * n - 1 ) * 24 );
-    bvh.expandInfo.Reserve( size_t( slots ) * sizeof( uint4 ) );
-    bvh.treeLists.Reserve( TreeListBytes( n ) );
-    bvh.expansion.Reserve( size_t( slots ) * 32 );
-    bvh.isNode8.Reserve( size_t( slots ) * 4 );
-    bvh.node8Index.Reserve( size_t( slots ) * 4 );
-    bvh.queue.Reserve( size_t( slots ) * 4 );
-    bvh.levelCounts.Reserve( ( BVH_MAX_LEVELS + 1 ) * 2 * 4 );
-    if( !bvh.hostCounts )
+    if( !bvh.hostLevels )
     {
-        RG_HIP_CHECK( hipHostMalloc( reinterpret_cast< void** >( &bvh.hostCounts ), 2 * 4, hipHostMallocDefault ) );
+        RG_HIP_CHECK( hipHostMalloc( reinterpret_cast< void** >( &bvh.hostLevels ), TreeScratch::LEVEL_WORDS * 2 * 4, hipHostMallocDefault ) );
+    }
+    if( view )
+    {
+        bvh.sortedTris.Reserve( size_t( n ) * 48 );
+        bvh.codes.Reserve( size_t( n ) * 8 );
+        bvh.keysA.Reserve( size_t( n ) * 8 );
+        bvh.keysB.Reserve( size_t( n ) * 8 );
+        bvh.valsA.Reserve( size_t( n ) * 4 );
+        bvh.valsB.Reserve( size_t( n ) * 4 );
+        bvh.hist.Reserve( size_t( 256 ) * ( rsBlocks + 1 ) * 4 );
+        bvh.scanScratch.Reserve( ScanScratchBytes( slots ) );
+        bvh.children.Reserve( size_t( slots ) * 8 );
+        bvh.rangeFirst.Reserve( size_t( slots ) * 4 );
+        bvh.rangeLast.Reserve( size_t( slots ) * 4 );
+        bvh.nodeBounds.Reserve( ( 2 * size_t( n ) - 1 ) * 24 );
+        bvh.expandInfo.Reserve( size_t( slots ) * sizeof( uint4 ) );
+        bvh.treeLists.Reserve( TreeListBytes( n ) );
+        bvh.expansion.Reserve( size_t( slots ) * 32 );
+        bvh.isNode8.Reserve( size_t( slots ) * 4 );
+        bvh.node8Index.Reserve( size_t( slots ) * 4 );
+        bvh.queue.Reserve( size_t( slots ) * 4 );
     }
 
-    double* partials    = bvh.boundsPartials.as< double >();
-    double* sceneBounds = partials + size_t( bndBlocks ) * 6;
-    const bool batched  = batchOffsets != nullptr;
-    bvh.sceneCount      = batched ? sceneCount : 0u;
-
-    if( !batched )
+    // 1. FP64 centroid bounds and 2. Morton keys (input order) with the
+    // identity permutation, per scene in a batch.
+    double*  partials    = bvh.boundsPartials.as< double >();
+    double*  sceneBounds = partials + size_t( bndBlocks ) * 6;
+    uint32_t* offs       = nullptr;
+    KeyOut   ko{ nullptr, nullptr, nullptr, ts.keys0, ts.vals0 };
+    if( view )
     {
-        // 1. FP64 centroid bounds.
+        ko.codes    = bvh.codes.as< uint64_t >();
+        ko.viewKeys = bvh.keysA.as< uint64_t >();
+        ko.viewVals = bvh.valsA.as< uint32_t >();
+    }
+    if( !batched || view )
+    {
+        // (a batch keeps these for the view's fields alone)
         k_centroid_bounds<<< bndBlocks, THREADS, 0, stream >>>( d_tris, n, partials );
         CheckLaunch( "k_centroid_bounds" );
         k_bounds_final<<< 1, THREADS, 0, stream >>>( partials, bndBlocks, sceneBounds );
         CheckLaunch( "k_bounds_final" );
-
-        // 2. Morton codes (input order) and the identity permutation.
-        k_morton<<< DivUp( n, THREADS ), THREADS, 0, stream >>>( d_tris, n, sceneBounds, bvh.codes.as< uint64_t >(), bvh.keysA.as< uint64_t >(), bvh.valsA.as< uint32_t >() );
+    }
+    if( !batched )
+    {
+        k_morton<<< DivUp( n, THREADS ), THREADS, 0, stream >>>( d_tris, n, sceneBounds, ko );
         CheckLaunch( "k_morton" );
     }
     else
     {
-        // 1-2 per scene: bounds of each scene's centroids, then keys with the
-        // scene in the top bits
         const uint32_t B = 16;
         bvh.sceneOffsets.Reserve( size_t( sceneCount + 1 ) * 4 );
         bvh.sceneRoots.Reserve( size_t( sceneCount ) * 4 );
@@ -1310,70 +1587,82 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
         bvh.scenePartials.Reserve( size_t( sceneCount ) * B * 6 * 8 );
         bvh.hostSceneOffsets.assign( batchOffsets, batchOffsets + sceneCount + 1 );
         RG_HIP_CHECK( hipMemcpyAsync( bvh.sceneOffsets.ptr, bvh.hostSceneOffsets.data(), size_t( sceneCount + 1 ) * 4, hipMemcpyHostToDevice, stream ) );
-        const uint32_t* offs = bvh.sceneOffsets.as< uint32_t >();
+        offs = bvh.sceneOffsets.as< uint32_t >();
         k_centroid_bounds_seg<<< sceneCount * B, THREADS, 0, stream >>>( d_tris, offs, B, bvh.scenePartials.as< double >() );
         CheckLaunch( "k_centroid_bounds_seg" );
         k_bounds_final_seg<<< sceneCount, 64, 0, stream >>>( bvh.scenePartials.as< double >(), B, bvh.sceneBounds.as< double >() );
         CheckLaunch( "k_bounds_final_seg" );
-        k_morton_seg<<< DivUp( n, THREADS ), THREADS, 0, stream >>>( d_tris, n, offs, sceneCount, bvh.sceneBounds.as< double >(),
-                                                                     bvh.codes.as< uint64_t >(), bvh.keysA.as< uint64_t >(), bvh.valsA.as< uint32_t >() );
+        k_morton_seg<<< DivUp( n, THREADS ), THREADS, 0, stream >>>( d_tris, n, offs, sceneCount, bvh.sceneBounds.as< double >(), ko );
         CheckLaunch( "k_morton_seg" );
-        // the whole-batch bounds are not used; keep the view's fields defined
-        k_centroid_bounds<<< bndBlocks, THREADS, 0, stream >>>( d_tris, n, partials );
-        CheckLaunch( "k_centroid_bounds" );
-        k_bounds_final<<< 1, THREADS, 0, stream >>>( partials, bndBlocks, sceneBounds );
-        CheckLaunch( "k_bounds_final" );
     }
 
     // 3. Stable LSD radix sort, 8 passes of 8 bits.
-    uint64_t* kin  = bvh.keysA.as< uint64_t >();
-    uint64_t* kout = bvh.keysB.as< uint64_t >();
-    uint32_t* vin  = bvh.valsA.as< uint32_t >();
-    uint32_t* vout = bvh.valsB.as< uint32_t >();
-    RadixSort( &kin, &kout, &vin, &vout, n, 0, 64, bvh.hist.as< uint32_t >(), stream );
-    bvh.sortedKeys = kin;
-    bvh.sortedIdx  = vin;
+    SortSets ss{};
+    ss.s[ 0 ] = SortSet{ { ts.keys0, ts.keys1 }, { ts.vals0, ts.vals1 }, ts.hist, ts.hist + size_t( 256 ) * rsBlocks };
+    if( view )
+    {
+        ss.s[ 1 ] = SortSet{ { bvh.keysA.as< uint64_t >(), bvh.keysB.as< uint64_t >() },
+                             { bvh.valsA.as< uint32_t >(), bvh.valsB.as< uint32_t >() },
+                             bvh.hist.as< uint32_t >(),
+                             bvh.hist.as< uint32_t >() + size_t( 256 ) * rsBlocks };
+    }
+    RadixSort( ss, sets, n, stream );
+    bvh.sortedIdx = view ? bvh.valsA.as< uint32_t >() : nullptr;
 
-    // 4. The binary hierarchy with its boxes.
-    uint32_t* children = bvh.children.as< uint32_t >();
-    uint32_t* rf       = bvh.rangeFirst.as< uint32_t >();
-    uint32_t* rl       = bvh.rangeLast.as< uint32_t >();
-    float*    bounds   = bvh.nodeBounds.as< float >();
-    TreeArgs  ta{};
-    ta.tris       = d_tris;
-    ta.keys       = kin;
-    ta.order      = vin;
-    ta.n          = n;
-    ta.leafMax    = bvh.leafMax;
-    ta.children   = bvh.children.as< uint2 >();
-    ta.rangeFirst = rf;
-    ta.rangeLast  = rl;
-    ta.bounds     = bounds;
-    ta.info       = bvh.expandInfo.as< uint4 >();
-    BuildTree( ta, bvh.treeLists.as< uint2 >(), stream );
+    // 4. The binary hierarchies with their boxes.
+    uint32_t* rf     = view ? bvh.rangeFirst.as< uint32_t >() : nullptr;
+    uint32_t* rl     = view ? bvh.rangeLast.as< uint32_t >() : nullptr;
+    float*    bounds = view ? bvh.nodeBounds.as< float >() : nullptr;
+    TreeSets  ta{};
+    ta.s[ 0 ] = TreeArgs{ d_tris, ts.keys0, ts.vals0, n, 1, ts.children, ts.rf, ts.rl, ts.bounds, ts.info };
+    if( view )
+    {
+        ta.s[ 1 ] = TreeArgs{ d_tris, bvh.keysA.as< uint64_t >(), bvh.valsA.as< uint32_t >(), n, bvh.leafMax, bvh.children.as< uint2 >(), rf, rl, bounds,
+                              bvh.expandInfo.as< uint4 >() };
+    }
+    uint2* const lists[ 2 ] = { ts.lists, view ? bvh.treeLists.as< uint2 >() : nullptr };
+    BuildTree( ta, lists, sets, stream );
 
-    // 5. Collapse to 8-wide nodes, level by level.
-    uint32_t* queue  = bvh.queue.as< uint32_t >();
-    uint32_t* counts = bvh.levelCounts.as< uint32_t >();  // nodes of each level
-    uint32_t* bases  = counts + BVH_MAX_LEVELS + 1;       // its first node in the queue
-    RG_HIP_CHECK( hipMemsetAsync( counts, 0, ( BVH_MAX_LEVELS + 1 ) * 2 * 4, stream ) );
-    RG_HIP_CHECK( hipMemsetAsync( bvh.isNode8.ptr, 0, size_t( slots ) * 4, stream ) );
+    // 5. Collapse to 8-wide nodes, level by level; the traversal's tree with
+    // one triangle per leaf.
+    constexpr uint32_t LW     = TreeScratch::LEVEL_WORDS;
+    uint32_t* const    levels = ts.levels;
+    CollapseSets       cs{};
+    cs.s[ 0 ] = CollapseArgs{ ts.queue, levels + BVH_MAX_LEVELS + 1, levels, n, 1, ts.info, ts.rf, ts.rl, ts.expansion, nullptr, ts.nodeBase,
+                              levels + LW * 2 };
+    RG_HIP_CHECK( hipMemsetAsync( levels, 0, ( LW * 2 + 1 ) * 4, stream ) );
+    if( view )
+    {
+        cs.s[ 1 ] = CollapseArgs{ bvh.queue.as< uint32_t >(), levels + LW + BVH_MAX_LEVELS + 1, levels + LW, n, bvh.leafMax, bvh.expandInfo.as< uint4 >(),
+                                  rf, rl, bvh.expansion.as< uint32_t >(), bvh.isNode8.as< uint32_t >(), nullptr, nullptr };
+        RG_HIP_CHECK( hipMemsetAsync( bvh.isNode8.ptr, 0, size_t( slots ) * 4, stream ) );
+    }
     if( !batched )
     {
-        k_seed_frontier<<< 1, 1, 0, stream >>>( queue, counts );
+        k_seed_frontier<<< 1, 64, 0, stream >>>( cs, sets );
         CheckLaunch( "k_seed_frontier" );
     }
     else
     {
-        RG_HIP_CHECK( hipMemsetAsync( bvh.sceneRoots.ptr, 0xFF, size_t( sceneCount ) * 4, stream ) );
-        k_scene_roots<<< DivUp( internal, THREADS ), THREADS, 0, stream >>>( internal, rf, rl, bvh.sceneOffsets.as< uint32_t >(), sceneCount,
-                                                                           bvh.sceneRoots.as< uint32_t >() );
-        CheckLaunch( "k_scene_roots" );
-        k_seed_frontier_seg<<< 1, 256, 0, stream >>>( bvh.sceneRoots.as< uint32_t >(), sceneCount, queue, counts );
-        CheckLaunch( "k_seed_frontier_seg" );
+        uint32_t* const roots[ 2 ] = { ts.roots, bvh.sceneRoots.as< uint32_t >() };
+        for( uint32_t k = 0; k < sets; k++ )
+        {
+            RG_HIP_CHECK( hipMemsetAsync( roots[ k ], 0xFF, size_t( sceneCount ) * 4, stream ) );
+            if( internal > 0 )
+            {
+                k_scene_roots<<< DivUp( internal, THREADS ), THREADS, 0, stream >>>( internal, ta.s[ k ].rangeFirst, ta.s[ k ].rangeLast, offs, sceneCount,
+                                                                                   roots[ k ] );
+                CheckLaunch( "k_scene_roots" );
+            }
+            k_seed_frontier_seg<<< 1, 256, 0, stream >>>( roots[ k ], sceneCount, offs, internal, k == 0, cs.s[ k ].queue, cs.s[ k ].levelCount,
+                                                          ta.s[ k ].bounds, k == 0 ? ts.boxes : nullptr );
+            CheckLaunch( "k_seed_frontier_seg" );
+        }
+        bvh.hostSegBoxes.resize( size_t( sceneCount ) * 8 );
+        RG_HIP_CHECK( hipMemcpyAsync( bvh.hostSegBoxes.data(), ts.boxes, size_t( sceneCount ) * 8 * sizeof( float ), hipMemcpyDeviceToHost, stream ) );
     }
 
-    const uint32_t maxFrontier  = n / ( bvh.leafMax + 1 ) + 1;
+    const uint32_t maxFrontier  = n / 2 + 1 + S;
     const uint32_t collapseGrid = DivUp( maxFrontier, THREADS ) < 4096 ? DivUp( maxFrontier, THREADS ) : 4096;
     // levels before the first look at how many nodes are left: an 8-wide
     // node stands for about 1.75 binary levels
@@ -1382,78 +1671,71 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
     {
         bits++;
     }
-    uint32_t level = 0, batch = bits * 4 / 7 + 2;
+    uint32_t        level = 0, batch = bits * 4 / 7 + 2;
+    uint32_t* const host  = bvh.hostLevels;
     do
     {
         for( uint32_t k = 0; k < batch; k++, level++ )
         {
             RG_REQUIRE( level + 1 < BVH_MAX_LEVELS, RG_RESULT_INTERNAL_ERROR, "BVH deeper than the level limit" );
-            k_collapse_level<<< collapseGrid, THREADS, 0, stream >>>( queue, bases + level, counts + level, n, bvh.leafMax,
-                                                                      bvh.expandInfo.as< uint4 >(), rf, rl, bvh.expansion.as< uint32_t >(),
-                                                                      bvh.isNode8.as< uint32_t >() );
+            k_collapse_level<<< dim3( collapseGrid, sets ), THREADS, 0, stream >>>( cs, level );
             CheckLaunch( "k_collapse_level" );
         }
-        RG_HIP_CHECK( hipMemcpyAsync( bvh.hostCounts, counts + level, 4, hipMemcpyDeviceToHost, stream ) );
-        RG_HIP_CHECK( hipMemcpyAsync( bvh.hostCounts + 1, bases + level, 4, hipMemcpyDeviceToHost, stream ) );
+        RG_HIP_CHECK( hipMemcpyAsync( host, levels, LW * 2 * 4, hipMemcpyDeviceToHost, stream ) );
         RG_HIP_CHECK( hipStreamSynchronize( stream ) );
         batch = 4;
-    } while( bvh.hostCounts[ 0 ] != 0 );
-    bvh.nodeCount = bvh.hostCounts[ 1 ];
-    // a batch of one-triangle frame segments has leaves for roots and no node
-    RG_REQUIRE( bvh.nodeCount >= 1 || segmentBoxes, RG_RESULT_INTERNAL_ERROR, "BVH collapse produced no nodes" );
-    ExclusiveScan( bvh.isNode8.as< uint32_t >(), slots, bvh.node8Index.as< uint32_t >(), nullptr, bvh.scanScratch.as< uint32_t >(), stream );
+    } while( host[ level ] != 0 || host[ LW + level ] != 0 );
+    const uint32_t countQ    = host[ BVH_MAX_LEVELS + 1 + level ];
+    const uint32_t countView = host[ LW + BVH_MAX_LEVELS + 1 + level ];
+    RG_REQUIRE( countQ >= 1 && ( !view || countView >= 1 ), RG_RESULT_INTERNAL_ERROR, "BVH collapse produced no nodes" );
 
-    const bool    half    = params.nodeFormat == RG_EXT_BVH_NODE_FP16;
-    DeviceBuffer& fp32Out = half ? bvh.nodes32 : bvh.nodes;
-    fp32Out.Reserve( size_t( bvh.nodeCount ) * sizeof( BvhNode8 ) );
-    if( bvh.nodeCount > 0 )
+    // 6. The nodes.
+    bvh.nodesQ.Reserve( size_t( countQ ) * sizeof( BvhNodeQ ) );
+    k_pack_nodes<<< DivUp( uint64_t( countQ ) * 8u, THREADS ), THREADS, 0, stream >>>( countQ, n, ts.expansion, ts.nodeBase, ts.bounds, ts.vals0, d_tris,
+                                                                                     bvh.nodesQ.as< BvhNodeQ >(), bvh.nodeTris.as< float4 >() );
+    CheckLaunch( "k_pack_nodes" );
+    if( view )
     {
-        k_write_nodes<<< DivUp( uint64_t( bvh.nodeCount ) * 8u, THREADS ), THREADS, 0, stream >>>(
-            bvh.nodeCount, n, queue, bvh.node8Index.as< uint32_t >(), bvh.expansion.as< uint32_t >(), rf, rl, bounds, fp32Out.as< BvhNode8 >() );
+        ExclusiveScan( bvh.isNode8.as< uint32_t >(), slots, bvh.node8Index.as< uint32_t >(), nullptr, bvh.scanScratch.as< uint32_t >(), stream );
+        const bool    half    = params.nodeFormat == RG_EXT_BVH_NODE_FP16;
+        DeviceBuffer& fp32Out = half ? bvh.nodes32 : bvh.nodes;
+        fp32Out.Reserve( size_t( countView ) * sizeof( BvhNode8 ) );
+        k_write_nodes<<< DivUp( uint64_t( countView ) * 8u, THREADS ), THREADS, 0, stream >>>(
+            countView, n, bvh.queue.as< uint32_t >(), bvh.node8Index.as< uint32_t >(), bvh.expansion.as< uint32_t >(), rf, rl, bounds, fp32Out.as< BvhNode8 >() );
         CheckLaunch( "k_write_nodes" );
-    }
-    k_sorted_tris<<< DivUp( n, THREADS ), THREADS, 0, stream >>>( d_tris, vin, n, bvh.sortedTris.as< float4 >() );
-    CheckLaunch( "k_sorted_tris" );
-    if( batched )
-    {
-        k_gather_roots8<<< 1, 256, 0, stream >>>( bvh.sceneRoots.as< uint32_t >(), bvh.sceneOffsets.as< uint32_t >(), sceneCount,
-                                                  bvh.node8Index.as< uint32_t >(), bvh.sceneRoots8.as< uint32_t >() );
-        CheckLaunch( "k_gather_roots8" );
-        bvh.hostSceneRoots.resize( sceneCount );
-        RG_HIP_CHECK( hipMemcpyAsync( bvh.hostSceneRoots.data(), bvh.sceneRoots8.ptr, size_t( sceneCount ) * 4, hipMemcpyDeviceToHost, stream ) );
-        if( segmentBoxes )
+        k_sorted_tris<<< DivUp( n, THREADS ), THREADS, 0, stream >>>( d_tris, bvh.sortedIdx, n, bvh.sortedTris.as< float4 >() );
+        CheckLaunch( "k_sorted_tris" );
+        if( batched )
         {
-            RG_REQUIRE( sceneCount <= 64, RG_RESULT_INTERNAL_ERROR, "too many frame segments" );
-            bvh.segBoxes.Reserve( size_t( sceneCount ) * 8 * sizeof( float ) );
-            k_segment_boxes<<< 1, 64, 0, stream >>>( fp32Out.as< BvhNode8 >(), bvh.sortedTris.as< float4 >(), bvh.sceneRoots8.as< uint32_t >(), sceneCount,
-                                                     bvh.segBoxes.as< float >() );
-            CheckLaunch( "k_segment_boxes" );
-            bvh.hostSegBoxes.resize( size_t( sceneCount ) * 8 );
-            RG_HIP_CHECK( hipMemcpyAsync( bvh.hostSegBoxes.data(), bvh.segBoxes.ptr, size_t( sceneCount ) * 8 * sizeof( float ), hipMemcpyDeviceToHost,
-                                          stream ) );
+            k_gather_roots8<<< 1, 256, 0, stream >>>( bvh.sceneRoots.as< uint32_t >(), sceneCount, bvh.node8Index.as< uint32_t >(),
+                                                      bvh.sceneRoots8.as< uint32_t >() );
+            CheckLaunch( "k_gather_roots8" );
+            bvh.hostSceneRoots.resize( sceneCount );
+            RG_HIP_CHECK( hipMemcpyAsync( bvh.hostSceneRoots.data(), bvh.sceneRoots8.ptr, size_t( sceneCount ) * 4, hipMemcpyDeviceToHost, stream ) );
         }
+        if( half )
+        {
+            bvh.nodes.Reserve( size_t( countView ) * sizeof( BvhNode8H ) );
+            k_half_nodes<<< DivUp( countView, THREADS ), THREADS, 0, stream >>>( bvh.nodes32.as< BvhNode8 >(), countView, bvh.nodes.as< BvhNode8H >() );
+            CheckLaunch( "k_half_nodes" );
+        }
+        RG_HIP_CHECK( hipMemcpyAsync( bvh.sceneMin, sceneBounds, 3 * sizeof( double ), hipMemcpyDeviceToHost, stream ) );
+        RG_HIP_CHECK( hipMemcpyAsync( bvh.sceneMax, sceneBounds + 3, 3 * sizeof( double ), hipMemcpyDeviceToHost, stream ) );
     }
-    if( half && bvh.nodeCount > 0 )
-    {
-        bvh.nodes.Reserve( size_t( bvh.nodeCount ) * sizeof( BvhNode8H ) );
-        k_half_nodes<<< DivUp( bvh.nodeCount, THREADS ), THREADS, 0, stream >>>( bvh.nodes32.as< BvhNode8 >(), bvh.nodeCount, bvh.nodes.as< BvhNode8H >() );
-        CheckLaunch( "k_half_nodes" );
-    }
-
-    RG_HIP_CHECK( hipMemcpyAsync( bvh.sceneMin, sceneBounds, 3 * sizeof( double ), hipMemcpyDeviceToHost, stream ) );
-    RG_HIP_CHECK( hipMemcpyAsync( bvh.sceneMax, sceneBounds + 3, 3 * sizeof( double ), hipMemcpyDeviceToHost, stream ) );
     RG_HIP_CHECK( hipStreamSynchronize( stream ) );
+    bvh.nodeCountQ = countQ;
+    bvh.nodeCount  = view ? countView : countQ;
 }
 } // namespace
 
 void BuildBvh( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtBvhBuildParams& params, hipStream_t stream )
 {
-    BuildBvhImpl( bvh, d_tris, n, params, nullptr, 0, stream );
+    BuildBvhImpl( bvh, d_tris, n, params, nullptr, 0, stream, true );
     bvh.frameSegs.clear();
 }
 
 void BuildBvhBatch( BvhObject& bvh, const float* d_tris, const uint32_t* offsets, uint32_t sceneCount, const RgExtBvhBuildParams& params,
-                    hipStream_t stream )
+                    hipStream_t stream, bool view )
 {
     RG_REQUIRE( offsets && sceneCount >= 1 && sceneCount <= 128, RG_RESULT_WRONG_FUNCTION_ARGUMENT, "1..128 scenes" );
     RG_REQUIRE( offsets[ 0 ] == 0, RG_RESULT_WRONG_FUNCTION_ARGUMENT, "scene offsets must start at 0" );
@@ -1461,9 +1743,9 @@ void BuildBvhBatch( BvhObject& bvh, const float* d_tris, const uint32_t* offsets
     {
         RG_REQUIRE( offsets[ s + 1 ] >= offsets[ s ] + 2, RG_RESULT_WRONG_FUNCTION_ARGUMENT, "every scene needs at least 2 triangles" );
     }
-    BuildBvhImpl( bvh, d_tris, offsets[ sceneCount ], params, offsets, sceneCount, stream );
+    BuildBvhImpl( bvh, d_tris, offsets[ sceneCount ], params, offsets, sceneCount, stream, view );
     bvh.frameSegs.clear();
-    for( uint32_t s = 0; s < sceneCount; s++ )
+    for( uint32_t s = 0; view && s < sceneCount; s++ )
     {
         RG_REQUIRE( bvh.hostSceneRoots[ s ] < bvh.nodeCount, RG_RESULT_INTERNAL_ERROR, "a scene has no root node" );
     }
@@ -1488,7 +1770,7 @@ void BuildFrameBvh( BvhObject& bvh, const float* d_tris, const uint32_t* classTr
     {
         // one class: the single-scene build (21 Morton bits per axis); rays
         // whose mask admits it start at its root
-        BuildBvhImpl( bvh, d_tris, n, params, nullptr, 0, stream );
+        BuildBvhImpl( bvh, d_tris, n, params, nullptr, 0, stream, false );
         bvh.frameSegs[ 0 ].cls  = cls[ 0 ];
         bvh.frameSegs[ 0 ].root = 0;
         for( int k = 0; k < 3; k++ )
@@ -1499,15 +1781,12 @@ void BuildFrameBvh( BvhObject& bvh, const float* d_tris, const uint32_t* classTr
         return;
     }
     // several classes: one batched build, each class a segment with its own
-    // root (a leaf for a one-triangle class) and root box
-    BuildBvhImpl( bvh, d_tris, n, params, offsets.data(), S, stream, true );
+    // root (node s of segment s) and root box
+    BuildBvhImpl( bvh, d_tris, n, params, offsets.data(), S, stream, false );
     for( uint32_t s = 0; s < S; s++ )
     {
-        const uint32_t r = bvh.hostSceneRoots[ s ];
-        RG_REQUIRE( ( r & RG_EXT_BVH_CHILD_LEAF_BIT ) ? ( ( r >> 3 ) & 0x0FFFFFFFu ) == offsets[ s ] : r < bvh.nodeCount, RG_RESULT_INTERNAL_ERROR,
-                    "a frame segment has no root" );
         bvh.frameSegs[ s ].cls  = cls[ s ];
-        bvh.frameSegs[ s ].root = r;
+        bvh.frameSegs[ s ].root = s;
         std::memcpy( bvh.frameSegs[ s ].box, &bvh.hostSegBoxes[ size_t( s ) * 8 ], 6 * sizeof( float ) );
     }
     bvh.sceneCount = 0; // traced as a frame (TraceRaysFrame), not as a batch of scenes

@@ -745,7 +745,7 @@ RgResult rgExtSceneBuild( RgExtScene scene )
         sc.vertices.Free();
         sc.indices.Free();
         const size_t n = scene->ds.triCount;
-        scene->bytes   = n * ( 9 + 9 + 1 + 9 ) * 4 + size_t( scene->bvh.nodeCount ) * scene->bvh.NodeStride() + n * 48;
+        scene->bytes   = n * ( 9 + 9 + 1 + 9 ) * 4 + size_t( scene->bvh.nodeCountQ ) * sizeof( BvhNodeQ ) + n * 48;
         scene->built   = true;
         std::lock_guard< std::mutex > lk( s.m );
         s.sceneBytes += scene->bytes;
@@ -822,7 +822,7 @@ RgResult rgExtSceneGroupCreate( RgExtServer server, const RgExtScene* pScenes, u
                                               size_t( grp->members[ k ]->ds.triCount ) * 9 * sizeof( float ), hipMemcpyDeviceToDevice, s.setup ) );
             }
             const RgExtBvhBuildParams bp = { 1, s.nodeFormat };
-            BuildBvhBatch( grp->bvh, tris.as< float >(), offsets.data(), sceneCount, bp, s.setup );
+            BuildBvhBatch( grp->bvh, tris.as< float >(), offsets.data(), sceneCount, bp, s.setup, false );
             RG_HIP_CHECK( hipStreamSynchronize( s.setup ) );
         }
         catch( ... )
@@ -834,7 +834,7 @@ RgResult rgExtSceneGroupCreate( RgExtServer server, const RgExtScene* pScenes, u
             }
             throw;
         }
-        grp->bytes = size_t( grp->bvh.nodeCount ) * grp->bvh.NodeStride() + size_t( offsets.back() ) * 48;
+        grp->bytes = size_t( grp->bvh.nodeCountQ ) * sizeof( BvhNodeQ ) + size_t( offsets.back() ) * 48;
         RgExtSceneGroup out = grp.get();
         std::lock_guard< std::mutex > lk( s.m );
         for( uint32_t k = 0; k < sceneCount; k++ )

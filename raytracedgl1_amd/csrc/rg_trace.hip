@@ -1,4 +1,4 @@
-// Software ray traversal of the 8-wide LBVH on gfx950.
+// Software ray traversal on gfx950.
 //
 // Stands in for traceRayEXT (Source/Shaders/RaygenCommon.h:217-269 closest
 // hit; :322-359 shadow rays with gl_RayFlagsSkipClosestHitShaderEXT).
@@ -9,17 +9,27 @@
 // empty.  Chunks of 64 rays come from 32 counters 256 bytes apart (block b
 // takes chunks j * 32 + b % 32), one atomic per chunk: a refill atomic per
 // wave iteration on a single address serialises at the memory side and made
-// the kernel 5.5x slower at 1080p.  The traversal stack is a short LDS
-// stack (24 entries per lane, interleaved by lane to avoid bank conflicts)
-// backed by a per-lane overflow area in global memory.
+// the kernel 5.5x slower at 1080p.
+//
+// k_trace walks the traversal's tree (BvhNodeQ): a node visit is five
+// 16-byte loads, eight byte-plane boxes by conversion and multiply-add, and a
+// sort of 32-bit keys whose low bits are the child's slot.  A node's hit
+// leaves are tested before its child nodes; the child nodes left over are one
+// group of two words on a stack that is short in LDS (12 groups by default,
+// interleaved by lane) and goes on in global memory.
 //
 // Closest hit is order-independent: a hit replaces the best one if its t is
 // smaller, or equal with a smaller primitive id, so the result equals a
 // brute-force loop over all triangles with the same intersection routine.
+//
+// k_trace_view walks the published 8-wide nodes near to far and counts its
+// node visits and triangle tests (RG_EXT_TRACE_COLLECT_STATS of
+// rgExtTraceRays): the algorithmic work on the tree that a program can read.
 #include "rg_bvh.h"
 #include "rg_trace_common.h"
 #include "rg_textures.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace rg
@@ -43,8 +53,8 @@ constexpr uint32_t COUNTER_STRIDE    = 64;  // u32 between counters (256 B)
 
 struct TraceArgs
 {
-    const void*     nodes; // BvhNode8 or BvhNode8H
-    const float4*   tris;
+    const void*     nodes; // k_trace: BvhNodeQ; k_trace_view: BvhNode8 or BvhNode8H
+    const float4*   tris;  // nodeTris or sortedTris
     const RgExtRay* rays;
     RgExtHit*       hits;
     uint32_t        count;
@@ -57,8 +67,9 @@ struct TraceArgs
     uint32_t*       errorFlag;
     uint64_t*       stats; // [0] node visits, [1] triangle tests (RG_EXT_TRACE_COLLECT_STATS)
     // rays of several scenes of a batched BVH (segCount > 0): rays of scene s
-    // are [segRays[s], segRays[s+1]), traversed from segRoots[s]; hits report
-    // primitive ids relative to segTris[s]
+    // are [segRays[s], segRays[s+1]), traversed from node s (k_trace) or
+    // segRoots[s] (k_trace_view); hits report primitive ids relative to
+    // segTris[s]
     const uint32_t* segRays;
     const uint32_t* segRoots;
     const uint32_t* segTris;
@@ -68,8 +79,8 @@ struct TraceArgs
     // the texture table
     const AlphaRec* alpha;
     TexView         tex;
-    // frame launches (rootCount > 0): a ray starts at the entry roots whose
-    // instance mask shares a bit with its cull mask (rayMasks[ray], or
+    // frame launches (rootCount > 0): a ray starts at the entry roots (nodes)
+    // whose instance mask shares a bit with its cull mask (rayMasks[ray], or
     // defaultMask); with several, their boxes are slab-tested first, like
     // the children of a node, without counting a node visit
     const uint8_t*  rayMasks;
@@ -182,10 +193,53 @@ __device__ __forceinline__ void LoadHalfNode( const void* nodes, uint32_t node, 
     }
 }
 
-template< bool H, int STACK_LDS, bool ALPHA >
+// Distances of a traversal node's planes are fma(q, scale / d, (origin - o) / d);
+// against the exact distance of the byte plane the rounding errors are at
+// most 4 u |t| (u = 2^-24) and 3e-5 grid steps.  The planes were moved out by
+// 1e-3 steps, and the relative part of both sides is covered by scaling the
+// far distances by 1 + 2e-6 and the best hit so far by 1 + 1e-6: every box
+// that the exact ray meets before the best hit is visited.
+constexpr float FAR_SLACK  = 1.000002f;
+constexpr float BEST_SLACK = 1e-6f;
+
+__device__ __forceinline__ void CmpSwap32( uint32_t& a, uint32_t& b )
+{
+    const uint32_t lo = a < b ? a : b;
+    const uint32_t hi = a < b ? b : a;
+    a                 = lo;
+    b                 = hi;
+}
+
+// Batcher odd-even merge sort network for 8 keys (19 compare-exchanges).
+__device__ __forceinline__ void Sort8( uint32_t k[ 8 ] )
+{
+#define CS( a, b ) CmpSwap32( k[ a ], k[ b ] )
+    CS( 0, 1 ); CS( 2, 3 ); CS( 4, 5 ); CS( 6, 7 );
+    CS( 0, 2 ); CS( 1, 3 ); CS( 4, 6 ); CS( 5, 7 );
+    CS( 1, 2 ); CS( 5, 6 );
+    CS( 0, 4 ); CS( 1, 5 ); CS( 2, 6 ); CS( 3, 7 );
+    CS( 2, 4 ); CS( 3, 5 );
+    CS( 1, 2 ); CS( 3, 4 ); CS( 5, 6 );
+#undef CS
+}
+
+__device__ __forceinline__ float ByteOf( uint32_t w, int k )
+{
+    return float( ( w >> ( 8 * k ) ) & 0xFFu );
+}
+
+// Bound by instruction issue and by the latency of the chain stack -> node.
+// Against the walk of the FP32 nodes (14 loads, 48 subtractions and
+// products, a sort of 64-bit keys that carry the references): 2.07M camera
+// rays over 1.0M triangles 770 -> 304 us, 0.75M bounce rays 614 -> 257,
+// 1.24M shadow rays 963 -> 509, of which the cubic keys of the tree give
+// about a third; 14,400 rays over 10,592 triangles 150 -> 68 us.
+// 5 waves per SIMD (94 registers) measured as 4 (108), 6 spill and lose 5%.
+template< int STACK_LDS, bool ALPHA >
 __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
 {
-    __shared__ uint32_t s_stack[ STACK_LDS * TR_THREADS ];
+    constexpr int    GROUPS = STACK_LDS / 2; // groups of child nodes in LDS
+    __shared__ uint2 s_stack[ GROUPS * TR_THREADS ];
     // The frame's entry roots, staged in LDS once per block: read from the
     // kernel arguments inside the loop they would hold 64 scalar registers,
     // which the compiler spills to vector-register lanes and reloads.
@@ -204,6 +258,352 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
         }
     }
     __syncthreads();
+    const int      lane      = tid & 63;
+    const uint64_t ltMask    = lane == 0 ? 0ull : ( ~0ull >> ( 64 - lane ) );
+    const uint32_t gthread   = blockIdx.x * TR_THREADS + tid;
+    uint2*         ovf       = reinterpret_cast< uint2* >( a.overflowStack + size_t( gthread ) * a.ovfStride );
+    const int      maxGroups = GROUPS + int( a.ovfStride / 2 );
+    const bool     anyHit    = ( a.flags & RG_EXT_TRACE_ANY_HIT ) != 0;
+    const bool     cullFront = ( a.flags & RG_EXT_TRACE_CULL_FRONT_FACE ) != 0;
+    const BvhNodeQ* nodes    = reinterpret_cast< const BvhNodeQ* >( a.nodes );
+
+    bool     active = false, exhausted = false;
+    uint32_t rayId  = 0;
+    RayPre   ray;
+    float    tmin = 0.0f, bestT = 0.0f, bestU = 0.0f, bestV = 0.0f, bestBox = 0.0f;
+    uint32_t bestPrim = RG_EXT_MISS;
+    // The current group: the next kids child nodes are base + the slots in
+    // list, three bits each; and the leaves of the last node visited that are
+    // still to be tested: triangles leafBase + the bits of leaves.
+    uint32_t base = 0, kids = 0, list = 0, leaves = 0, leafBase = 0;
+    uint32_t sgn      = 0; // bit a: the ray's direction is negative on axis a
+    uint32_t triBase  = 0; // first triangle of the ray's scene (batched BVHs)
+    int      sp       = 0;
+    uint32_t steps    = 0;
+    uint32_t nodeVisits = 0, triTests = 0;
+    const uint32_t part = blockIdx.x % a.partitions; // chunks j * partitions + part
+    uint32_t chunkNext = 0, chunkEnd = 0; // this wave's rays [chunkNext, chunkEnd), wave-uniform
+    bool     drained   = false;           // the global counter has passed the last ray
+
+    auto push = [ & ]( uint32_t b, uint32_t c, uint32_t l ) __attribute__( ( always_inline ) ) {
+        const uint2 e = make_uint2( b | c << 28, l );
+        if( sp < GROUPS )
+        {
+            s_stack[ sp * TR_THREADS + tid ] = e;
+        }
+        else if( sp < maxGroups )
+        {
+            ovf[ sp - GROUPS ] = e;
+        }
+        else
+        {
+            atomicOr( a.errorFlag, RG_EXT_TRACE_ERROR_STACK_OVERFLOW ); // dropped entry
+            return;
+        }
+        sp++;
+    };
+
+    while( true )
+    {
+        // Refill idle lanes.  Each wave owns a chunk of a.chunk consecutive
+        // rays taken with one atomic on its partition's counter; idle lanes
+        // take rays from the chunk (wave-uniform bookkeeping, no atomic).
+        const bool     need = !active && !exhausted;
+        const uint64_t mask = __ballot( need );
+        if( mask != 0ull && ( __popcll( mask ) >= REFILL_MIN_LANES || __ballot( active ) == 0ull ) )
+        {
+            const uint32_t cnt    = __popcll( mask );
+            const uint32_t rank   = __popcll( mask & ltMask );
+            const uint32_t left   = chunkEnd - chunkNext;
+            const int      leader = __ffsll( ( long long )mask ) - 1;
+            uint32_t       newBase = 0;
+            const bool     grab    = left < cnt && !drained;
+            if( grab )
+            {
+                uint32_t b = 0;
+                if( lane == leader )
+                {
+                    const uint32_t j = atomicAdd( a.rayCounter + part * COUNTER_STRIDE, 1u );
+                    const uint64_t g = uint64_t( j ) * a.partitions + part;
+                    b                = g * a.chunk < a.count ? uint32_t( g * a.chunk ) : a.count;
+                }
+                newBase = __shfl( b, leader, 64 );
+            }
+            if( need )
+            {
+                uint32_t my = a.count;
+                if( rank < left )
+                {
+                    my = chunkNext + rank;
+                }
+                else if( grab && newBase < a.count )
+                {
+                    my = newBase + ( rank - left );
+                }
+                if( my < a.count )
+                {
+                    const RgExtRay r = a.rays[ my ];
+                    rayId            = my;
+                    ray              = MakeRayPre( mk3( r.origin[ 0 ], r.origin[ 1 ], r.origin[ 2 ] ),
+                                                   mk3( r.direction[ 0 ], r.direction[ 1 ], r.direction[ 2 ] ) );
+                    sgn              = ( ray.invd.x < 0.0f ? 1u : 0u ) | ( ray.invd.y < 0.0f ? 2u : 0u ) | ( ray.invd.z < 0.0f ? 4u : 0u );
+                    tmin             = r.tmin;
+                    bestT            = r.tmax;
+                    bestU = bestV = 0.0f;
+                    bestPrim      = RG_EXT_MISS;
+                    bestBox       = r.tmax + fabsf( r.tmax ) * BEST_SLACK;
+                    base          = 0; // the root
+                    kids          = 1;
+                    list          = 0;
+                    leaves        = 0;
+                    triBase       = 0;
+                    if( a.segCount )
+                    {
+                        base    = SegmentOf( a.segRays, a.segCount, my );
+                        triBase = a.segTris[ base ];
+                    }
+                    sp            = 0;
+                    steps         = 0;
+                    active        = true;
+                    if( a.rootCount )
+                    {
+                        // frame launch: the entry roots the ray's cull mask admits
+                        const uint32_t rm      = a.rayMasks ? uint32_t( a.rayMasks[ my ] ) : a.defaultMask;
+                        uint32_t       admit   = 0;
+                        kids                   = 0;
+#pragma unroll
+                        for( int k = 0; k < 8; k++ )
+                        {
+                            if( uint32_t( k ) < a.rootCount && ( s_rootMask[ k ] & rm ) != 0u )
+                            {
+                                admit++;
+                                base = s_rootRef[ k ];
+                                kids = 1;
+                            }
+                        }
+                        if( admit > 1u )
+                        {
+                            // several segments: those whose box the ray
+                            // meets, in segment order (closest hit does
+                            // not depend on the order)
+                            kids = 0;
+#pragma unroll
+                            for( int k = 7; k >= 0; k-- )
+                            {
+                                float tn;
+                                if( uint32_t( k ) < a.rootCount && ( s_rootMask[ k ] & rm ) != 0u &&
+                                    SlabTest( ray, s_rootBox[ k ][ 0 ], s_rootBox[ k ][ 1 ], s_rootBox[ k ][ 2 ], s_rootBox[ k ][ 3 ],
+                                              s_rootBox[ k ][ 4 ], s_rootBox[ k ][ 5 ], tmin, bestT, &tn ) )
+                                {
+                                    if( kids )
+                                    {
+                                        push( base, 1u, 0u );
+                                    }
+                                    base = s_rootRef[ k ];
+                                    kids = 1;
+                                }
+                            }
+                        }
+                        if( kids == 0u )
+                        {
+                            // no segment to visit: a miss
+                            RgExtHit h;
+                            h.t         = bestT;
+                            h.u         = 0.0f;
+                            h.v         = 0.0f;
+                            h.primitiveId = RG_EXT_MISS;
+                            a.hits[ my ] = h;
+                            active       = false;
+                        }
+                    }
+                }
+                else
+                {
+                    exhausted = true;
+                }
+            }
+            if( !grab )
+            {
+                chunkNext += cnt < left ? cnt : left;
+            }
+            else if( newBase < a.count )
+            {
+                chunkEnd  = a.count - newBase > a.chunk ? newBase + a.chunk : a.count;
+                chunkNext = newBase + ( cnt - left ) < chunkEnd ? newBase + ( cnt - left ) : chunkEnd;
+            }
+            else
+            {
+                drained   = true;
+                chunkNext = chunkEnd;
+            }
+        }
+        if( __ballot( active ) == 0ull )
+        {
+            if( __ballot( !exhausted ) != 0ull )
+            {
+                continue; // rays that ended at the frame roots: take the next ones
+            }
+            if( a.stats )
+            {
+                uint64_t nv = nodeVisits, tt = triTests;
+                for( int off = 32; off > 0; off >>= 1 )
+                {
+                    nv += __shfl_xor( nv, off, 64 );
+                    tt += __shfl_xor( tt, off, 64 );
+                }
+                if( lane == 0 )
+                {
+                    atomicAdd( reinterpret_cast< unsigned long long* >( &a.stats[ 0 ] ), ( unsigned long long )nv );
+                    atomicAdd( reinterpret_cast< unsigned long long* >( &a.stats[ 1 ] ), ( unsigned long long )tt );
+                }
+            }
+            break;
+        }
+        if( !active )
+        {
+            continue;
+        }
+
+        bool finished = false;
+        if( ++steps > MAX_STEPS_PER_RAY )
+        {
+            // Only a malformed tree can get here; end the ray instead of spinning.
+            atomicOr( a.errorFlag, RG_EXT_TRACE_ERROR_STEP_LIMIT );
+            finished = true;
+        }
+        else
+        {
+            if( leaves == 0u )
+            {
+                nodeVisits++;
+                const uint4*   np = reinterpret_cast< const uint4* >( nodes + ( base + ( list & 7u ) ) );
+                const uint4    r0 = np[ 0 ], r1 = np[ 1 ], r2 = np[ 2 ], r3 = np[ 3 ];
+                const uint2    r4 = *reinterpret_cast< const uint2* >( np + 4 );
+                list >>= 3;
+                kids--;
+                // per axis: scale / d and (origin - o) / d, and the byte planes
+                // that the ray enters and leaves through
+                const float sx = __uint_as_float( ( r0.w & 0xFFu ) << 23 ) * ray.invd.x, bx = ( __uint_as_float( r0.x ) - ray.o.x ) * ray.invd.x;
+                const float sy = __uint_as_float( ( r0.w & 0xFF00u ) << 15 ) * ray.invd.y, by = ( __uint_as_float( r0.y ) - ray.o.y ) * ray.invd.y;
+                const float sz = __uint_as_float( ( r0.w & 0xFF0000u ) << 7 ) * ray.invd.z, bz = ( __uint_as_float( r0.z ) - ray.o.z ) * ray.invd.z;
+                const float fsx = sx * FAR_SLACK, fbx = bx * FAR_SLACK, fsy = sy * FAR_SLACK, fby = by * FAR_SLACK, fsz = sz * FAR_SLACK, fbz = bz * FAR_SLACK;
+                const bool     nx = ( sgn & 1u ) != 0u, ny = ( sgn & 2u ) != 0u, nz = ( sgn & 4u ) != 0u;
+                const uint32_t qnx[ 2 ] = { nx ? r2.z : r1.x, nx ? r2.w : r1.y }, qfx[ 2 ] = { nx ? r1.x : r2.z, nx ? r1.y : r2.w };
+                const uint32_t qny[ 2 ] = { ny ? r3.x : r1.z, ny ? r3.y : r1.w }, qfy[ 2 ] = { ny ? r1.z : r3.x, ny ? r1.w : r3.y };
+                const uint32_t qnz[ 2 ] = { nz ? r3.z : r2.x, nz ? r3.w : r2.y }, qfz[ 2 ] = { nz ? r2.x : r3.z, nz ? r2.y : r3.w };
+                const uint32_t inner = ( r0.w >> 24 ) & 15u, leaf = r0.w >> 28;
+                uint32_t       key[ 8 ], hits = 0u;
+#pragma unroll
+                for( int k = 0; k < 8; k++ )
+                {
+                    const int   w = k >> 2, j = k & 3;
+                    const float tx0 = __builtin_fmaf( ByteOf( qnx[ w ], j ), sx, bx ), tx1 = __builtin_fmaf( ByteOf( qfx[ w ], j ), fsx, fbx );
+                    const float ty0 = __builtin_fmaf( ByteOf( qny[ w ], j ), sy, by ), ty1 = __builtin_fmaf( ByteOf( qfy[ w ], j ), fsy, fby );
+                    const float tz0 = __builtin_fmaf( ByteOf( qnz[ w ], j ), sz, bz ), tz1 = __builtin_fmaf( ByteOf( qfz[ w ], j ), fsz, fbz );
+                    const float tn  = fmaxf( fmaxf( fmaxf( tx0, ty0 ), tz0 ), tmin );
+                    const float tf  = fminf( fminf( fminf( tx1, ty1 ), tz1 ), bestBox );
+                    const bool  h   = tn <= tf;
+                    hits |= h ? 1u << k : 0u;
+                    key[ k ] = h && uint32_t( k ) < inner ? ( __float_as_uint( tn ) & ~7u ) | uint32_t( k ) : ~0u;
+                }
+                const uint32_t innerMask = ( 1u << inner ) - 1u;
+                leaves                   = hits & ( ( ( 1u << leaf ) - 1u ) << inner );
+                leafBase                 = r4.y;
+                const uint32_t found     = __popc( hits & innerMask );
+                if( found )
+                {
+                    if( kids )
+                    {
+                        push( base, kids, list );
+                    }
+                    Sort8( key );
+                    base = r4.x;
+                    kids = found;
+                    list = 0u;
+#pragma unroll
+                    for( int k = 7; k >= 0; k-- )
+                    {
+                        list = list << 3 | ( key[ k ] & 7u );
+                    }
+                }
+            }
+            if( leaves )
+            {
+                triTests++;
+                const uint32_t slot = __ffs( leaves ) - 1;
+                leaves &= leaves - 1u;
+                const float4* tp = a.tris + size_t( leafBase + slot ) * 3;
+                const float4  q0 = tp[ 0 ], q1 = tp[ 1 ], q2 = tp[ 2 ];
+                float         t, u, v;
+                if( IntersectTri( ray, mk3( q0.x, q0.y, q0.z ), mk3( q1.x, q1.y, q1.z ), mk3( q2.x, q2.y, q2.z ), tmin, bestT, cullFront, &t, &u, &v ) )
+                {
+                    const uint32_t prim = __float_as_uint( q0.w );
+                    bool           take = t < bestT || prim < bestPrim;
+                    if constexpr( ALPHA )
+                    {
+                        const AlphaRec& ar = a.alpha[ prim ];
+                        if( take && TexValid( a.tex, ar.tex ) && !AlphaPasses( a.tex, ar, u, v ) )
+                        {
+                            take = false; // ignoreIntersectionEXT
+                        }
+                    }
+                    if( take )
+                    {
+                        bestT    = t;
+                        bestBox  = t + fabsf( t ) * BEST_SLACK;
+                        bestU    = u;
+                        bestV    = v;
+                        bestPrim = prim;
+                        finished = anyHit;
+                    }
+                }
+            }
+            if( !finished && leaves == 0u && kids == 0u )
+            {
+                if( sp == 0 )
+                {
+                    finished = true;
+                }
+                else
+                {
+                    sp--;
+                    uint2 e;
+                    if( sp < GROUPS )
+                    {
+                        e = s_stack[ sp * TR_THREADS + tid ];
+                    }
+                    else
+                    {
+                        // Keeps the rare overflow read a separate global load
+                        // (no generic-address load on the common LDS path).
+                        asm volatile( "" ::: "memory" );
+                        e = ovf[ sp - GROUPS ];
+                    }
+                    base = e.x & 0x0FFFFFFFu;
+                    kids = e.x >> 28;
+                    list = e.y;
+                }
+            }
+        }
+        if( finished )
+        {
+            RgExtHit h;
+            h.t                = bestT;
+            h.u                = bestU;
+            h.v                = bestV;
+            h.primitiveId      = bestPrim == RG_EXT_MISS ? RG_EXT_MISS : bestPrim - triBase;
+            a.hits[ rayId ]    = h;
+            active             = false;
+        }
+    }
+}
+
+template< bool H >
+__global__ __launch_bounds__( TR_THREADS ) void k_trace_view( TraceArgs a )
+{
+    constexpr int       STACK_LDS = 24;
+    __shared__ uint32_t s_stack[ STACK_LDS * TR_THREADS ];
+    const int      tid       = threadIdx.x;
     const int      lane      = tid & 63;
     const uint64_t ltMask    = lane == 0 ? 0ull : ( ~0ull >> ( 64 - lane ) );
     const uint32_t gthread   = blockIdx.x * TR_THREADS + tid;
@@ -303,55 +703,6 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
                     sp            = 0;
                     steps         = 0;
                     active        = true;
-                    if( a.rootCount )
-                    {
-                        // frame launch: the entry roots the ray's cull mask admits
-                        const uint32_t rm      = a.rayMasks ? uint32_t( a.rayMasks[ my ] ) : a.defaultMask;
-                        uint32_t       admit   = 0, only = RG_EXT_BVH_CHILD_EMPTY;
-#pragma unroll
-                        for( int k = 0; k < 8; k++ )
-                        {
-                            if( uint32_t( k ) < a.rootCount && ( s_rootMask[ k ] & rm ) != 0u )
-                            {
-                                admit++;
-                                only = s_rootRef[ k ];
-                            }
-                        }
-                        node = only;
-                        if( admit > 1u )
-                        {
-                            // several segments: those whose box the ray
-                            // meets, in segment order (closest hit does
-                            // not depend on the order)
-                            node = RG_EXT_BVH_CHILD_EMPTY;
-#pragma unroll
-                            for( int k = 7; k >= 0; k-- )
-                            {
-                                float tn;
-                                if( uint32_t( k ) < a.rootCount && ( s_rootMask[ k ] & rm ) != 0u &&
-                                    SlabTest( ray, s_rootBox[ k ][ 0 ], s_rootBox[ k ][ 1 ], s_rootBox[ k ][ 2 ], s_rootBox[ k ][ 3 ],
-                                              s_rootBox[ k ][ 4 ], s_rootBox[ k ][ 5 ], tmin, bestT, &tn ) )
-                                {
-                                    if( node != RG_EXT_BVH_CHILD_EMPTY )
-                                    {
-                                        push( node );
-                                    }
-                                    node = s_rootRef[ k ];
-                                }
-                            }
-                        }
-                        if( node == RG_EXT_BVH_CHILD_EMPTY )
-                        {
-                            // no segment to visit: a miss
-                            RgExtHit h;
-                            h.t         = bestT;
-                            h.u         = 0.0f;
-                            h.v         = 0.0f;
-                            h.primitiveId = RG_EXT_MISS;
-                            a.hits[ my ] = h;
-                            active       = false;
-                        }
-                    }
                 }
                 else
                 {
@@ -375,10 +726,6 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
         }
         if( __ballot( active ) == 0ull )
         {
-            if( __ballot( !exhausted ) != 0ull )
-            {
-                continue; // rays that ended at the frame roots: take the next ones
-            }
             if( a.stats )
             {
                 uint64_t nv = nodeVisits, tt = triTests;
@@ -559,14 +906,6 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
                 if( IntersectTri( ray, mk3( q0.x, q0.y, q0.z ), mk3( q1.x, q1.y, q1.z ), mk3( q2.x, q2.y, q2.z ), tmin, bestT, cullFront, &t, &u, &v ) )
                 {
                     const uint32_t prim = __float_as_uint( q0.w );
-                    if constexpr( ALPHA )
-                    {
-                        const AlphaRec& ar = a.alpha[ prim ];
-                        if( TexValid( a.tex, ar.tex ) && !AlphaPasses( a.tex, ar, u, v ) )
-                        {
-                            continue; // ignoreIntersectionEXT
-                        }
-                    }
                     if( t < bestT || prim < bestPrim )
                     {
                         bestT    = t;
@@ -652,21 +991,25 @@ constexpr int TRACE_STACK_DEPTH[ TRACE_STACK_VARIANTS ] = { 16, 24, 32 };
 
 using TraceKernelFn = void ( * )( TraceArgs );
 
-TraceKernelFn TraceKernel( int half, int v, bool alpha = false )
+TraceKernelFn TraceKernel( int v, bool alpha )
 {
-    if( alpha )
-    {
-        static const TraceKernelFn ka[ 2 ][ TRACE_STACK_VARIANTS ] = {
-            { k_trace< false, 16, true >, k_trace< false, 24, true >, k_trace< false, 32, true > },
-            { k_trace< true, 16, true >, k_trace< true, 24, true >, k_trace< true, 32, true > },
-        };
-        return ka[ half ][ v ];
-    }
     static const TraceKernelFn k[ 2 ][ TRACE_STACK_VARIANTS ] = {
-        { k_trace< false, 16, false >, k_trace< false, 24, false >, k_trace< false, 32, false > },
-        { k_trace< true, 16, false >, k_trace< true, 24, false >, k_trace< true, 32, false > },
+        { k_trace< 16, false >, k_trace< 24, false >, k_trace< 32, false > },
+        { k_trace< 16, true >, k_trace< 24, true >, k_trace< 32, true > },
     };
-    return k[ half ][ v ];
+    return k[ alpha ? 1 : 0 ][ v ];
+}
+
+TraceKernelFn ViewKernel( uint32_t nodeFormat )
+{
+    return nodeFormat == RG_EXT_BVH_NODE_FP16 ? k_trace_view< true > : k_trace_view< false >;
+}
+
+uint32_t ResidentBlocks( TraceKernelFn k, int cus )
+{
+    int perCu = 0;
+    RG_HIP_CHECK( hipOccupancyMaxActiveBlocksPerMultiprocessor( &perCu, k, TR_THREADS, 0 ) );
+    return uint32_t( cus * ( perCu > 0 ? perCu : 1 ) );
 }
 
 // Resident blocks of every variant; the overflow stacks are sized for the
@@ -681,15 +1024,13 @@ void InitGrids( TraceContext& s )
     RG_HIP_CHECK( hipGetDevice( &dev ) );
     RG_HIP_CHECK( hipDeviceGetAttribute( &cus, hipDeviceAttributeMultiprocessorCount, dev ) );
     uint32_t maxGrid = 0;
-    for( int h = 0; h < 2; h++ )
+    for( int v = 0; v <= TRACE_STACK_VARIANTS; v++ )
     {
-        for( int v = 0; v < TRACE_STACK_VARIANTS; v++ )
-        {
-            int perCu = 0;
-            RG_HIP_CHECK( hipOccupancyMaxActiveBlocksPerMultiprocessor( &perCu, TraceKernel( h, v ), TR_THREADS, 0 ) );
-            s.grid[ h ][ v ] = uint32_t( cus * ( perCu > 0 ? perCu : 1 ) );
-            maxGrid          = s.grid[ h ][ v ] > maxGrid ? s.grid[ h ][ v ] : maxGrid;
-        }
+        // the plain kernels' grids, which their alpha-testing forms (more
+        // registers) share; last, the counting walk of the published nodes
+        s.grid[ v ] = v < TRACE_STACK_VARIANTS ? ResidentBlocks( TraceKernel( v, false ), cus )
+                                               : std::min( ResidentBlocks( ViewKernel( RG_EXT_BVH_NODE_FP32 ), cus ), ResidentBlocks( ViewKernel( RG_EXT_BVH_NODE_FP16 ), cus ) );
+        maxGrid     = s.grid[ v ] > maxGrid ? s.grid[ v ] : maxGrid;
     }
     s.overflow.Reserve( size_t( maxGrid ) * TR_THREADS * STACK_OVF_STRIDE * sizeof( uint32_t ) );
     s.gridBlocks = maxGrid;
@@ -710,9 +1051,7 @@ void TraceRaysImpl( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
                     hipStream_t stream, hipEvent_t evBefore, hipEvent_t evAfter, const TraceAccum* accum, const uint32_t* d_segRays,
                     const FrameRoots* frame = nullptr, const AlphaRec* alpha = nullptr, const TexView* tex = nullptr )
 {
-    RG_REQUIRE( bvh.nodeCount > 0 || ( frame && frame->rootCount > 0 ), RG_RESULT_WRONG_FUNCTION_CALL, "BVH is not built" );
-    RG_REQUIRE( bvh.nodeFormat == RG_EXT_BVH_NODE_FP32 || bvh.nodeFormat == RG_EXT_BVH_NODE_FP16, RG_RESULT_WRONG_FUNCTION_ARGUMENT,
-                "unsupported node format" );
+    RG_REQUIRE( bvh.nodeCountQ > 0, RG_RESULT_WRONG_FUNCTION_CALL, "BVH is not built" );
     // the chunk counter runs up to count + (waves + 1) * chunk without wrapping
     RG_REQUIRE( count <= 0xF0000000u, RG_RESULT_WRONG_FUNCTION_ARGUMENT, "too many rays in one launch" );
     if( count == 0 )
@@ -720,17 +1059,18 @@ void TraceRaysImpl( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
         return;
     }
     InitGrids( s );
-    const int      h      = bvh.nodeFormat == RG_EXT_BVH_NODE_FP16 ? 1 : 0;
+    // statistics of a program's own BVH are those of its published nodes
+    const bool     view   = !frame && !accum && ( flags & RG_EXT_TRACE_COLLECT_STATS ) != 0;
     const int      v      = int( s.stackVariant < TRACE_STACK_VARIANTS ? s.stackVariant : 1u );
-    const uint32_t grid   = s.grid[ h ][ v ];
+    const uint32_t grid   = s.grid[ view ? TRACE_STACK_VARIANTS : v ];
     const uint32_t blocks = DivUp( count, TR_THREADS ) < grid ? DivUp( count, TR_THREADS ) : grid;
     s.counter.Reserve( ( RAY_PARTITIONS * COUNTER_STRIDE + 1 ) * sizeof( uint32_t ) );
     s.stats.Reserve( 2 * sizeof( uint64_t ) );
     RG_HIP_CHECK( hipMemsetAsync( s.counter.ptr, 0, ( RAY_PARTITIONS * COUNTER_STRIDE + 1 ) * sizeof( uint32_t ), stream ) );
 
     TraceArgs a;
-    a.nodes         = bvh.nodes.ptr;
-    a.tris          = reinterpret_cast< const float4* >( bvh.sortedTris.ptr );
+    a.nodes         = view ? bvh.nodes.ptr : bvh.nodesQ.ptr;
+    a.tris          = reinterpret_cast< const float4* >( view ? bvh.sortedTris.ptr : bvh.nodeTris.ptr );
     a.rays          = d_rays;
     a.hits          = d_hits;
     a.count         = count;
@@ -752,7 +1092,7 @@ void TraceRaysImpl( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
     for( int k = 0; k < 8; k++ )
     {
         a.rootMask[ k ] = 0;
-        a.rootRef[ k ]  = RG_EXT_BVH_CHILD_EMPTY;
+        a.rootRef[ k ]  = 0;
         for( int j = 0; j < 6; j++ )
         {
             a.rootBox[ k ][ j ] = 0.0f;
@@ -791,7 +1131,7 @@ void TraceRaysImpl( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
     {
         RG_HIP_CHECK( hipEventRecord( evBefore, stream ) );
     }
-    hipLaunchKernelGGL( TraceKernel( h, v, a.alpha != nullptr ), dim3( blocks ), dim3( TR_THREADS ), 0, stream, a );
+    hipLaunchKernelGGL( view ? ViewKernel( bvh.nodeFormat ) : TraceKernel( v, a.alpha != nullptr ), dim3( blocks ), dim3( TR_THREADS ), 0, stream, a );
     CheckLaunch( "k_trace" );
     if( evAfter )
     {
@@ -846,7 +1186,7 @@ __global__ __launch_bounds__( 64 ) void k_noalloc_clear( uint32_t* hdr )
 struct NoAllocDevice
 {
     uint32_t* scratch = nullptr; // the device address of `scratch` on this GPU
-    uint32_t  grid[ 2 ] = {};    // persistent blocks per node format (FP32, FP16)
+    uint32_t  grid[ 2 ] = {};    // persistent blocks of k_trace and of the counting walk
 };
 constexpr int MAX_DEVICES = 64;
 std::mutex    g_noAllocMutex;
@@ -870,13 +1210,9 @@ const NoAllocDevice& NoAllocFor( int dev )
         RG_HIP_CHECK( hipGetSymbolAddress( &ptr, HIP_SYMBOL( scratch ) ) );
         int cus = 0;
         RG_HIP_CHECK( hipDeviceGetAttribute( &cus, hipDeviceAttributeMultiprocessorCount, dev ) );
-        for( int h = 0; h < 2; h++ )
-        {
-            int perCu = 0;
-            RG_HIP_CHECK( hipOccupancyMaxActiveBlocksPerMultiprocessor( &perCu, TraceKernel( h, NOALLOC_VARIANT ), TR_THREADS, 0 ) );
-            const uint32_t g = uint32_t( cus * ( perCu > 0 ? perCu : 1 ) );
-            d.grid[ h ]      = g < NOALLOC_MAX_BLOCKS ? g : NOALLOC_MAX_BLOCKS;
-        }
+        d.grid[ 0 ] = std::min( ResidentBlocks( TraceKernel( NOALLOC_VARIANT, false ), cus ), NOALLOC_MAX_BLOCKS );
+        d.grid[ 1 ] = std::min( std::min( ResidentBlocks( ViewKernel( RG_EXT_BVH_NODE_FP32 ), cus ), ResidentBlocks( ViewKernel( RG_EXT_BVH_NODE_FP16 ), cus ) ),
+                                NOALLOC_MAX_BLOCKS );
         d.scratch = static_cast< uint32_t* >( ptr );
     }
     return d;
@@ -886,9 +1222,7 @@ const NoAllocDevice& NoAllocFor( int dev )
 void TraceRaysNoAlloc( const BvhObject& bvh, const RgExtRay* d_rays, uint32_t count, RgExtHit* d_hits, uint32_t flags, hipStream_t stream )
 {
     RG_REQUIRE( bvh.sceneCount == 0, RG_RESULT_WRONG_FUNCTION_ARGUMENT, "a batched BVH is traced with TraceRaysBatch" );
-    RG_REQUIRE( bvh.nodeCount > 0, RG_RESULT_WRONG_FUNCTION_CALL, "BVH is not built" );
-    RG_REQUIRE( bvh.nodeFormat == RG_EXT_BVH_NODE_FP32 || bvh.nodeFormat == RG_EXT_BVH_NODE_FP16, RG_RESULT_WRONG_FUNCTION_ARGUMENT,
-                "unsupported node format" );
+    RG_REQUIRE( bvh.nodeCountQ > 0, RG_RESULT_WRONG_FUNCTION_CALL, "BVH is not built" );
     RG_REQUIRE( count <= RG_EXT_TRACE_NOALLOC_MAX_RAYS, RG_RESULT_WRONG_FUNCTION_ARGUMENT,
                 "too many rays for one call (at most RG_EXT_TRACE_NOALLOC_MAX_RAYS)" );
     int dev = 0;
@@ -898,16 +1232,16 @@ void TraceRaysNoAlloc( const BvhObject& bvh, const RgExtRay* d_rays, uint32_t co
     {
         return;
     }
-    const int      h      = bvh.nodeFormat == RG_EXT_BVH_NODE_FP16 ? 1 : 0;
-    const uint32_t blocks = DivUp( count, TR_THREADS ) < nd.grid[ h ] ? DivUp( count, TR_THREADS ) : nd.grid[ h ];
+    const bool     view   = ( flags & RG_EXT_TRACE_COLLECT_STATS ) != 0;
+    const uint32_t blocks = std::min( DivUp( count, TR_THREADS ), nd.grid[ view ? 1 : 0 ] );
     RG_REQUIRE( size_t( blocks ) * TR_THREADS * NOALLOC_OVF <= NOALLOC_WORDS - NOALLOC_HEADER, RG_RESULT_INTERNAL_ERROR,
                 "no-alloc traversal grid exceeds its scratch" );
     k_noalloc_clear<<< 1, 64, 0, stream >>>( nd.scratch );
     CheckLaunch( "k_noalloc_clear" );
 
     TraceArgs a{};
-    a.nodes         = bvh.nodes.ptr;
-    a.tris          = reinterpret_cast< const float4* >( bvh.sortedTris.ptr );
+    a.nodes         = view ? bvh.nodes.ptr : bvh.nodesQ.ptr;
+    a.tris          = reinterpret_cast< const float4* >( view ? bvh.sortedTris.ptr : bvh.nodeTris.ptr );
     a.rays          = d_rays;
     a.hits          = d_hits;
     a.count         = count;
@@ -923,12 +1257,12 @@ void TraceRaysNoAlloc( const BvhObject& bvh, const RgExtRay* d_rays, uint32_t co
     a.rootCount     = 0;
     for( int k = 0; k < 8; k++ )
     {
-        a.rootRef[ k ] = RG_EXT_BVH_CHILD_EMPTY;
+        a.rootRef[ k ] = 0;
     }
     a.chunk = RAY_CHUNK_DEFAULT;
     a.alpha = nullptr;
     a.tex   = TexView{};
-    hipLaunchKernelGGL( TraceKernel( h, NOALLOC_VARIANT, false ), dim3( blocks ), dim3( TR_THREADS ), 0, stream, a );
+    hipLaunchKernelGGL( view ? ViewKernel( bvh.nodeFormat ) : TraceKernel( NOALLOC_VARIANT, false ), dim3( blocks ), dim3( TR_THREADS ), 0, stream, a );
     CheckLaunch( "k_trace" );
 }
 

@@ -206,6 +206,66 @@ def test_trace_terrain_spheres_1080p(gpu, oracle):
     assert np.abs(pb - pr).max() < 1e-2
 
 
+def _edge_scene(kind, r):
+    """Triangles at the limits of the traversal nodes' byte grids, and their spread."""
+    if kind.startswith("n"):  # leaves per node, and nodes of one child
+        return _random_tris(int(kind[1:]), seed=int(kind[1:])), 10.0
+    t = _random_tris(3000, seed=7)
+    if kind == "flat":  # no extent on one axis
+        t[:, 1::3] = 2.5
+    elif kind == "thin":  # extents of 1e-30 and 0 beside 10
+        t[:, 1::3] = np.where(r.random((3000, 3)) < 0.5, 0.0, 1e-30)
+    elif kind == "far":  # 20,000 units out: a grid step is a few units in the last place
+        t += np.float32(20000.0)
+    elif kind == "huge":
+        t *= np.float32(1e10)
+    elif kind == "broken":  # triangles that nothing hits, in every part of the tree
+        bad = r.random(3000) < 0.03
+        t[bad, 4] = np.where(r.random(bad.sum()) < 0.5, np.inf, np.nan)
+        t[::701] = np.nan
+    return t, 10.0
+
+
+@pytest.mark.parametrize("kind", ["n1", "n2", "n7", "n8", "n9", "n15", "n57", "n500", "flat", "thin", "far", "huge", "broken"])
+def test_traversal_nodes_at_their_limits(gpu, kind):
+    """Hits through the traversal's byte-grid nodes against the walk of the
+    published FP32 nodes: the same, or a hit that the FP32 boxes' rounding
+    hid, nearer by rounding (1e-5 t bounds the triangle test's error) or as
+    near with a lower id.  At most 1e-4 of the rays differ, but where all
+    triangles lie in one plane and overlap: there every ray meets several
+    within rounding of each other, and a ray in that plane meets them edge
+    on, where the triangle test is all rounding and no bound on t holds."""
+    print(f"traversal nodes {kind}", flush=True)
+    r = np.random.default_rng(11)
+    tris, spread = _edge_scene(kind, r)
+    finite = tris[np.isfinite(tris).all(1)].reshape(-1, 3, 3)
+    n = 60000
+    rays = np.zeros(n, RAY_DTYPE)
+    target = finite[r.integers(0, len(finite), n)].mean(1).astype(np.float64)
+    scale = max(1.0, np.abs(finite).max() if kind == "huge" else spread)
+    origin = target + r.normal(size=(n, 3)) * scale
+    if kind in ("flat", "thin"):
+        origin[: n // 4, 1] = finite[0, 0, 1]  # in the plane of the triangles
+    d = target - origin + r.normal(size=(n, 3)) * scale * 0.02
+    d[: n // 8, r.integers(0, 3)] = 0.0  # parallel to a slab
+    d[n // 8: n // 6, :2] = 0.0
+    rays["origin"] = origin
+    rays["direction"] = d / np.maximum(np.linalg.norm(d, axis=1, keepdims=True), 1e-30)
+    rays["tmin"] = np.where(r.random(n) < 0.5, 0.0, 0.1 * scale)
+    rays["tmax"] = np.where(r.random(n) < 0.2, np.inf, 100.0 * scale)
+    b, _ = _gpu_bvh(tris, 1)
+    g = _trace_gpu(b, rays, 0)
+    v = _trace_gpu(b, rays, RG_EXT_TRACE_COLLECT_STATS)
+    assert (v["prim"] != RG_EXT_MISS).mean() > 0.02
+    diff = (g["prim"] != v["prim"]) | (g["t"] != v["t"]) | (g["u"] != v["u"]) | (g["v"] != v["v"])
+    assert kind in ("flat", "thin") or diff.mean() <= 1e-4, diff.sum()
+    near = diff & ((np.arange(n) >= n // 4) if kind in ("flat", "thin") else True)
+    assert (v["t"][near] - g["t"][near] <= 1e-5 * g["t"][near]).all()
+    assert ((g["t"] < v["t"]) | ((g["t"] == v["t"]) & (g["prim"] < v["prim"])))[diff].all()
+    occ = _trace_gpu(b, rays, RG_EXT_TRACE_ANY_HIT)["prim"] != RG_EXT_MISS
+    assert np.array_equal(occ, g["prim"] != RG_EXT_MISS)
+
+
 def test_histogram_bit_exact(gpu, oracle):
     r = np.random.default_rng(11)
     w, h = 1920, 1080
