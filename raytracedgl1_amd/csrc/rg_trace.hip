@@ -11,8 +11,8 @@
 // wave iteration on a single address serialises at the memory side and made
 // the kernel 5.5x slower at 1080p.
 //
-// k_trace walks the traversal's tree (BvhNodeQ): a node visit is five
-// 16-byte loads, eight byte-plane boxes by conversion and multiply-add, and a
+// k_trace walks the traversal's tree (BvhNodeQ): a node visit is eight
+// loads of one cache line, eight boxes of one multiply-add per plane, and a
 // sort of 32-bit keys whose low bits are the child's slot.  A node's hit
 // leaves are tested before its child nodes; the child nodes left over are one
 // group of two words on a stack that is short in LDS (12 groups by default,
@@ -75,6 +75,7 @@ struct TraceArgs
     const uint32_t* segTris;
     uint32_t        segCount;
     uint32_t        chunk; // rays per counter atomic (tuned)
+    uint32_t        lanes; // lanes of a wave that take rays
     // alpha test (the ALPHA kernels): per-triangle records by global id and
     // the texture table
     const AlphaRec* alpha;
@@ -193,11 +194,12 @@ __device__ __forceinline__ void LoadHalfNode( const void* nodes, uint32_t node, 
     }
 }
 
-// Distances of a traversal node's planes are fma(q, scale / d, (origin - o) / d);
-// against the exact distance of the byte plane the rounding errors are at
-// most 4 u |t| (u = 2^-24) and 3e-5 grid steps.  The planes were moved out by
-// 1e-3 steps, and the relative part of both sides is covered by scaling the
-// far distances by 1 + 2e-6 and the best hit so far by 1 + 1e-6: every box
+// Distances of a traversal node's planes are fma(q, scale / d, (origin - o) / d),
+// the far ones with both terms scaled by FAR_SLACK; against the exact
+// distance of the plane the rounding errors are at most 8 u |t| (u = 2^-24;
+// the hardware reciprocal's is in it) and 2^-11 grid steps.  The planes were
+// moved out by 2^-9 steps, and the relative part of both sides is covered by
+// the slack of the far distances, 33 u, and of the best hit so far: every box
 // that the exact ray meets before the best hit is visited.
 constexpr float FAR_SLACK  = 1.000002f;
 constexpr float BEST_SLACK = 1e-6f;
@@ -223,23 +225,30 @@ __device__ __forceinline__ void Sort8( uint32_t k[ 8 ] )
 #undef CS
 }
 
-__device__ __forceinline__ float ByteOf( uint32_t w, int k )
+typedef _Float16 half8 __attribute__( ( ext_vector_type( 8 ) ) );
+__device__ __forceinline__ half8 LoadHalves( const uint4* p )
 {
-    return float( ( w >> ( 8 * k ) ) & 0xFFu );
+    return *reinterpret_cast< const half8* >( p );
 }
 
-// Bound by instruction issue and by the latency of the chain stack -> node.
+// Bound by instruction issue (0.78 of the issue rate on 2.07M camera rays).
 // Against the walk of the FP32 nodes (14 loads, 48 subtractions and
 // products, a sort of 64-bit keys that carry the references): 2.07M camera
-// rays over 1.0M triangles 770 -> 304 us, 0.75M bounce rays 614 -> 257,
-// 1.24M shadow rays 963 -> 509, of which the cubic keys of the tree give
-// about a third; 14,400 rays over 10,592 triangles 150 -> 68 us.
-// 5 waves per SIMD (94 registers) measured as 4 (108), 6 spill and lose 5%.
+// rays over 1.0M triangles 746 -> 272 us, 0.75M bounce rays 614 -> 225,
+// 1.24M shadow rays 1015 -> 440, 14,400 rays over 10,592 triangles 148 -> 45.
+// About a third of it is the tree's cubic keys.  The steps run in a loop of
+// their own within the refills: with the refill in the same loop the
+// compiler copied some 70 registers per step (camera 304 -> 285 us).
+// 4 waves per SIMD: left to itself the compiler takes 140 registers and 3
+// waves (+7%); 5 waves spill (+28%).  Measured and dropped: making lanes
+// wait until 4, 8 or 12 hold leaves (+5, +10, +14%), reading the next node's
+// first row ahead of the leaf tests (+6%).
 template< int STACK_LDS, bool ALPHA >
-__global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
+__global__ __launch_bounds__( TR_THREADS, 4 ) void k_trace( TraceArgs a )
 {
     constexpr int    GROUPS = STACK_LDS / 2; // groups of child nodes in LDS
     __shared__ uint2 s_stack[ GROUPS * TR_THREADS ];
+    __shared__ uint32_t s_slots[ 256 ]; // the bits of a byte, three bits each, lowest first
     // The frame's entry roots, staged in LDS once per block: read from the
     // kernel arguments inside the loop they would hold 64 scalar registers,
     // which the compiler spills to vector-register lanes and reloads.
@@ -247,6 +256,15 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
     __shared__ float    s_rootBox[ 8 ][ 6 ];
 
     const int      tid       = threadIdx.x;
+    static_assert( TR_THREADS == 256, "one table entry per thread" );
+    {
+        uint32_t slots = 0u;
+        for( int b = 7; b >= 0; b-- )
+        {
+            slots = ( tid >> b ) & 1 ? slots << 3 | uint32_t( b ) : slots;
+        }
+        s_slots[ tid ] = slots;
+    }
     if( tid < 8 )
     {
         s_rootMask[ tid ] = a.rootMask[ tid ];
@@ -259,15 +277,17 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
     }
     __syncthreads();
     const int      lane      = tid & 63;
-    const uint64_t ltMask    = lane == 0 ? 0ull : ( ~0ull >> ( 64 - lane ) );
-    const uint32_t gthread   = blockIdx.x * TR_THREADS + tid;
-    uint2*         ovf       = reinterpret_cast< uint2* >( a.overflowStack + size_t( gthread ) * a.ovfStride );
+    // this lane's part of the stack in global memory (its address is not
+    // kept: it is needed once in thousands of visits)
+    auto ovf = [ & ]( int g ) __attribute__( ( always_inline ) ) {
+        return reinterpret_cast< uint2* >( a.overflowStack + size_t( blockIdx.x * TR_THREADS + tid ) * a.ovfStride ) + g;
+    };
     const int      maxGroups = GROUPS + int( a.ovfStride / 2 );
     const bool     anyHit    = ( a.flags & RG_EXT_TRACE_ANY_HIT ) != 0;
     const bool     cullFront = ( a.flags & RG_EXT_TRACE_CULL_FRONT_FACE ) != 0;
     const BvhNodeQ* nodes    = reinterpret_cast< const BvhNodeQ* >( a.nodes );
 
-    bool     active = false, exhausted = false;
+    bool     active = false, exhausted = uint32_t( lane ) >= a.lanes;
     uint32_t rayId  = 0;
     RayPre   ray;
     float    tmin = 0.0f, bestT = 0.0f, bestU = 0.0f, bestV = 0.0f, bestBox = 0.0f;
@@ -293,7 +313,7 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
         }
         else if( sp < maxGroups )
         {
-            ovf[ sp - GROUPS ] = e;
+            *ovf( sp - GROUPS ) = e;
         }
         else
         {
@@ -310,10 +330,10 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
         // take rays from the chunk (wave-uniform bookkeeping, no atomic).
         const bool     need = !active && !exhausted;
         const uint64_t mask = __ballot( need );
-        if( mask != 0ull && ( __popcll( mask ) >= REFILL_MIN_LANES || __ballot( active ) == 0ull ) )
+        if( mask != 0ull )
         {
             const uint32_t cnt    = __popcll( mask );
-            const uint32_t rank   = __popcll( mask & ltMask );
+            const uint32_t rank   = __builtin_amdgcn_mbcnt_hi( uint32_t( mask >> 32 ), __builtin_amdgcn_mbcnt_lo( uint32_t( mask ), 0u ) );
             const uint32_t left   = chunkEnd - chunkNext;
             const int      leader = __ffsll( ( long long )mask ) - 1;
             uint32_t       newBase = 0;
@@ -327,7 +347,7 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
                     const uint64_t g = uint64_t( j ) * a.partitions + part;
                     b                = g * a.chunk < a.count ? uint32_t( g * a.chunk ) : a.count;
                 }
-                newBase = __shfl( b, leader, 64 );
+                newBase = __builtin_amdgcn_readlane( b, leader );
             }
             if( need )
             {
@@ -346,6 +366,10 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
                     rayId            = my;
                     ray              = MakeRayPre( mk3( r.origin[ 0 ], r.origin[ 1 ], r.origin[ 2 ] ),
                                                    mk3( r.direction[ 0 ], r.direction[ 1 ], r.direction[ 2 ] ) );
+                    // the reciprocals only place boxes: a unit in the last place
+                    // is inside the slack
+                    ray.invd         = mk3( __builtin_amdgcn_rcpf( GuardDir( ray.d.x ) ), __builtin_amdgcn_rcpf( GuardDir( ray.d.y ) ),
+                                            __builtin_amdgcn_rcpf( GuardDir( ray.d.z ) ) );
                     sgn              = ( ray.invd.x < 0.0f ? 1u : 0u ) | ( ray.invd.y < 0.0f ? 2u : 0u ) | ( ray.invd.z < 0.0f ? 4u : 0u );
                     tmin             = r.tmin;
                     bestT            = r.tmax;
@@ -393,7 +417,7 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
                                 float tn;
                                 if( uint32_t( k ) < a.rootCount && ( s_rootMask[ k ] & rm ) != 0u &&
                                     SlabTest( ray, s_rootBox[ k ][ 0 ], s_rootBox[ k ][ 1 ], s_rootBox[ k ][ 2 ], s_rootBox[ k ][ 3 ],
-                                              s_rootBox[ k ][ 4 ], s_rootBox[ k ][ 5 ], tmin, bestT, &tn ) )
+                                              s_rootBox[ k ][ 4 ], s_rootBox[ k ][ 5 ], tmin, bestBox, &tn, FAR_SLACK ) )
                                 {
                                     if( kids )
                                     {
@@ -459,142 +483,154 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace( TraceArgs a )
             }
             break;
         }
-        if( !active )
+        // steps until enough lanes are idle for a refill, or all are
+        do
         {
-            continue;
-        }
-
-        bool finished = false;
-        if( ++steps > MAX_STEPS_PER_RAY )
-        {
-            // Only a malformed tree can get here; end the ray instead of spinning.
-            atomicOr( a.errorFlag, RG_EXT_TRACE_ERROR_STEP_LIMIT );
-            finished = true;
-        }
-        else
-        {
-            if( leaves == 0u )
+            if( active )
             {
-                nodeVisits++;
-                const uint4*   np = reinterpret_cast< const uint4* >( nodes + ( base + ( list & 7u ) ) );
-                const uint4    r0 = np[ 0 ], r1 = np[ 1 ], r2 = np[ 2 ], r3 = np[ 3 ];
-                const uint2    r4 = *reinterpret_cast< const uint2* >( np + 4 );
-                list >>= 3;
-                kids--;
-                // per axis: scale / d and (origin - o) / d, and the byte planes
-                // that the ray enters and leaves through
-                const float sx = __uint_as_float( ( r0.w & 0xFFu ) << 23 ) * ray.invd.x, bx = ( __uint_as_float( r0.x ) - ray.o.x ) * ray.invd.x;
-                const float sy = __uint_as_float( ( r0.w & 0xFF00u ) << 15 ) * ray.invd.y, by = ( __uint_as_float( r0.y ) - ray.o.y ) * ray.invd.y;
-                const float sz = __uint_as_float( ( r0.w & 0xFF0000u ) << 7 ) * ray.invd.z, bz = ( __uint_as_float( r0.z ) - ray.o.z ) * ray.invd.z;
-                const float fsx = sx * FAR_SLACK, fbx = bx * FAR_SLACK, fsy = sy * FAR_SLACK, fby = by * FAR_SLACK, fsz = sz * FAR_SLACK, fbz = bz * FAR_SLACK;
-                const bool     nx = ( sgn & 1u ) != 0u, ny = ( sgn & 2u ) != 0u, nz = ( sgn & 4u ) != 0u;
-                const uint32_t qnx[ 2 ] = { nx ? r2.z : r1.x, nx ? r2.w : r1.y }, qfx[ 2 ] = { nx ? r1.x : r2.z, nx ? r1.y : r2.w };
-                const uint32_t qny[ 2 ] = { ny ? r3.x : r1.z, ny ? r3.y : r1.w }, qfy[ 2 ] = { ny ? r1.z : r3.x, ny ? r1.w : r3.y };
-                const uint32_t qnz[ 2 ] = { nz ? r3.z : r2.x, nz ? r3.w : r2.y }, qfz[ 2 ] = { nz ? r2.x : r3.z, nz ? r2.y : r3.w };
-                const uint32_t inner = ( r0.w >> 24 ) & 15u, leaf = r0.w >> 28;
-                uint32_t       key[ 8 ], hits = 0u;
+                bool finished = false;
+                steps++;
+                if( leaves == 0u )
+                {
+                    nodeVisits++;
+                    // rows of 16 bytes: origin and meta, then per axis the lo
+                    // and the hi planes, of which the sign of the direction
+                    // says which one the ray enters through, then the bases
+                    const uint4*   np = reinterpret_cast< const uint4* >( nodes + ( base + ( list & 7u ) ) );
+                    const uint32_t nx = sgn & 1u, ny = ( sgn >> 1 ) & 1u, nz = ( sgn >> 2 ) & 1u;
+                    const uint4    r0 = np[ 0 ];
+                    const half8    qnx = LoadHalves( np + 1 + nx ), qfx = LoadHalves( np + 2 - nx );
+                    const half8    qny = LoadHalves( np + 3 + ny ), qfy = LoadHalves( np + 4 - ny );
+                    const half8    qnz = LoadHalves( np + 5 + nz ), qfz = LoadHalves( np + 6 - nz );
+                    const uint2    r7 = *reinterpret_cast< const uint2* >( np + 7 );
+                    list >>= 3;
+                    kids--;
+                    // per axis: scale / d and (origin - o) / d
+                    const float sx = __uint_as_float( ( r0.w & 0xFFu ) << 23 ) * ray.invd.x, bx = ( __uint_as_float( r0.x ) - ray.o.x ) * ray.invd.x;
+                    const float sy = __uint_as_float( ( r0.w & 0xFF00u ) << 15 ) * ray.invd.y, by = ( __uint_as_float( r0.y ) - ray.o.y ) * ray.invd.y;
+                    const float sz = __uint_as_float( ( r0.w & 0xFF0000u ) << 7 ) * ray.invd.z, bz = ( __uint_as_float( r0.z ) - ray.o.z ) * ray.invd.z;
+                    const float fsx = sx * FAR_SLACK, fbx = bx * FAR_SLACK, fsy = sy * FAR_SLACK, fby = by * FAR_SLACK, fsz = sz * FAR_SLACK, fbz = bz * FAR_SLACK;
+                    const uint32_t inner = ( r0.w >> 24 ) & 15u, leaf = r0.w >> 28;
+                    uint32_t       key[ 8 ], hits = 0u;
 #pragma unroll
-                for( int k = 0; k < 8; k++ )
-                {
-                    const int   w = k >> 2, j = k & 3;
-                    const float tx0 = __builtin_fmaf( ByteOf( qnx[ w ], j ), sx, bx ), tx1 = __builtin_fmaf( ByteOf( qfx[ w ], j ), fsx, fbx );
-                    const float ty0 = __builtin_fmaf( ByteOf( qny[ w ], j ), sy, by ), ty1 = __builtin_fmaf( ByteOf( qfy[ w ], j ), fsy, fby );
-                    const float tz0 = __builtin_fmaf( ByteOf( qnz[ w ], j ), sz, bz ), tz1 = __builtin_fmaf( ByteOf( qfz[ w ], j ), fsz, fbz );
-                    const float tn  = fmaxf( fmaxf( fmaxf( tx0, ty0 ), tz0 ), tmin );
-                    const float tf  = fminf( fminf( fminf( tx1, ty1 ), tz1 ), bestBox );
-                    const bool  h   = tn <= tf;
-                    hits |= h ? 1u << k : 0u;
-                    key[ k ] = h && uint32_t( k ) < inner ? ( __float_as_uint( tn ) & ~7u ) | uint32_t( k ) : ~0u;
-                }
-                const uint32_t innerMask = ( 1u << inner ) - 1u;
-                leaves                   = hits & ( ( ( 1u << leaf ) - 1u ) << inner );
-                leafBase                 = r4.y;
-                const uint32_t found     = __popc( hits & innerMask );
-                if( found )
-                {
-                    if( kids )
+                    for( int k = 0; k < 8; k++ )
                     {
-                        push( base, kids, list );
+                        const float tx0 = __builtin_fmaf( float( qnx[ k ] ), sx, bx ), tx1 = __builtin_fmaf( float( qfx[ k ] ), fsx, fbx );
+                        const float ty0 = __builtin_fmaf( float( qny[ k ] ), sy, by ), ty1 = __builtin_fmaf( float( qfy[ k ] ), fsy, fby );
+                        const float tz0 = __builtin_fmaf( float( qnz[ k ] ), sz, bz ), tz1 = __builtin_fmaf( float( qfz[ k ] ), fsz, fbz );
+                        const float tn  = fmaxf( fmaxf( fmaxf( tx0, ty0 ), tz0 ), tmin );
+                        const float tf  = fminf( fminf( fminf( tx1, ty1 ), tz1 ), bestBox );
+                        const bool  h   = tn <= tf;
+                        hits |= h ? 1u << k : 0u;
+                        key[ k ] = h && uint32_t( k ) < inner ? ( __float_as_uint( tn ) & ~7u ) | uint32_t( k ) : ~0u;
                     }
-                    Sort8( key );
-                    base = r4.x;
-                    kids = found;
-                    list = 0u;
-#pragma unroll
-                    for( int k = 7; k >= 0; k-- )
+                    const uint32_t innerMask = ( 1u << inner ) - 1u;
+                    leaves                   = hits & ( ( ( 1u << leaf ) - 1u ) << inner );
+                    leafBase                 = r7.y;
+                    const uint32_t found     = __popc( hits & innerMask );
+                    if( found )
                     {
-                        list = list << 3 | ( key[ k ] & 7u );
-                    }
-                }
-            }
-            if( leaves )
-            {
-                triTests++;
-                const uint32_t slot = __ffs( leaves ) - 1;
-                leaves &= leaves - 1u;
-                const float4* tp = a.tris + size_t( leafBase + slot ) * 3;
-                const float4  q0 = tp[ 0 ], q1 = tp[ 1 ], q2 = tp[ 2 ];
-                float         t, u, v;
-                if( IntersectTri( ray, mk3( q0.x, q0.y, q0.z ), mk3( q1.x, q1.y, q1.z ), mk3( q2.x, q2.y, q2.z ), tmin, bestT, cullFront, &t, &u, &v ) )
-                {
-                    const uint32_t prim = __float_as_uint( q0.w );
-                    bool           take = t < bestT || prim < bestPrim;
-                    if constexpr( ALPHA )
-                    {
-                        const AlphaRec& ar = a.alpha[ prim ];
-                        if( take && TexValid( a.tex, ar.tex ) && !AlphaPasses( a.tex, ar, u, v ) )
+                        if( kids )
                         {
-                            take = false; // ignoreIntersectionEXT
+                            push( base, kids, list );
+                        }
+                        base = r7.x;
+                        kids = found;
+                        if( anyHit )
+                        {
+                            // the interval never shrinks before the ray ends:
+                            // slot order (1.24M shadow rays visit 3% fewer
+                            // nodes so than near to far)
+                            list = s_slots[ hits & innerMask ];
+                        }
+                        else
+                        {
+                            Sort8( key );
+                            // three bits per slot, shifted in from the top
+                            list = 0u;
+#pragma unroll
+                            for( int k = 0; k < 8; k++ )
+                            {
+                                list = key[ k ] << 29 | list >> 3;
+                            }
+                            list >>= 8;
                         }
                     }
-                    if( take )
+                }
+                if( leaves )
+                {
+                    triTests++;
+                    const uint32_t slot = __ffs( leaves ) - 1;
+                    leaves &= leaves - 1u;
+                    const float4* tp = a.tris + size_t( leafBase + slot ) * 3;
+                    const float4  q0 = tp[ 0 ], q1 = tp[ 1 ], q2 = tp[ 2 ];
+                    float         t, u, v;
+                    if( IntersectTri( ray, mk3( q0.x, q0.y, q0.z ), mk3( q1.x, q1.y, q1.z ), mk3( q2.x, q2.y, q2.z ), tmin, bestT, cullFront, &t, &u, &v ) )
                     {
-                        bestT    = t;
-                        bestBox  = t + fabsf( t ) * BEST_SLACK;
-                        bestU    = u;
-                        bestV    = v;
-                        bestPrim = prim;
-                        finished = anyHit;
+                        const uint32_t prim = __float_as_uint( q0.w );
+                        bool           take = t < bestT || prim < bestPrim;
+                        if constexpr( ALPHA )
+                        {
+                            const AlphaRec& ar = a.alpha[ prim ];
+                            if( take && TexValid( a.tex, ar.tex ) && !AlphaPasses( a.tex, ar, u, v ) )
+                            {
+                                take = false; // ignoreIntersectionEXT
+                            }
+                        }
+                        if( take )
+                        {
+                            bestT    = t;
+                            bestBox  = t + fabsf( t ) * BEST_SLACK;
+                            bestU    = u;
+                            bestV    = v;
+                            bestPrim = prim;
+                            finished = anyHit;
+                        }
                     }
                 }
-            }
-            if( !finished && leaves == 0u && kids == 0u )
-            {
-                if( sp == 0 )
+                if( leaves == 0u && kids == 0u )
                 {
-                    finished = true;
-                }
-                else
-                {
-                    sp--;
-                    uint2 e;
-                    if( sp < GROUPS )
+                    if( sp == 0 )
                     {
-                        e = s_stack[ sp * TR_THREADS + tid ];
+                        finished = true;
                     }
                     else
                     {
-                        // Keeps the rare overflow read a separate global load
-                        // (no generic-address load on the common LDS path).
-                        asm volatile( "" ::: "memory" );
-                        e = ovf[ sp - GROUPS ];
+                        sp--;
+                        uint2 e;
+                        if( sp < GROUPS )
+                        {
+                            e = s_stack[ sp * TR_THREADS + tid ];
+                        }
+                        else
+                        {
+                            // Keeps the rare overflow read a separate global load
+                            // (no generic-address load on the common LDS path).
+                            asm volatile( "" ::: "memory" );
+                            e = *ovf( sp - GROUPS );
+                        }
+                        base = e.x & 0x0FFFFFFFu;
+                        kids = e.x >> 28;
+                        list = e.y;
                     }
-                    base = e.x & 0x0FFFFFFFu;
-                    kids = e.x >> 28;
-                    list = e.y;
+                }
+                if( finished || steps > MAX_STEPS_PER_RAY )
+                {
+                    if( !finished )
+                    {
+                        // Only a malformed tree can get here; end the ray instead of spinning.
+                        atomicOr( a.errorFlag, RG_EXT_TRACE_ERROR_STEP_LIMIT );
+                    }
+                    RgExtHit h;
+                    h.t                = bestT;
+                    h.u                = bestU;
+                    h.v                = bestV;
+                    h.primitiveId      = bestPrim == RG_EXT_MISS ? RG_EXT_MISS : bestPrim - triBase;
+                    a.hits[ rayId ]    = h;
+                    active             = false;
                 }
             }
-        }
-        if( finished )
-        {
-            RgExtHit h;
-            h.t                = bestT;
-            h.u                = bestU;
-            h.v                = bestV;
-            h.primitiveId      = bestPrim == RG_EXT_MISS ? RG_EXT_MISS : bestPrim - triBase;
-            a.hits[ rayId ]    = h;
-            active             = false;
-        }
+        } while( __ballot( active ) != 0ull && __popcll( __ballot( !active && !exhausted ) ) < int( REFILL_MIN_LANES ) );
     }
 }
 
@@ -1005,6 +1041,22 @@ TraceKernelFn ViewKernel( uint32_t nodeFormat )
     return nodeFormat == RG_EXT_BVH_NODE_FP16 ? k_trace_view< true > : k_trace_view< false >;
 }
 
+// Lanes of each wave that take rays: as few as still give the resident waves
+// every ray at once, 4 at least.  A small launch lasts as long as its slowest
+// wave, and a wave of fewer rays has a shorter longest chain: 14,400 camera
+// rays over 10,592 triangles 67 -> 54 us with 4 lanes, 57,600 60 -> 55 with
+// 16, 129,600 74 -> 71 with 32.  With more rays than resident lanes the same
+// widths are slower (230,400 rays: 71 us with 64 lanes, 79 with 32).
+uint32_t LanesPerWave( uint32_t count, uint32_t gridBlocks )
+{
+    uint32_t lanes = 4;
+    while( lanes < 64u && uint64_t( lanes ) * gridBlocks * ( TR_THREADS / 64 ) < count )
+    {
+        lanes *= 2;
+    }
+    return lanes;
+}
+
 uint32_t ResidentBlocks( TraceKernelFn k, int cus )
 {
     int perCu = 0;
@@ -1063,7 +1115,8 @@ void TraceRaysImpl( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
     const bool     view   = !frame && !accum && ( flags & RG_EXT_TRACE_COLLECT_STATS ) != 0;
     const int      v      = int( s.stackVariant < TRACE_STACK_VARIANTS ? s.stackVariant : 1u );
     const uint32_t grid   = s.grid[ view ? TRACE_STACK_VARIANTS : v ];
-    const uint32_t blocks = DivUp( count, TR_THREADS ) < grid ? DivUp( count, TR_THREADS ) : grid;
+    const uint32_t lanes  = view ? 64u : LanesPerWave( count, grid );
+    const uint32_t blocks = std::min( DivUp( count, lanes * ( TR_THREADS / 64 ) ), grid );
     s.counter.Reserve( ( RAY_PARTITIONS * COUNTER_STRIDE + 1 ) * sizeof( uint32_t ) );
     s.stats.Reserve( 2 * sizeof( uint64_t ) );
     RG_HIP_CHECK( hipMemsetAsync( s.counter.ptr, 0, ( RAY_PARTITIONS * COUNTER_STRIDE + 1 ) * sizeof( uint32_t ), stream ) );
@@ -1113,7 +1166,8 @@ void TraceRaysImpl( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
             }
         }
     }
-    a.chunk         = s.rayChunk >= 16 && s.rayChunk <= 1024 ? s.rayChunk : RAY_CHUNK_DEFAULT;
+    a.lanes         = lanes;
+    a.chunk         = lanes < 64u ? lanes : ( s.rayChunk >= 16 && s.rayChunk <= 1024 ? s.rayChunk : RAY_CHUNK_DEFAULT );
     a.alpha         = alpha && tex ? alpha : nullptr;
     a.tex           = tex ? *tex : TexView{};
     if( accum )
@@ -1233,7 +1287,8 @@ void TraceRaysNoAlloc( const BvhObject& bvh, const RgExtRay* d_rays, uint32_t co
         return;
     }
     const bool     view   = ( flags & RG_EXT_TRACE_COLLECT_STATS ) != 0;
-    const uint32_t blocks = std::min( DivUp( count, TR_THREADS ), nd.grid[ view ? 1 : 0 ] );
+    const uint32_t lanes  = view ? 64u : LanesPerWave( count, nd.grid[ 0 ] );
+    const uint32_t blocks = std::min( DivUp( count, lanes * ( TR_THREADS / 64 ) ), nd.grid[ view ? 1 : 0 ] );
     RG_REQUIRE( size_t( blocks ) * TR_THREADS * NOALLOC_OVF <= NOALLOC_WORDS - NOALLOC_HEADER, RG_RESULT_INTERNAL_ERROR,
                 "no-alloc traversal grid exceeds its scratch" );
     k_noalloc_clear<<< 1, 64, 0, stream >>>( nd.scratch );
@@ -1259,7 +1314,8 @@ void TraceRaysNoAlloc( const BvhObject& bvh, const RgExtRay* d_rays, uint32_t co
     {
         a.rootRef[ k ] = 0;
     }
-    a.chunk = RAY_CHUNK_DEFAULT;
+    a.lanes = lanes;
+    a.chunk = lanes < 64u ? lanes : RAY_CHUNK_DEFAULT;
     a.alpha = nullptr;
     a.tex   = TexView{};
     hipLaunchKernelGGL( view ? ViewKernel( bvh.nodeFormat ) : TraceKernel( NOALLOC_VARIANT, false ), dim3( blocks ), dim3( TR_THREADS ), 0, stream, a );

@@ -65,13 +65,13 @@ __host__ __device__ __forceinline__ RayPre MakeRayPre( v3 o, v3 d )
 __host__ __device__ __forceinline__ bool SlabTest( const RayPre& r,
                                                    float lx, float ly, float lz,
                                                    float hx, float hy, float hz,
-                                                   float tmin, float tmax, float* tnearOut )
+                                                   float tmin, float tmax, float* tnearOut, float farSlack = 1.0000004f )
 {
     const float tx0 = ( lx - r.o.x ) * r.invd.x, tx1 = ( hx - r.o.x ) * r.invd.x;
     const float ty0 = ( ly - r.o.y ) * r.invd.y, ty1 = ( hy - r.o.y ) * r.invd.y;
     const float tz0 = ( lz - r.o.z ) * r.invd.z, tz1 = ( hz - r.o.z ) * r.invd.z;
     const float tn  = fmaxf( fmaxf( fminf( tx0, tx1 ), fminf( ty0, ty1 ) ), fmaxf( fminf( tz0, tz1 ), tmin ) );
-    const float tf  = fminf( fminf( fmaxf( tx0, tx1 ), fmaxf( ty0, ty1 ) ), fmaxf( tz0, tz1 ) ) * 1.0000004f;
+    const float tf  = fminf( fminf( fmaxf( tx0, tx1 ), fmaxf( ty0, ty1 ) ), fmaxf( tz0, tz1 ) ) * farSlack;
     *tnearOut       = tn;
     return tn <= fminf( tf, tmax );
 }

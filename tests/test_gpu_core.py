@@ -266,6 +266,26 @@ def test_traversal_nodes_at_their_limits(gpu, kind):
     assert np.array_equal(occ, g["prim"] != RG_EXT_MISS)
 
 
+@pytest.mark.parametrize("n", [1, 5, 4097, 16383, 16385, 65537, 131073, 262145, 300001])
+def test_launch_widths(gpu, n):
+    """Ray counts about the change between the lanes per wave that take rays
+    (powers of two times the resident waves): every ray has its hit, those of
+    the walk over the published nodes."""
+    print(f"launch width {n}", flush=True)
+    s = scenes.terrain_boxes_scene()
+    r = np.random.default_rng(n)
+    rays = np.zeros(n, RAY_DTYPE)
+    rays["origin"] = r.uniform(-30, 30, (n, 3)) + np.array([0, 8, 0])
+    d = r.normal(size=(n, 3)) - np.array([0, 0.5, 0])
+    rays["direction"] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    rays["tmax"] = 1000.0
+    b, _ = _gpu_bvh(s.tris, 1)
+    v = _trace_gpu(b, rays, RG_EXT_TRACE_COLLECT_STATS)
+    for _ in range(2):  # the second launch finds the counters of the first
+        _assert_same_hits(_trace_gpu(b, rays, 0), v)
+        _assert_same_hits(_trace_gpu(b, rays, RG_EXT_TRACE_ANY_HIT), v, any_hit=True)
+
+
 def test_histogram_bit_exact(gpu, oracle):
     r = np.random.default_rng(11)
     w, h = 1920, 1080
