@@ -147,7 +147,11 @@ void BuildFrameBvh( BvhObject& bvh, const float* d_tris, const uint32_t* classTr
 
 constexpr int TRACE_STACK_VARIANTS = 3;
 
-// Per-caller traversal scratch: the ray counter, an overflow-flag word and
+// Sets of ray counters a context holds, one for each launch that
+// ClearTraceCounters prepares (a frame traces 6 to 8 times and more).
+constexpr uint32_t TRACE_COUNTER_SETS = 8;
+
+// Per-caller traversal scratch: the ray counters, an overflow-flag word and
 // the global overflow stacks of the persistent grid.  Launches that share a
 // context must not overlap on the device.
 struct TraceContext
@@ -163,12 +167,27 @@ struct TraceContext
     uint32_t     rayChunk     = 64;                     // rays per counter atomic
 };
 
-// Device accumulators a caller clears once and lets several launches add to.
+// Device accumulators that several launches add to.  Each of these launches
+// takes a counter set of its own from the last ClearTraceCounters.
 struct TraceAccum
 {
     uint64_t* stats  = nullptr; // node visits, triangle tests (with RG_EXT_TRACE_COLLECT_STATS)
     uint32_t* errors = nullptr; // OR of RG_EXT_TRACE_ERROR_* bits
+    uint32_t  counterSet = 0;   // below TRACE_COUNTER_SETS
+    // When this launch runs, in ticks of the device's wall clock (low words):
+    // block 0's start, then each block's end; *blocks is set to their number.
+    // In the kernel, because events recorded around every traversal of a frame
+    // are packets that hold up the stream: 11 us a launch between kernels, a
+    // tenth of a 640x360 frame.  A word per block, because waves that add to a
+    // few shared words wait for each other: 20 us a launch with eight.
+    uint32_t* times     = nullptr;
+    uint32_t  timeWords = 0;
+    uint32_t* blocks    = nullptr;
 };
+
+// Clears every counter set of ctx for the launches that follow on stream,
+// and accum's statistics and error word where given.
+void ClearTraceCounters( TraceContext& ctx, const TraceAccum* accum, hipStream_t stream );
 
 // evBefore / evAfter (optional) are recorded right around the kernel launch.
 // Without accum, the statistics and error bits of this launch alone are kept
@@ -182,8 +201,8 @@ void TraceRays( const BvhObject& bvh, TraceContext& ctx, const RgExtRay* d_rays,
 // alpha (with tex): per-triangle alpha-test records; the hits of
 // alpha-tested triangles whose texture is transparent there are ignored.
 void TraceRaysFrame( const BvhObject& bvh, TraceContext& ctx, const RgExtRay* d_rays, const uint8_t* d_rayMasks, uint32_t defaultMask, uint32_t count,
-                     RgExtHit* d_hits, uint32_t flags, const uint32_t* classMasks, uint32_t classCount, hipStream_t stream, hipEvent_t evBefore,
-                     hipEvent_t evAfter, const TraceAccum* accum, const struct AlphaRec* alpha = nullptr, const struct TexView* tex = nullptr );
+                     RgExtHit* d_hits, uint32_t flags, const uint32_t* classMasks, uint32_t classCount, hipStream_t stream, const TraceAccum* accum,
+                     const struct AlphaRec* alpha = nullptr, const struct TexView* tex = nullptr );
 // One persistent launch over the rays of every scene of a batched BVH: rays
 // of scene s are [rayOffsets[s], rayOffsets[s+1]) (host array, sceneCount + 1
 // entries); primitive ids in the hits are relative to the scene.

@@ -235,9 +235,8 @@ void FinishFrame( FrameGpu& g, const RgExtFrameParams& p, FramebufferSet& fb, co
     }
     LuminanceHistogram( reinterpret_cast< const float* >( fb.Cur( RG_EXT_PLANE_HISTOGRAM_INPUT ) ), w * h, p.minLogLuminance, p.maxLogLuminance,
                         g.hist.as< uint32_t >(), s );
-    RG_HIP_CHECK( hipMemcpyAsync( g.histCopy.ptr, g.hist.ptr, 256 * 4, hipMemcpyDeviceToDevice, s ) );
     LuminanceAverage( g.hist.as< uint32_t >(), w * h, p.minLogLuminance, p.maxLogLuminance, p.timeDelta, p.stopEyeAdaptation != 0,
-                      g.avgLum.as< float >(), s );
+                      g.avgLum.as< float >(), s, g.histCopy.as< uint32_t >() );
     // ImageComposition::Finalize (Source/ImageComposition.cpp:94-156)
     const auto* tm       = FindParams< RgDrawFrameTonemappingParams >( di, RG_STRUCTURE_TYPE_TONEMAPPING );
     float       sat[ 3 ] = { 0.0f, 0.0f, 0.0f }, ct[ 3 ] = { 1.0f, 1.0f, 1.0f }; // DrawFrameInfo.h:104-105

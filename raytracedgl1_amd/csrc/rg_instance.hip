@@ -150,9 +150,8 @@ struct Instance
         };
         stats.gpuMsUpload       = ms( ST_BEGIN, ST_UPLOADED );
         stats.gpuMsAssemble     = ms( ST_UPLOADED, ST_ASSEMBLED );
-        stats.gpuMsTraversal    = g.pt.TraversalMs();
         stats.traversalLaunches = g.pt.traceLaunches;
-        g.pt.TraversalCounts( &stats.nodeVisits, &stats.triangleTests, &stats.traversalErrors );
+        g.pt.Traversal( &stats.gpuMsTraversal, &stats.nodeVisits, &stats.triangleTests, &stats.traversalErrors );
         stats.gpuMsBvh     = ms( ST_ASSEMBLED, ST_BVH );
         stats.gpuMsTrace   = ms( ST_BVH, ST_TRACED );
         stats.gpuMsDenoise = ms( ST_TRACED, ST_DENOISED );

@@ -21,7 +21,8 @@ struct LpmConsts
 
 // rg_tonemap.hip
 void LuminanceHistogram( const float* d_lum, uint32_t count, float minLog, float maxLog, uint32_t* d_hist, hipStream_t stream );
-void LuminanceAverage( uint32_t* d_hist, uint32_t pixelCount, float minLog, float maxLog, float timeDelta, bool stop, float* d_avg, hipStream_t stream );
+void LuminanceAverage( uint32_t* d_hist, uint32_t pixelCount, float minLog, float maxLog, float timeDelta, bool stop, float* d_avg, hipStream_t stream,
+                       uint32_t* d_kept = nullptr );
 LpmConsts MakeLpmConsts( const float saturation[ 3 ], const float crosstalk[ 3 ] );
 // PRE_FINAL -> FINAL: checkerboard resolve, auto exposure from *d_avgLum, LPM tone map
 // emissionMaxScreenColor weights SCREEN_EMISSION into the tone map's input.

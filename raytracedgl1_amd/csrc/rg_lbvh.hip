@@ -319,6 +319,33 @@ __global__ __launch_bounds__( THREADS ) void k_scene_roots( uint32_t internal, c
 // segments only) has no internal node: the published tree leaves it out, the
 // traversal's tree gives it a node of one leaf, so that scene s's root is
 // its node s.  With boxes: each root's box (lo xyz, hi xyz, 2 unused).
+// The words a build starts from: the collapse's level counts at 0, the node
+// flags at 0 and the scene roots at none; one launch for what were up to
+// four memsets of two kernels each.
+__global__ __launch_bounds__( THREADS ) void k_build_init( uint32_t* levels, uint32_t levelWords, uint32_t* isNode, uint32_t nodeWords, uint32_t* roots0,
+                                                           uint32_t* roots1, uint32_t rootWords )
+{
+    for( uint32_t i = blockIdx.x * THREADS + threadIdx.x; i < levelWords || i < nodeWords || i < rootWords; i += gridDim.x * THREADS )
+    {
+        if( i < levelWords )
+        {
+            levels[ i ] = 0u;
+        }
+        if( i < nodeWords )
+        {
+            isNode[ i ] = 0u;
+        }
+        if( i < rootWords && roots0 )
+        {
+            roots0[ i ] = RG_EXT_MISS;
+        }
+        if( i < rootWords && roots1 )
+        {
+            roots1[ i ] = RG_EXT_MISS;
+        }
+    }
+}
+
 __global__ void k_seed_frontier_seg( const uint32_t* roots, uint32_t S, const uint32_t* offsets, uint32_t internal, bool leaves, uint32_t* queue,
                                      uint32_t* counts, const float* bounds, float* boxes )
 {
@@ -1673,13 +1700,17 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
     CollapseSets       cs{};
     cs.s[ 0 ] = CollapseArgs{ ts.queue, levels + BVH_MAX_LEVELS + 1, levels, n, 1, ts.info, ts.rf, ts.rl, ts.expansion, nullptr, ts.nodeBase,
                               levels + LW * 2 };
-    RG_HIP_CHECK( hipMemsetAsync( levels, 0, ( LW * 2 + 1 ) * 4, stream ) );
     if( view )
     {
         cs.s[ 1 ] = CollapseArgs{ bvh.queue.as< uint32_t >(), levels + LW + BVH_MAX_LEVELS + 1, levels + LW, n, bvh.leafMax, bvh.expandInfo.as< uint4 >(),
                                   rf, rl, bvh.expansion.as< uint32_t >(), bvh.isNode8.as< uint32_t >(), nullptr, nullptr };
-        RG_HIP_CHECK( hipMemsetAsync( bvh.isNode8.ptr, 0, size_t( slots ) * 4, stream ) );
     }
+    uint32_t* const roots[ 2 ] = { batched ? ts.roots : nullptr, batched && view ? bvh.sceneRoots.as< uint32_t >() : nullptr };
+    const uint32_t  nodeWords  = view ? slots : 0u;
+    const uint32_t  initWords  = std::max( std::max( nodeWords, LW * 2 + 1 ), batched ? sceneCount : 0u );
+    k_build_init<<< std::min( DivUp( initWords, THREADS ), 1024u ), THREADS, 0, stream >>>( levels, LW * 2 + 1, view ? bvh.isNode8.as< uint32_t >() : nullptr,
+                                                                                          nodeWords, roots[ 0 ], roots[ 1 ], batched ? sceneCount : 0u );
+    CheckLaunch( "k_build_init" );
     if( !batched )
     {
         k_seed_frontier<<< 1, 64, 0, stream >>>( cs, sets );
@@ -1687,10 +1718,8 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
     }
     else
     {
-        uint32_t* const roots[ 2 ] = { ts.roots, bvh.sceneRoots.as< uint32_t >() };
         for( uint32_t k = 0; k < sets; k++ )
         {
-            RG_HIP_CHECK( hipMemsetAsync( roots[ k ], 0xFF, size_t( sceneCount ) * 4, stream ) );
             if( internal > 0 )
             {
                 k_scene_roots<<< DivUp( internal, THREADS ), THREADS, 0, stream >>>( internal, ta.s[ k ].rangeFirst, ta.s[ k ].rangeLast, offs, sceneCount,

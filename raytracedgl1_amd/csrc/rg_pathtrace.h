@@ -44,9 +44,18 @@ struct PathTracer
     uint32_t     geomMapCount = 0;
     DeviceBuffer grid[ 2 ];                // 16^3 * 128 light-grid reservoirs, ping-pong
     const uint32_t* blueNoise = nullptr;   // 128 layers of 128x128 RGBA8, one table per process
-    DeviceBuffer frameAccum;               // node visits, triangle tests (u64), error bits (u32) of the frame
-    static constexpr uint32_t TRACE_EVENT_PAIRS = 32; // traversal launches timed per frame
-    hipEvent_t   traceEv[ 2 * TRACE_EVENT_PAIRS ] = {};
+    // What a frame's traversal launches add up and when they ran.
+    struct FrameAccum
+    {
+        static constexpr uint32_t TIMED      = 32;   // launches timed per frame
+        static constexpr uint32_t TIME_WORDS = 2049; // of a launch: blocks + 1
+        uint64_t stats[ 2 ];                         // node visits, triangle tests
+        uint32_t errors, pad;                        // RG_EXT_TRACE_ERROR_*
+        uint32_t times[ TIMED ][ TIME_WORDS ];
+    };
+    uint32_t traceBlocks[ FrameAccum::TIMED ] = {}; // of the frame's launches (0: none ran)
+    DeviceBuffer frameAccum;
+    double       msPerTick     = 0.0; // of the device's wall clock
     uint32_t     traceLaunches = 0;
     bool         collectStats  = false;
     int          gridParity = 0;
@@ -56,11 +65,9 @@ struct PathTracer
     void Init( hipStream_t s );
     // Device bytes a path tracer owns apart from its wavefront buffers.
     static size_t OwnBytes();
-    ~PathTracer();
     // After the stream has finished the frame: traversal time summed over the
     // frame's launches, and the node / triangle counts when collected.
-    float    TraversalMs() const;
-    void     TraversalCounts( uint64_t* nodes, uint64_t* tris, uint32_t* errors ) const;
+    void Traversal( float* ms, uint64_t* nodes, uint64_t* tris, uint32_t* errors ) const;
     void Resize( uint32_t w, uint32_t h );
     void UploadLights( const SceneCollector& sc, hipStream_t s );
     void UploadGeomMap( const std::vector< uint32_t >& map, hipStream_t s );

@@ -20,6 +20,8 @@
 #include "rg_shading.h"
 #include "rg_textures.h"
 
+#include <algorithm>
+#include <cstddef>
 #include <mutex>
 
 namespace rg
@@ -2168,41 +2170,28 @@ __global__ __launch_bounds__( THREADS ) void k_grad_b( RgExtFrameParams p, FbPtr
 
 } // namespace
 
-PathTracer::~PathTracer()
+void PathTracer::Traversal( float* ms, uint64_t* nodes, uint64_t* tris, uint32_t* errors ) const
 {
-    for( auto& e : traceEv )
-    {
-        if( e )
-        {
-            ( void )hipEventDestroy( e );
-        }
-    }
-}
-
-float PathTracer::TraversalMs() const
-{
-    float total = 0.0f;
-    for( uint32_t k = 0; k < traceLaunches; k++ )
-    {
-        float ms = 0.0f;
-        if( hipEventElapsedTime( &ms, traceEv[ 2 * k ], traceEv[ 2 * k + 1 ] ) == hipSuccess )
-        {
-            total += ms;
-        }
-    }
-    return total;
-}
-
-void PathTracer::TraversalCounts( uint64_t* nodes, uint64_t* tris, uint32_t* errors ) const
-{
-    uint64_t v[ 3 ] = {};
+    std::vector< uint8_t > host( sizeof( FrameAccum ) );
+    const auto&            v = *reinterpret_cast< const FrameAccum* >( host.data() );
     if( traceLaunches > 0 )
     {
-        RG_HIP_CHECK( hipMemcpy( v, frameAccum.ptr, sizeof( v ), hipMemcpyDeviceToHost ) );
+        const uint32_t timed = std::min( traceLaunches, FrameAccum::TIMED );
+        RG_HIP_CHECK( hipMemcpy( host.data(), frameAccum.ptr, offsetof( FrameAccum, times ) + timed * sizeof( v.times[ 0 ] ), hipMemcpyDeviceToHost ) );
     }
-    *nodes  = collectStats ? v[ 0 ] : 0;
-    *tris   = collectStats ? v[ 1 ] : 0;
-    *errors = uint32_t( v[ 2 ] );
+    *ms     = 0.0f;
+    *nodes  = collectStats ? v.stats[ 0 ] : 0;
+    *tris   = collectStats ? v.stats[ 1 ] : 0;
+    *errors = v.errors;
+    for( uint32_t k = 0; k < FrameAccum::TIMED && k < traceLaunches; k++ )
+    {
+        int32_t ticks = 0; // of the last block's end after the start
+        for( uint32_t b = 0; b < traceBlocks[ k ]; b++ )
+        {
+            ticks = std::max( ticks, int32_t( v.times[ k ][ 1 + b ] - v.times[ k ][ 0 ] ) );
+        }
+        *ms += float( ticks * msPerTick );
+    }
 }
 
 namespace
@@ -2262,16 +2251,16 @@ void Wavefront::Reserve( size_t n )
 
 size_t PathTracer::OwnBytes()
 {
-    return 2 * size_t( GRID_ENTRIES ) * 16 + 3 * sizeof( uint64_t );
+    return 2 * size_t( GRID_ENTRIES ) * 16 + sizeof( FrameAccum );
 }
 
 void PathTracer::Init( hipStream_t s )
 {
-    for( auto& e : traceEv )
-    {
-        RG_HIP_CHECK( hipEventCreate( &e ) );
-    }
-    frameAccum.Reserve( 3 * sizeof( uint64_t ) );
+    int dev = 0, khz = 0;
+    RG_HIP_CHECK( hipGetDevice( &dev ) );
+    RG_HIP_CHECK( hipDeviceGetAttribute( &khz, hipDeviceAttributeWallClockRate, dev ) );
+    msPerTick = khz > 0 ? 1.0 / khz : 0.0;
+    frameAccum.Reserve( sizeof( FrameAccum ) );
     blueNoise = SharedBlueNoise( s );
     for( int k = 0; k < 2; k++ )
     {
@@ -2410,10 +2399,10 @@ uint64_t TraceFrames( const TraceSlot* slots, uint32_t B, const BvhObject& bvh, 
     const bool haveGeometry = grouped ? bvh.nodeCount > 0 : scene.triCount > 0 && !bvh.frameSegs.empty();
 
     lead.traceLaunches = 0;
-    RG_HIP_CHECK( hipMemsetAsync( lead.frameAccum.ptr, 0, 3 * sizeof( uint64_t ), s ) );
     TraceAccum accum;
-    accum.stats  = lead.frameAccum.as< uint64_t >();
-    accum.errors = reinterpret_cast< uint32_t* >( lead.frameAccum.as< uint64_t >() + 2 );
+    auto* const fa = lead.frameAccum.as< PathTracer::FrameAccum >();
+    accum.stats    = fa->stats;
+    accum.errors   = &fa->errors;
     // The frame's TLAS: each geometry class with its instance mask, or 0
     // when rayCullMaskWorld leaves its world out (ASManager.cpp:837-963).
     uint32_t classMasks[ GC_COUNT ];
@@ -2421,6 +2410,7 @@ uint64_t TraceFrames( const TraceSlot* slots, uint32_t B, const BvhObject& bvh, 
     {
         classMasks[ c ] = GeomClassPresent( c, p0.rayCullMaskWorld ) ? GeomClassMask( c ) : 0u;
     }
+    uint32_t launches = 0; // of this call: one clear serves TRACE_COUNTER_SETS of them
     // rr's rays carry their cull masks in mm (null: every ray has mask);
     // frame k's rays start at offs[k].  A grouped launch gives each scene of
     // the group the rays of its frames (plain scenes: the masks admit every
@@ -2429,8 +2419,18 @@ uint64_t TraceFrames( const TraceSlot* slots, uint32_t B, const BvhObject& bvh, 
     auto trace = [ & ]( RgExtRay* rr, const uint8_t* mm, uint32_t mask, RgExtHit* hh, uint32_t flags, size_t count, const size_t* offs ) {
         if( haveGeometry )
         {
-            const uint32_t k  = lead.traceLaunches < PathTracer::TRACE_EVENT_PAIRS ? lead.traceLaunches : PathTracer::TRACE_EVENT_PAIRS - 1;
+            const uint32_t k  = lead.traceLaunches < PathTracer::FrameAccum::TIMED ? lead.traceLaunches : PathTracer::FrameAccum::TIMED - 1;
             const uint32_t fl = flags | traceFlags | ( lead.collectStats ? RG_EXT_TRACE_COLLECT_STATS : 0u );
+            accum.counterSet  = launches % TRACE_COUNTER_SETS;
+            accum.times       = fa->times[ k ];
+            accum.timeWords   = PathTracer::FrameAccum::TIME_WORDS;
+            accum.blocks      = &lead.traceBlocks[ k ];
+            lead.traceBlocks[ k ] = 0;
+            if( accum.counterSet == 0 )
+            {
+                ClearTraceCounters( tc, launches == 0 ? &accum : nullptr, s );
+            }
+            launches++;
             if( grouped )
             {
                 groupOffs.assign( bvh.sceneCount + 1, uint32_t( count ) );
@@ -2443,12 +2443,11 @@ uint64_t TraceFrames( const TraceSlot* slots, uint32_t B, const BvhObject& bvh, 
                     }
                     groupOffs[ g ] = f < B ? uint32_t( offs[ f ] ) : uint32_t( count );
                 }
-                TraceRaysBatch( bvh, tc, rr, groupOffs.data(), hh, fl, s, lead.traceEv[ 2 * k ], lead.traceEv[ 2 * k + 1 ], &accum );
+                TraceRaysBatch( bvh, tc, rr, groupOffs.data(), hh, fl, s, nullptr, nullptr, &accum );
             }
             else
             {
-                TraceRaysFrame( bvh, tc, rr, mm, mask, uint32_t( count ), hh, fl, classMasks, GC_COUNT, s, lead.traceEv[ 2 * k ],
-                                lead.traceEv[ 2 * k + 1 ], &accum, alpha, &tex );
+                TraceRaysFrame( bvh, tc, rr, mm, mask, uint32_t( count ), hh, fl, classMasks, GC_COUNT, s, &accum, alpha, &tex );
             }
             lead.traceLaunches = k + 1;
         }

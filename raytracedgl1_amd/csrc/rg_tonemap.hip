@@ -81,7 +81,8 @@ __global__ __launch_bounds__( HIST_BINS ) void k_lum_average( uint32_t* hist,
                                                               float     maxLog,
                                                               float     timeDelta,
                                                               uint32_t  stop,
-                                                              float*    avgLum )
+                                                              float*    avgLum,
+                                                              uint32_t* kept )
 {
     __shared__ uint32_t s[ HIST_BINS ];
     const uint32_t      i     = threadIdx.x;
@@ -89,6 +90,10 @@ __global__ __launch_bounds__( HIST_BINS ) void k_lum_average( uint32_t* hist,
     s[ i ]                    = count * i;
     __syncthreads();
     hist[ i ] = 0; // cleared for the next frame
+    if( kept )
+    {
+        kept[ i ] = count;
+    }
     for( uint32_t cutoff = HIST_BINS >> 1; cutoff > 0; cutoff >>= 1 )
     {
         if( i < cutoff )
@@ -319,9 +324,10 @@ void LuminanceHistogram( const float* d_lum, uint32_t count, float minLog, float
     CheckLaunch( "k_lum_histogram" );
 }
 
-void LuminanceAverage( uint32_t* d_hist, uint32_t pixelCount, float minLog, float maxLog, float timeDelta, bool stop, float* d_avg, hipStream_t stream )
+void LuminanceAverage( uint32_t* d_hist, uint32_t pixelCount, float minLog, float maxLog, float timeDelta, bool stop, float* d_avg, hipStream_t stream,
+                       uint32_t* d_kept )
 {
-    k_lum_average<<< 1, HIST_BINS, 0, stream >>>( d_hist, pixelCount, minLog, maxLog, timeDelta, stop ? 1u : 0u, d_avg );
+    k_lum_average<<< 1, HIST_BINS, 0, stream >>>( d_hist, pixelCount, minLog, maxLog, timeDelta, stop ? 1u : 0u, d_avg, d_kept );
     CheckLaunch( "k_lum_average" );
 }
 

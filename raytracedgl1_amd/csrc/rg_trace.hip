@@ -6,10 +6,11 @@
 // Execution model: a persistent grid of 256-thread blocks.  Each lane owns
 // one ray at a time; whenever lanes of a wave go idle they take the next rays
 // of the wave's current chunk, so long rays do not hold the wave's SIMD lanes
-// empty.  Chunks of 64 rays come from 32 counters 256 bytes apart (block b
-// takes chunks j * 32 + b % 32), one atomic per chunk: a refill atomic per
-// wave iteration on a single address serialises at the memory side and made
-// the kernel 5.5x slower at 1080p.
+// empty.  A wave's first chunk of 64 rays is the one of its own number; the
+// later ones come from 32 counters 256 bytes apart (block b takes chunks
+// waves + j * 32 + b % 32), one atomic per chunk: a refill atomic per wave
+// iteration on a single address serialises at the memory side and made the
+// kernel 5.5x slower at 1080p.
 //
 // k_trace walks the traversal's tree (BvhNodeQ): a node visit is eight
 // loads of one cache line, eight boxes of one multiply-add per plane, and a
@@ -50,6 +51,8 @@ constexpr uint32_t RAY_CHUNK_DEFAULT = 64; // rays per counter atomic
 constexpr uint32_t REFILL_MIN_LANES = 16;
 constexpr uint32_t RAY_PARTITIONS    = 32;  // ray counters
 constexpr uint32_t COUNTER_STRIDE    = 64;  // u32 between counters (256 B)
+constexpr uint32_t COUNTER_SET_WORDS = RAY_PARTITIONS * COUNTER_STRIDE;
+constexpr uint32_t TRACE_ERROR_WORD  = TRACE_COUNTER_SETS * COUNTER_SET_WORDS; // of TraceContext::counter
 
 struct TraceArgs
 {
@@ -66,6 +69,7 @@ struct TraceArgs
     uint32_t        stackTotal; // LDS + global stack entries per lane
     uint32_t*       errorFlag;
     uint64_t*       stats; // [0] node visits, [1] triangle tests (RG_EXT_TRACE_COLLECT_STATS)
+    uint32_t*       times; // ticks of block 0's start and of every block's end, or null
     // rays of several scenes of a batched BVH (segCount > 0): rays of scene s
     // are [segRays[s], segRays[s+1]), traversed from node s (k_trace) or
     // segRoots[s] (k_trace_view); hits report primitive ids relative to
@@ -265,6 +269,10 @@ __global__ __launch_bounds__( TR_THREADS, 4 ) void k_trace( TraceArgs a )
         }
         s_slots[ tid ] = slots;
     }
+    if( a.times && blockIdx.x == 0 && tid == 0 )
+    {
+        a.times[ 0 ] = uint32_t( wall_clock64() ); // block 0 is the first to start
+    }
     if( tid < 8 )
     {
         s_rootMask[ tid ] = a.rootMask[ tid ];
@@ -301,9 +309,15 @@ __global__ __launch_bounds__( TR_THREADS, 4 ) void k_trace( TraceArgs a )
     int      sp       = 0;
     uint32_t steps    = 0;
     uint32_t nodeVisits = 0, triTests = 0;
-    const uint32_t part = blockIdx.x % a.partitions; // chunks j * partitions + part
-    uint32_t chunkNext = 0, chunkEnd = 0; // this wave's rays [chunkNext, chunkEnd), wave-uniform
-    bool     drained   = false;           // the global counter has passed the last ray
+    const uint32_t part = blockIdx.x % a.partitions; // chunks waves + j * partitions + part
+    // This wave's rays [chunkNext, chunkEnd), wave-uniform: at first the chunk
+    // of its own number, later ones by the counters.  A launch that gives
+    // every wave one chunk touches no counter.
+    const uint32_t waves     = gridDim.x * ( TR_THREADS / 64 );
+    const uint32_t wave      = blockIdx.x * ( TR_THREADS / 64 ) + __builtin_amdgcn_readfirstlane( tid / 64 );
+    uint32_t       chunkNext = uint64_t( wave ) * a.chunk < a.count ? wave * a.chunk : a.count;
+    uint32_t       chunkEnd  = a.count - chunkNext > a.chunk ? chunkNext + a.chunk : a.count;
+    bool           drained   = uint64_t( waves ) * a.chunk >= a.count; // no chunk is left on the counters
 
     auto push = [ & ]( uint32_t b, uint32_t c, uint32_t l ) __attribute__( ( always_inline ) ) {
         const uint2 e = make_uint2( b | c << 28, l );
@@ -344,7 +358,7 @@ __global__ __launch_bounds__( TR_THREADS, 4 ) void k_trace( TraceArgs a )
                 if( lane == leader )
                 {
                     const uint32_t j = atomicAdd( a.rayCounter + part * COUNTER_STRIDE, 1u );
-                    const uint64_t g = uint64_t( j ) * a.partitions + part;
+                    const uint64_t g = uint64_t( j ) * a.partitions + part + waves;
                     b                = g * a.chunk < a.count ? uint32_t( g * a.chunk ) : a.count;
                 }
                 newBase = __builtin_amdgcn_readlane( b, leader );
@@ -631,6 +645,14 @@ __global__ __launch_bounds__( TR_THREADS, 4 ) void k_trace( TraceArgs a )
                 }
             }
         } while( __ballot( active ) != 0ull && __popcll( __ballot( !active && !exhausted ) ) < int( REFILL_MIN_LANES ) );
+    }
+    if( a.times )
+    {
+        __syncthreads();
+        if( tid == 0 )
+        {
+            a.times[ 1 + blockIdx.x ] = uint32_t( wall_clock64() );
+        }
     }
 }
 
@@ -1014,9 +1036,50 @@ uint32_t ReadTraceErrors( const TraceContext& s )
     if( s.counter.ptr )
     {
         RG_HIP_CHECK( hipDeviceSynchronize() );
-        RG_HIP_CHECK( hipMemcpy( &e, s.counter.as< uint32_t >() + RAY_PARTITIONS * COUNTER_STRIDE, sizeof( e ), hipMemcpyDeviceToHost ) );
+        RG_HIP_CHECK( hipMemcpy( &e, s.counter.as< uint32_t >() + TRACE_ERROR_WORD, sizeof( e ), hipMemcpyDeviceToHost ) );
     }
     return e;
+}
+
+namespace
+{
+// Clears `sets` sets of ray counters and, where given, an error word and the
+// two statistics words.  A kernel: a graph that captures it replays right,
+// and one launch takes the place of the two that a memset of 8 KB and 4
+// bytes became (9 us with the gaps, before every traversal).
+__global__ __launch_bounds__( RAY_PARTITIONS* TRACE_COUNTER_SETS ) void k_trace_clear( uint32_t* counters, uint32_t sets, uint32_t* error, uint64_t* stats )
+{
+    const uint32_t t = threadIdx.x;
+    if( t < sets * RAY_PARTITIONS )
+    {
+        counters[ t * COUNTER_STRIDE ] = 0u;
+    }
+    if( t == 0 && error )
+    {
+        *error = 0u;
+    }
+    if( t < 2 && stats )
+    {
+        stats[ t ] = 0ull;
+    }
+}
+
+void LaunchClear( uint32_t* counters, uint32_t sets, uint32_t* error, uint64_t* stats, hipStream_t stream )
+{
+    k_trace_clear<<< 1, RAY_PARTITIONS * TRACE_COUNTER_SETS, 0, stream >>>( counters, sets, error, stats );
+    CheckLaunch( "k_trace_clear" );
+}
+
+void ReserveCounters( TraceContext& s )
+{
+    s.counter.Reserve( ( TRACE_ERROR_WORD + 1 ) * sizeof( uint32_t ) );
+}
+} // namespace
+
+void ClearTraceCounters( TraceContext& s, const TraceAccum* accum, hipStream_t stream )
+{
+    ReserveCounters( s );
+    LaunchClear( s.counter.as< uint32_t >(), TRACE_COUNTER_SETS, accum ? accum->errors : nullptr, accum ? accum->stats : nullptr, stream );
 }
 
 namespace
@@ -1117,9 +1180,13 @@ void TraceRaysImpl( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
     const uint32_t grid   = s.grid[ view ? TRACE_STACK_VARIANTS : v ];
     const uint32_t lanes  = view ? 64u : LanesPerWave( count, grid );
     const uint32_t blocks = std::min( DivUp( count, lanes * ( TR_THREADS / 64 ) ), grid );
-    s.counter.Reserve( ( RAY_PARTITIONS * COUNTER_STRIDE + 1 ) * sizeof( uint32_t ) );
     s.stats.Reserve( 2 * sizeof( uint64_t ) );
-    RG_HIP_CHECK( hipMemsetAsync( s.counter.ptr, 0, ( RAY_PARTITIONS * COUNTER_STRIDE + 1 ) * sizeof( uint32_t ), stream ) );
+    const bool collect = ( flags & RG_EXT_TRACE_COLLECT_STATS ) != 0;
+    if( !accum )
+    {
+        ReserveCounters( s );
+        LaunchClear( s.counter.as< uint32_t >(), 1, s.counter.as< uint32_t >() + TRACE_ERROR_WORD, collect ? s.stats.as< uint64_t >() : nullptr, stream );
+    }
 
     TraceArgs a;
     a.nodes         = view ? bvh.nodes.ptr : bvh.nodesQ.ptr;
@@ -1128,13 +1195,14 @@ void TraceRaysImpl( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
     a.hits          = d_hits;
     a.count         = count;
     a.flags         = flags;
-    a.rayCounter    = s.counter.as< uint32_t >();
-    a.errorFlag     = s.counter.as< uint32_t >() + RAY_PARTITIONS * COUNTER_STRIDE;
+    a.rayCounter    = s.counter.as< uint32_t >() + ( accum ? accum->counterSet * COUNTER_SET_WORDS : 0u );
+    a.errorFlag     = s.counter.as< uint32_t >() + TRACE_ERROR_WORD;
     a.partitions    = blocks < RAY_PARTITIONS ? blocks : RAY_PARTITIONS;
     a.overflowStack = s.overflow.as< uint32_t >();
     a.ovfStride     = STACK_OVF_STRIDE;
     a.stackTotal    = STACK_TOTAL;
     a.stats         = nullptr;
+    a.times         = nullptr;
     a.segRays       = d_segRays;
     a.segRoots      = d_segRays ? bvh.sceneRoots8.as< uint32_t >() : nullptr;
     a.segTris       = d_segRays ? bvh.sceneOffsets.as< uint32_t >() : nullptr;
@@ -1172,13 +1240,19 @@ void TraceRaysImpl( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
     a.tex           = tex ? *tex : TexView{};
     if( accum )
     {
-        RG_REQUIRE( accum->errors, RG_RESULT_WRONG_FUNCTION_ARGUMENT, "accumulator without an error word" );
+        RG_REQUIRE( accum->errors && accum->counterSet < TRACE_COUNTER_SETS && s.counter.ptr, RG_RESULT_WRONG_FUNCTION_ARGUMENT,
+                    "accumulator without an error word or a cleared counter set" );
         a.errorFlag = accum->errors;
-        a.stats     = ( flags & RG_EXT_TRACE_COLLECT_STATS ) ? accum->stats : nullptr;
+        a.stats     = collect ? accum->stats : nullptr;
+        a.times     = accum->times;
+        if( accum->times )
+        {
+            RG_REQUIRE( accum->blocks && blocks < accum->timeWords, RG_RESULT_INTERNAL_ERROR, "more blocks than time words" );
+            *accum->blocks = blocks;
+        }
     }
-    else if( flags & RG_EXT_TRACE_COLLECT_STATS )
+    else if( collect )
     {
-        RG_HIP_CHECK( hipMemsetAsync( s.stats.ptr, 0, 2 * sizeof( uint64_t ), stream ) );
         a.stats = s.stats.as< uint64_t >();
     }
     if( evBefore )
@@ -1215,27 +1289,13 @@ namespace
 constexpr uint32_t NOALLOC_MAX_BLOCKS = 1024;
 constexpr uint32_t NOALLOC_OVF        = 40;
 constexpr int      NOALLOC_VARIANT    = 1; // the 24-entry LDS stack
-constexpr uint32_t NOALLOC_ERROR      = RAY_PARTITIONS * COUNTER_STRIDE; // u32 index of the error word
+constexpr uint32_t NOALLOC_ERROR      = COUNTER_SET_WORDS;               // u32 index of the error word
 constexpr uint32_t NOALLOC_STATS      = NOALLOC_ERROR + 2;               // u32 index of 2 x u64
 constexpr uint32_t NOALLOC_HEADER     = NOALLOC_ERROR + 64;              // u32 index of the overflow stacks
 constexpr size_t   NOALLOC_WORDS      = NOALLOC_HEADER + size_t( NOALLOC_MAX_BLOCKS ) * TR_THREADS * NOALLOC_OVF;
 static_assert( ( NOALLOC_STATS * 4 ) % 8 == 0, "statistics alignment" );
 static_assert( ( NOALLOC_HEADER * 4 ) % 256 == 0, "stack alignment" );
 static_assert( TRACE_STACK_DEPTH[ NOALLOC_VARIANT ] == 24, "no-alloc stack variant" );
-
-// Clears the counters, the error word and the statistics.
-__global__ __launch_bounds__( 64 ) void k_noalloc_clear( uint32_t* hdr )
-{
-    const uint32_t t = threadIdx.x;
-    if( t < RAY_PARTITIONS )
-    {
-        hdr[ t * COUNTER_STRIDE ] = 0u;
-    }
-    if( t < 6 )
-    {
-        hdr[ NOALLOC_ERROR + t ] = 0u; // error word, pad, 2 x u64 statistics
-    }
-}
 
 struct NoAllocDevice
 {
@@ -1291,8 +1351,7 @@ void TraceRaysNoAlloc( const BvhObject& bvh, const RgExtRay* d_rays, uint32_t co
     const uint32_t blocks = std::min( DivUp( count, lanes * ( TR_THREADS / 64 ) ), nd.grid[ view ? 1 : 0 ] );
     RG_REQUIRE( size_t( blocks ) * TR_THREADS * NOALLOC_OVF <= NOALLOC_WORDS - NOALLOC_HEADER, RG_RESULT_INTERNAL_ERROR,
                 "no-alloc traversal grid exceeds its scratch" );
-    k_noalloc_clear<<< 1, 64, 0, stream >>>( nd.scratch );
-    CheckLaunch( "k_noalloc_clear" );
+    LaunchClear( nd.scratch, 1, nd.scratch + NOALLOC_ERROR, reinterpret_cast< uint64_t* >( nd.scratch + NOALLOC_STATS ), stream );
 
     TraceArgs a{};
     a.nodes         = view ? bvh.nodes.ptr : bvh.nodesQ.ptr;
@@ -1347,8 +1406,8 @@ void ReadTraceNoAllocWords( uint32_t* errors, uint64_t* nodeVisits, uint64_t* tr
 }
 
 void TraceRaysFrame( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_rays, const uint8_t* d_rayMasks, uint32_t defaultMask, uint32_t count,
-                     RgExtHit* d_hits, uint32_t flags, const uint32_t* classMasks, uint32_t classCount, hipStream_t stream, hipEvent_t evBefore,
-                     hipEvent_t evAfter, const TraceAccum* accum, const AlphaRec* alpha, const TexView* tex )
+                     RgExtHit* d_hits, uint32_t flags, const uint32_t* classMasks, uint32_t classCount, hipStream_t stream, const TraceAccum* accum,
+                     const AlphaRec* alpha, const TexView* tex )
 {
     RG_REQUIRE( !bvh.frameSegs.empty(), RG_RESULT_WRONG_FUNCTION_CALL, "not a frame BVH" );
     FrameRoots fr;
@@ -1372,21 +1431,13 @@ void TraceRaysFrame( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ra
     if( fr.rootCount == 0 || count == 0 )
     {
         // nothing in the TLAS: every ray misses
-        if( evBefore )
-        {
-            RG_HIP_CHECK( hipEventRecord( evBefore, stream ) );
-        }
         if( count )
         {
             RG_HIP_CHECK( hipMemsetAsync( d_hits, 0xFF, size_t( count ) * sizeof( RgExtHit ), stream ) );
         }
-        if( evAfter )
-        {
-            RG_HIP_CHECK( hipEventRecord( evAfter, stream ) );
-        }
         return;
     }
-    TraceRaysImpl( bvh, s, d_rays, count, d_hits, flags, stream, evBefore, evAfter, accum, nullptr, &fr, alpha, tex );
+    TraceRaysImpl( bvh, s, d_rays, count, d_hits, flags, stream, nullptr, nullptr, accum, nullptr, &fr, alpha, tex );
 }
 
 void TraceRaysBatch( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_rays, const uint32_t* rayOffsets, RgExtHit* d_hits, uint32_t flags,
