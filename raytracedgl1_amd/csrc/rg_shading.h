@@ -90,6 +90,34 @@ __device__ __forceinline__ float fastSafePositiveRcp( float f )
     return f <= 0.0f ? 0.0f : fastRcp( f );
 }
 
+// Whole powers as products of doubles, rounded to FP32 once: within half a
+// unit in the last place (powf is allowed one), in a handful of multiplies
+// where powf is some hundred and forty instructions: k_initial_a 300 -> 216 us
+// at 1920x1080 with 32 candidates a pixel.
+__device__ __forceinline__ float pow5( float x )
+{
+    const double d = x, d2 = d * d;
+    return float( d2 * d2 * d );
+}
+// x^e, e the same in every lane.  Whole e up to 64 by squaring (the products
+// stay inside the range of a double for every FP32 x in [0, 2] that has a
+// power in FP32, and underflow to the 0 that powf returns); others powf.
+__device__ __forceinline__ float powUniform( float x, float e )
+{
+    uint32_t n = uint32_t( __builtin_amdgcn_readfirstlane( int( e ) ) );
+    if( n > 64u || e != float( n ) )
+    {
+        return powf( x, e );
+    }
+    double r = 1.0, b = x;
+    for( ; n != 0u; n >>= 1 )
+    {
+        r = n & 1u ? r * b : r;
+        b = b * b;
+    }
+    return float( r );
+}
+
 // ----------------------------------------------------------- sampling
 
 // Random.h:36-51
@@ -201,7 +229,7 @@ __device__ __forceinline__ v3 evalBRDFSmithGGX( v3 n, v3 v, v3 l, float alpha, v
     {
         return mk3( 0, 0, 0 );
     }
-    const float f  = powf( 1.0f - fmaxf( nl, 0.0f ), 5.0f );
+    const float f  = pow5( 1.0f - fmaxf( nl, 0.0f ) );
     const v3    F  = specColor + ( mk3( 1, 1, 1 ) - specColor ) * f;
     const v3    h  = fastNormalize( v + l );
     const float D  = D_GGX( dot( n, h ), alpha, loose );
@@ -341,7 +369,7 @@ __device__ LightSample sampleLight( const LightEncoded& e, v3 surfPos, const Lig
             const float dist = fastLength( tl );
             tl               = tl * fastRcp( dist );
             const float ll   = fmaxf( dot( nrm, tl ), 0.0f );
-            r.color          = L3( e.color ) * powf( ll, polyFactor );
+            r.color          = L3( e.color ) * powUniform( ll, polyFactor );
             r.dw             = safeSolidAngle( area * ( fabsf( dot( nrm, tl ) ) * fastRcp( square( dist ) ) ) );
             return r;
         }

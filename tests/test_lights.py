@@ -100,3 +100,33 @@ def test_gradients_still_scene_and_removed_light_gpu():
                 assert np.abs(g[..., 2] - 0.5 * p.gradientMultSpecular).max() < 1e-3
     finally:
         r.close()
+
+
+@pytest.mark.parametrize("e", [1.0, 2.0, 5.0, 64.0])
+def test_triangle_light_powers_on_both_routes(e):
+    """The triangle light's cos^e at a whole exponent (products) and at the
+    next float above it (powf): the direct light may differ by cos^ulp(e)
+    and by the roundings of the two routes (64 units in the last place)."""
+    import numpy as np
+    print(f"lights: triangle light, exponent {e} and the next float", flush=True)
+    got = []
+    for factor in (np.float32(e), np.nextafter(np.float32(e), np.float32(100.0))):
+        r = rtgl.Renderer(W, H)
+        try:
+            r.path.restirTemporalSamples = 0
+            r.path.restirSpatialSamples = 0
+            r.set_illumination(cellWorldSize=1.0, polygonalLightSpotlightFactor=float(factor))
+            r.frame(rtgl.SceneUploader(lc.plane_scene({"polys": [lc.TRIANGLE]})), lc.CAM)
+            assert np.float32(r.frame_params().polyLightSpotlightFactor) == factor
+            fb = r.framebuffers()
+            got.append((fb.download(P["UNFILTERED_DIRECT"]), fb.download(P["SURFACE_POSITION"]), fb.download(P["IS_SKY"])))
+        finally:
+            r.close()
+    (a, pos, sky), (b, _, _) = got
+    to = lc.TRI_C - pos[..., :3].astype(np.float64)
+    cos = to[..., 1] / np.linalg.norm(to, axis=-1)
+    ok = (sky.reshape(cos.shape) == 0) & (cos > 0.3)
+    a, b = a[ok][:, :3].astype(np.float64), b[ok][:, :3].astype(np.float64)
+    assert ok.sum() > 1000 and (a > 0.0).any()
+    rtol = float(np.spacing(np.float32(e))) * -np.log(0.25) + 64 * 2.0 ** -24
+    assert np.abs(a - b).max() <= rtol * a.max() and (np.abs(a - b) <= rtol * a + 1e-30).all()

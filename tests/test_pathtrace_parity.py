@@ -202,6 +202,25 @@ def test_frames_match_the_fp64_oracle(oracle):
     assert oc[P["DIS_GRADIENT_HISTORY"]][..., 0].max() > 0.1
 
 
+@pytest.mark.parametrize("size", [(34, 9), (94, 41), (66, 70)])
+def test_bounce_light_at_ragged_tiles(oracle, monkeypatch, size):
+    """Bounce hits are packed to the front of each 32x8 tile: frames whose
+    last tile column and row are cut keep the 160x90 frames' smooth-normal
+    bounds on the planes that the bounce feeds; a bound on a share of the
+    pixels is widened by two pixels' share, its step at these sizes."""
+    monkeypatch.setitem(globals(), "W", size[0])
+    monkeypatch.setitem(globals(), "H", size[1])
+    print(f"parity: bounce light at {size[0]}x{size[1]}", flush=True)
+    s = _scene_with_spheres()
+    flags = {i: DONT_GENERATE_NORMALS for i in range(len(s.objects))}
+    for f, g, oc, m in _parity_frames(oracle, flags=flags):
+        hits = int((oc[P["IS_SKY"]][..., 0] == 0).sum())
+        assert hits > 0 and m["IS_SKY"] == 1.0 and m["VISIBILITY_BUFFER"] == 1.0, f
+        assert np.isfinite(g["UNFILTERED_INDIR"]).all(), f
+        assert m["RESERVOIRS_INITIAL"] >= 0.999 - 2.0 / hits, f
+        assert m["UNFILTERED_INDIR all"] >= 0.97 - 2.0 / hits, (f, m["UNFILTERED_INDIR all"])
+
+
 def test_spot_and_triangle_lights_match_the_fp64_oracle(oracle):
     """The plain frames with three spot and three triangle lights beside the
     sun and the eight spheres (Light.h:225-297 on both sides).  Same
