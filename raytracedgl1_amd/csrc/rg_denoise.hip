@@ -31,37 +31,32 @@ struct Dims
     int W, H, GW, GH;
 };
 
+// A texel, zero outside the image, without a branch: outside, texel 0 is
+// fetched and dropped.  A branch around each fetch makes a wave wait for the
+// data of one before it asks for the next (k_temporal at 1920x1080 with half
+// storage: 100 us with branches, 83 without).
+template< typename T >
+__device__ __forceinline__ T LdTexel( const void* base, int w, int h, int x, int y, T zero )
+{
+    const bool in = uint32_t( x ) < uint32_t( w ) && uint32_t( y ) < uint32_t( h );
+    const T    v  = reinterpret_cast< const T* >( base )[ in ? size_t( y ) * w + x : size_t( 0 ) ];
+    return in ? v : zero;
+}
 __device__ __forceinline__ float4 Ld4( const void* base, int w, int h, int x, int y )
 {
-    if( x < 0 || y < 0 || x >= w || y >= h )
-    {
-        return make_float4( 0.f, 0.f, 0.f, 0.f );
-    }
-    return reinterpret_cast< const float4* >( base )[ size_t( y ) * w + x ];
+    return LdTexel( base, w, h, x, y, make_float4( 0.f, 0.f, 0.f, 0.f ) );
 }
 __device__ __forceinline__ float2 Ld2( const void* base, int w, int h, int x, int y )
 {
-    if( x < 0 || y < 0 || x >= w || y >= h )
-    {
-        return make_float2( 0.f, 0.f );
-    }
-    return reinterpret_cast< const float2* >( base )[ size_t( y ) * w + x ];
+    return LdTexel( base, w, h, x, y, make_float2( 0.f, 0.f ) );
 }
 __device__ __forceinline__ float Ld1( const void* base, int w, int h, int x, int y )
 {
-    if( x < 0 || y < 0 || x >= w || y >= h )
-    {
-        return 0.f;
-    }
-    return reinterpret_cast< const float* >( base )[ size_t( y ) * w + x ];
+    return LdTexel( base, w, h, x, y, 0.f );
 }
 __device__ __forceinline__ uint32_t LdU( const void* base, int w, int h, int x, int y )
 {
-    if( x < 0 || y < 0 || x >= w || y >= h )
-    {
-        return 0u;
-    }
-    return reinterpret_cast< const uint32_t* >( base )[ size_t( y ) * w + x ];
+    return LdTexel( base, w, h, x, y, 0u );
 }
 __device__ __forceinline__ void St4( void* base, int w, int x, int y, float4 v )
 {
@@ -94,11 +89,7 @@ __device__ __forceinline__ float4 LdP4( const void* base, int w, int h, int x, i
     }
     else
     {
-        if( x < 0 || y < 0 || x >= w || y >= h )
-        {
-            return make_float4( 0.f, 0.f, 0.f, 0.f );
-        }
-        const half4v v = reinterpret_cast< const half4v* >( base )[ size_t( y ) * w + x ];
+        const half4v v = LdTexel( base, w, h, x, y, half4v{} );
         return make_float4( float( v.x ), float( v.y ), float( v.z ), float( v.w ) );
     }
 }
@@ -111,11 +102,7 @@ __device__ __forceinline__ float2 LdP2( const void* base, int w, int h, int x, i
     }
     else
     {
-        if( x < 0 || y < 0 || x >= w || y >= h )
-        {
-            return make_float2( 0.f, 0.f );
-        }
-        const half2v v = reinterpret_cast< const half2v* >( base )[ size_t( y ) * w + x ];
+        const half2v v = LdTexel( base, w, h, x, y, half2v{} );
         return make_float2( float( v.x ), float( v.y ) );
     }
 }
@@ -128,11 +115,7 @@ __device__ __forceinline__ float LdP1( const void* base, int w, int h, int x, in
     }
     else
     {
-        if( x < 0 || y < 0 || x >= w || y >= h )
-        {
-            return 0.f;
-        }
-        return float( reinterpret_cast< const _Float16* >( base )[ size_t( y ) * w + x ] );
+        return float( LdTexel( base, w, h, x, y, _Float16( 0 ) ) );
     }
 }
 template< bool F16 >
@@ -199,13 +182,8 @@ __device__ __forceinline__ v3 DecodeNormal( uint32_t p )
 // the values of a zero fetch of both (decoded normal code 0, depth 0).
 __device__ __forceinline__ void LdGuide( const FbPtrs& P, int w, int h, int x, int y, v3& n, float& depth )
 {
-    if( x < 0 || y < 0 || x >= w || y >= h )
-    {
-        n     = DecodeNormal( 0u );
-        depth = 0.0f;
-        return;
-    }
-    const float4 g = reinterpret_cast< const float4* >( P.cur[ RG_EXT_PLANE_DENOISE_GUIDE ] )[ size_t( y ) * w + x ];
+    // sin and cos of 0: code 0 is exactly +z
+    const float4 g = LdTexel( P.cur[ RG_EXT_PLANE_DENOISE_GUIDE ], w, h, x, y, make_float4( 0.f, 0.f, 1.f, 0.f ) );
     n              = mk3( g.x, g.y, g.z );
     depth          = g.w;
 }
@@ -364,6 +342,27 @@ __global__ __launch_bounds__( THREADS ) void k_grad_atrous( FbPtrs P, Dims d, in
 
 // ---------------------------------------------------------- temporal
 
+// Which of the 2x2 previous-frame texels from (x0, y0) belong to the surface
+// of this pixel: in its half of the checkerboard, at its depth and normal.
+__device__ __forceinline__ void TestTaps( const FbPtrs& P, int W, int H, int x0, int y0, int alo, int ahi, float depth, float zMotion, v3 normal,
+                                          bool ( &pass )[ 2 ][ 2 ] )
+{
+    float    dPrev[ 2 ][ 2 ];
+    uint32_t code[ 2 ][ 2 ];
+#pragma unroll
+    for( int k = 0; k < 4; k++ )
+    {
+        dPrev[ k / 2 ][ k % 2 ] = Ld1( P.prev[ RG_EXT_PLANE_DEPTH_WORLD ], W, H, x0 + k % 2, y0 + k / 2 );
+        code[ k / 2 ][ k % 2 ]  = LdU( P.prev[ RG_EXT_PLANE_NORMAL ], W, H, x0 + k % 2, y0 + k / 2 );
+    }
+#pragma unroll
+    for( int k = 0; k < 4; k++ )
+    {
+        pass[ k / 2 ][ k % 2 ] = inRenderArea( x0 + k % 2, y0 + k / 2, alo, ahi, H ) & TestDepth( depth, dPrev[ k / 2 ][ k % 2 ], zMotion ) &
+                                 TestNormal( normal, DecodeNormal( code[ k / 2 ][ k % 2 ] ) );
+    }
+}
+
 template< bool F16 >
 __global__ __launch_bounds__( THREADS ) void k_temporal( FbPtrs P, Dims d, RgExtFrameParams g )
 {
@@ -397,29 +396,42 @@ __global__ __launch_bounds__( THREADS ) void k_temporal( FbPtrs P, Dims d, RgExt
     v3     diffPrev  = mk3( 0, 0, 0 ), specPrev = mk3( 0, 0, 0 ), indirPrev = mk3( 0, 0, 0 );
     float2 momPrev   = make_float2( 0.f, 0.f );
     float  weightSum = 0.0f;
+    // The four taps' tests are fetched together, then each row's data (of a
+    // tap that fails its tests, the pixel's own, which is dropped).
+    bool pass[ 2 ][ 2 ];
+    TestTaps( P, W, H, ppx, ppy, alo, ahi, depth, motion.z, normal, pass );
 #pragma unroll
     for( int yy = 0; yy <= 1; yy++ )
     {
+        float2 mp[ 2 ];
+        float4 hp[ 2 ];
+        v3     dp[ 2 ], sp[ 2 ], ip[ 2 ];
 #pragma unroll
         for( int xx = 0; xx <= 1; xx++ )
         {
-            const int   qx = ppx + xx, qy = ppy + yy;
-            const float dPrev = Ld1( P.prev[ RG_EXT_PLANE_DEPTH_WORLD ], W, H, qx, qy );
-            const v3    nPrev = DecodeNormal( LdU( P.prev[ RG_EXT_PLANE_NORMAL ], W, H, qx, qy ) );
-            if( inRenderArea( qx, qy, alo, ahi, H ) && TestDepth( depth, dPrev, motion.z ) && TestNormal( normal, nPrev ) )
+            const bool ok = pass[ yy ][ xx ];
+            const int  qx = ok ? ppx + xx : x, qy = ok ? ppy + yy : y;
+            mp[ xx ]      = LdP2< F16 >( P.prev[ RG_EXT_PLANE_DIFF_ACCUM_MOMENTS ], W, H, qx, qy );
+            hp[ xx ]      = LdP4< F16 >( P.prev[ RG_EXT_PLANE_ACCUM_HISTORY_LENGTH ], W, H, qx, qy );
+            dp[ xx ]      = xyz( LdP4< F16 >( P.cur[ RG_EXT_PLANE_DIFF_COLOR_HISTORY ], W, H, qx, qy ) );
+            sp[ xx ]      = xyz( LdP4< F16 >( P.prev[ RG_EXT_PLANE_SPEC_ACCUM_COLOR ], W, H, qx, qy ) );
+            ip[ xx ]      = xyz( LdP4< F16 >( P.prev[ RG_EXT_PLANE_INDIR_ACCUM ], W, H, qx, qy ) );
+        }
+#pragma unroll
+        for( int xx = 0; xx <= 1; xx++ )
+        {
+            if( pass[ yy ][ xx ] )
             {
-                const float  w  = bw[ yy ][ xx ];
-                const float2 mp = LdP2< F16 >( P.prev[ RG_EXT_PLANE_DIFF_ACCUM_MOMENTS ], W, H, qx, qy );
-                const float4 hp = LdP4< F16 >( P.prev[ RG_EXT_PLANE_ACCUM_HISTORY_LENGTH ], W, H, qx, qy );
-                diffPrev        = diffPrev + xyz( LdP4< F16 >( P.cur[ RG_EXT_PLANE_DIFF_COLOR_HISTORY ], W, H, qx, qy ) ) * w;
-                momPrev.x += w * mp.x;
-                momPrev.y += w * mp.y;
-                hist.x += w * hp.x;
-                hist.y += w * hp.y;
-                hist.z += w * hp.z;
-                hist.w += w * hp.w;
-                specPrev  = specPrev + xyz( LdP4< F16 >( P.prev[ RG_EXT_PLANE_SPEC_ACCUM_COLOR ], W, H, qx, qy ) ) * w;
-                indirPrev = indirPrev + xyz( LdP4< F16 >( P.prev[ RG_EXT_PLANE_INDIR_ACCUM ], W, H, qx, qy ) ) * w;
+                const float w = bw[ yy ][ xx ];
+                diffPrev      = diffPrev + dp[ xx ] * w;
+                momPrev.x += w * mp[ xx ].x;
+                momPrev.y += w * mp[ xx ].y;
+                hist.x += w * hp[ xx ].x;
+                hist.y += w * hp[ xx ].y;
+                hist.z += w * hp[ xx ].z;
+                hist.w += w * hp[ xx ].w;
+                specPrev  = specPrev + sp[ xx ] * w;
+                indirPrev = indirPrev + ip[ xx ] * w;
                 weightSum += w;
             }
         }
@@ -464,22 +476,14 @@ __global__ __launch_bounds__( THREADS ) void k_temporal( FbPtrs P, Dims d, RgExt
         const float tx = ( qpx - 0.5f ) - floorf( qpx - 0.5f ), ty = ( qpy - 0.5f ) - floorf( qpy - 0.5f );
         const float bws[ 2 ][ 2 ] = { { ( 1.0f - tx ) * ( 1.0f - ty ), tx * ( 1.0f - ty ) }, { ( 1.0f - tx ) * ty, tx * ty } };
         float       wsv = 0.0f;
+        // the reference accumulates the virtual-motion sample but blends
+        // specPrevOnSurf (CmSVGFTemporalAccumulation.comp:262-275)
+        bool passV[ 2 ][ 2 ];
+        TestTaps( P, W, H, vpx, vpy, alo, ahi, depth, motion.z, normal, passV );
 #pragma unroll
-        for( int yy = 0; yy <= 1; yy++ )
+        for( int k = 0; k < 4; k++ )
         {
-#pragma unroll
-            for( int xx = 0; xx <= 1; xx++ )
-            {
-                const int   qx = vpx + xx, qy = vpy + yy;
-                const float dPrev = Ld1( P.prev[ RG_EXT_PLANE_DEPTH_WORLD ], W, H, qx, qy );
-                const v3    nPrev = DecodeNormal( LdU( P.prev[ RG_EXT_PLANE_NORMAL ], W, H, qx, qy ) );
-                if( inRenderArea( qx, qy, alo, ahi, H ) && TestDepth( depth, dPrev, motion.z ) && TestNormal( normal, nPrev ) )
-                {
-                    // the reference accumulates the virtual-motion sample but
-                    // blends specPrevOnSurf (CmSVGFTemporalAccumulation.comp:262-275)
-                    wsv += bws[ yy ][ xx ];
-                }
-            }
+            wsv += passV[ k / 2 ][ k % 2 ] ? bws[ k / 2 ][ k % 2 ] : 0.0f;
         }
         if( wsv > 0.0001f )
         {
@@ -801,42 +805,40 @@ __device__ void AtrousPixel( const FbPtrs& P, const Dims& d, int x, int y, int k
     // 1 / max(grad * (|dx| + |dy|), 0.01) of the edge and diagonal taps
     const float zInv1 = 1.0f / fmaxf( c_grad, 0.01f ), zInv2 = 1.0f / fmaxf( c_grad * 2.0f, 0.01f );
     float ws = 1.0f, wss = 1.0f, wsi = 1.0f;
-#pragma unroll 1
+    auto add = [ & ]( int xx, int yy, v3 nq, float dq, float rq, float4 cq, v3 sq, v3 iq ) __attribute__( ( always_inline ) ) {
+        const float lq  = luminance( xyz( cq ) );
+        const float nn  = fmaxf( 0.0f, dot( c_n, nq ) );
+        const float w_z = fabsf( c_depth - dq ) * ( xx != 0 && yy != 0 ? zInv2 : zInv1 );
+        const float w_n = Pow128( nn );
+        const float w_l = fabsf( l - lq ) * wLum;
+        float       w_r = fmaxf( 0.0f, 1.0f - 10.0f * fabsf( c_rough - rq ) ) * wRough;
+        w_r             = nws > 0.0f ? w_r * FastPow( nn, nws ) : w_r;
+        const float kw     = ( xx == 0 ? 1.0f : 0.5f ) * ( yy == 0 ? 1.0f : 0.5f );
+        const float inside = inRenderArea( x + xx * step, y + yy * step, alo, ahi, H ) ? 1.0f : 0.0f;
+        const float wBase  = FastExp( -w_z * w_z ) * w_n * kw * inside;
+        const float wD = wBase * FastExp( -w_l ), wS = wBase * w_r, wI = wBase;
+        outD = outD + xyz( cq ) * wD;
+        outS = outS + sq * wS;
+        outI = outI + iq * wI;
+        outV += cq.w * wD * wD;
+        ws += wD;
+        wss += wS;
+        wsi += wI;
+    };
+#pragma unroll
     for( int yy = -1; yy <= 1; yy++ )
     {
 #pragma unroll
         for( int xx = -1; xx <= 1; xx++ )
         {
-            if( xx == 0 && yy == 0 )
+            if( xx != 0 || yy != 0 )
             {
-                continue;
+                v3     nq, sq, iq;
+                float4 cq;
+                float  dq, rq;
+                tap( xx, yy, nq, dq, rq, cq, sq, iq );
+                add( xx, yy, nq, dq, rq, cq, sq, iq );
             }
-            const int qx = x + xx * step, qy = y + yy * step;
-            v3        nq, sq, iq;
-            float4    cq;
-            float     dq, rq;
-            tap( xx, yy, qx, qy, nq, dq, rq, cq, sq, iq );
-            const float lq  = luminance( xyz( cq ) );
-            const float nn  = fmaxf( 0.0f, dot( c_n, nq ) );
-            const float w_z = fabsf( c_depth - dq ) * ( xx != 0 && yy != 0 ? zInv2 : zInv1 );
-            const float w_n = Pow128( nn );
-            const float w_l = fabsf( l - lq ) * wLum;
-            float       w_r = fmaxf( 0.0f, 1.0f - 10.0f * fabsf( c_rough - rq ) ) * wRough;
-            if( nws > 0.0f )
-            {
-                w_r *= FastPow( nn, nws );
-            }
-            const float kw     = ( xx == 0 ? 1.0f : 0.5f ) * ( yy == 0 ? 1.0f : 0.5f );
-            const float inside = inRenderArea( qx, qy, alo, ahi, H ) ? 1.0f : 0.0f;
-            const float wBase  = FastExp( -w_z * w_z ) * w_n * kw * inside;
-            const float wD = wBase * FastExp( -w_l ), wS = wBase * w_r, wI = wBase;
-            outD = outD + xyz( cq ) * wD;
-            outS = outS + sq * wS;
-            outI = outI + iq * wI;
-            outV += cq.w * wD * wD;
-            ws += wD;
-            wss += wS;
-            wsi += wI;
         }
     }
     const float iw = 1.0f / ws;
@@ -856,98 +858,66 @@ __device__ void AtrousPixel( const FbPtrs& P, const Dims& d, int x, int y, int k
     }
 }
 
-// Iteration 0: the 3x3 footprint (plus the 3x3 Gaussian of the variance) is
-// staged in LDS (CmSVGFAtrous_Iter0.comp:96-163).
-template< bool F16 >
-__global__ __launch_bounds__( THREADS ) void k_atrous0( FbPtrs P, Dims d, AtrousPlanes ap )
+// Iteration k (step 2^k).  A workgroup takes TBX columns of every step-th
+// row, THREADS / TBX of them, so that one staged row is a tap row of up to
+// three of them: texels are fetched into LDS once (with a halo of step columns
+// and one lattice row) and read there eight times.  Gathered from memory, the
+// taps of steps 2 to 16 were bound by the L1, which passed every texel nine
+// times: 122 us an iteration over 1920x1080 dense pixels, 85 staged (58 and 36
+// with half storage).  64 columns: fewer make more halo, and 128 leave two
+// rows to share the halo rows.
+// FIRST: iteration 0 also filters the variance (a 3x3 Gaussian over its own
+// footprint) and keeps its root (CmSVGFAtrous_Iter0.comp:96-163).
+constexpr int ATROUS_TEXEL = 16 + 3 * 12 + 2 * 4; // bytes staged per texel
+
+template< bool F16, int TBX, bool FIRST >
+__global__ __launch_bounds__( THREADS ) void k_atrous( FbPtrs P, Dims d, AtrousPlanes ap, int k )
 {
-    constexpr int R = 1, TW = BX + 2 * R, TH = BY + 2 * R;
-    __shared__ float4 s_diff[ TH ][ TW ];
-    __shared__ v3     s_spec[ TH ][ TW ];
-    __shared__ v3     s_ind[ TH ][ TW ];
-    __shared__ v3     s_nrm[ TH ][ TW ];
-    __shared__ float  s_dep[ TH ][ TW ];
-    __shared__ float  s_rgh[ TH ][ TW ];
-    const int         W = d.W, H = d.H;
-    const int         bx0 = blockIdx.x * BX - R, by0 = blockIdx.y * BY - R;
-    for( int i = threadIdx.x; i < TW * TH; i += THREADS )
+    extern __shared__ float4 s_texels[];
+    constexpr int            ROWS = THREADS / TBX;
+    const int                W = d.W, H = d.H;
+    const int                step = 1 << k, TW = TBX + 2 * step, count = TW * ( ROWS + 2 );
+    float4* const            s_diff = s_texels;
+    v3* const                s_spec = reinterpret_cast< v3* >( s_diff + count );
+    v3* const                s_ind  = s_spec + count;
+    v3* const                s_nrm  = s_ind + count;
+    float* const             s_dep  = reinterpret_cast< float* >( s_nrm + count );
+    float* const             s_rgh  = s_dep + count;
+    const int lx = threadIdx.x % TBX, ly = threadIdx.x / TBX;
+    const int x0 = blockIdx.x * TBX, y0 = ( int( blockIdx.y >> k ) * ROWS << k ) + int( blockIdx.y & uint32_t( step - 1 ) );
+    for( int ty = ly; ty < ROWS + 2; ty += ROWS )
     {
-        const int tx = i % TW, ty = i / TW, gx = bx0 + tx, gy = by0 + ty;
-        s_diff[ ty ][ tx ] = LdP4< F16 >( P.cur[ ap.srcD ], W, H, gx, gy );
-        s_spec[ ty ][ tx ] = xyz( LdP4< F16 >( P.cur[ ap.srcS ], W, H, gx, gy ) );
-        s_ind[ ty ][ tx ]  = xyz( LdP4< F16 >( P.cur[ ap.srcI ], W, H, gx, gy ) );
-        LdGuide( P, W, H, gx, gy, s_nrm[ ty ][ tx ], s_dep[ ty ][ tx ] );
-        s_rgh[ ty ][ tx ]  = Ld2( P.cur[ RG_EXT_PLANE_METALLIC_ROUGHNESS ], W, H, gx, gy ).y;
+        const int gy = y0 + ( ty - 1 ) * step;
+        for( int tx = lx; tx < TW; tx += TBX )
+        {
+            const int gx = x0 + tx - step, i = ty * TW + tx;
+            s_diff[ i ] = LdP4< F16 >( P.cur[ ap.srcD ], W, H, gx, gy );
+            s_spec[ i ] = xyz( LdP4< F16 >( P.cur[ ap.srcS ], W, H, gx, gy ) );
+            s_ind[ i ]  = xyz( LdP4< F16 >( P.cur[ ap.srcI ], W, H, gx, gy ) );
+            LdGuide( P, W, H, gx, gy, s_nrm[ i ], s_dep[ i ] );
+            s_rgh[ i ] = Ld2( P.cur[ RG_EXT_PLANE_METALLIC_ROUGHNESS ], W, H, gx, gy ).y;
+        }
     }
     __syncthreads();
-    const int lx = threadIdx.x % BX + R, ly = threadIdx.x / BX + R;
-    const int x = lx - R + blockIdx.x * BX, y = ly - R + blockIdx.y * BY;
+    const int x = x0 + lx, y = y0 + ly * step;
     if( x >= W || y >= H )
     {
         return;
     }
-    const float depth = s_dep[ ly ][ lx ];
+    const int    c     = ( ly + 1 ) * TW + lx + step; // the pixel's own texel
+    const float4 cd    = s_diff[ c ];
+    const v3     cs    = s_spec[ c ], ci = s_ind[ c ];
+    const float  depth = s_dep[ c ];
     if( depth < 0.0f || depth > MAX_RAY_LENGTH )
     {
-        const float4 z = make_float4( 0.f, 0.f, 0.f, 0.f );
-        if( ap.dstD >= 0 )
+        if( FIRST )
         {
+            const float4 z = make_float4( 0.f, 0.f, 0.f, 0.f );
             StP4< F16 >( P.cur[ ap.dstD ], W, x, y, z );
             StP4< F16 >( P.cur[ ap.dstS ], W, x, y, z );
             StP4< F16 >( P.cur[ ap.dstI ], W, x, y, z );
         }
-        else
-        {
-            Compose( P, d, x, y, mk3( 0, 0, 0 ), mk3( 0, 0, 0 ), mk3( 0, 0, 0 ) );
-        }
-        return;
-    }
-    float r = 0.0f;
-#pragma unroll
-    for( int yy = -1; yy <= 1; yy++ )
-    {
-#pragma unroll
-        for( int xx = -1; xx <= 1; xx++ )
-        {
-            r += s_diff[ ly + yy ][ lx + xx ].w * ( ( xx == 0 ? 0.5f : 0.25f ) * ( yy == 0 ? 0.5f : 0.25f ) );
-        }
-    }
-    const float pvar = sqrtf( fmaxf( r, 0.0f ) );
-    StP1< F16 >( P.cur[ RG_EXT_PLANE_ATROUS_FILTERED_VARIANCE ], W, x, y, pvar );
-    AtrousPixel< F16 >( P, d, x, y, 0, 1, ap, s_nrm[ ly ][ lx ], depth, Ld1( P.cur[ RG_EXT_PLANE_DEPTH_GRAD ], W, H, x, y ),
-                 s_rgh[ ly ][ lx ], s_diff[ ly ][ lx ], s_spec[ ly ][ lx ], s_ind[ ly ][ lx ], pvar,
-                 [ & ]( int xx, int yy, int, int, v3& nq, float& dq, float& rq, float4& cq, v3& sq, v3& iq ) {
-                     nq = s_nrm[ ly + yy ][ lx + xx ];
-                     dq = s_dep[ ly + yy ][ lx + xx ];
-                     rq = s_rgh[ ly + yy ][ lx + xx ];
-                     cq = s_diff[ ly + yy ][ lx + xx ];
-                     sq = s_spec[ ly + yy ][ lx + xx ];
-                     iq = s_ind[ ly + yy ][ lx + xx ];
-                 } );
-}
-
-// Iterations >= 1 (steps 2, 4, 8, 16): taps gathered from global memory.
-// Each pixel is computed on its own, so the workgroup tile (TBX x
-// THREADS / TBX pixels) changes only which tap rows share a cache.
-template< bool F16, int TBX >
-__global__ __launch_bounds__( THREADS ) void k_atrousN( FbPtrs P, Dims d, AtrousPlanes ap, int k )
-{
-    const int x = blockIdx.x * TBX + threadIdx.x % TBX;
-    const int y = blockIdx.y * ( THREADS / TBX ) + threadIdx.x / TBX;
-    const int W = d.W, H = d.H;
-    if( x >= W || y >= H )
-    {
-        return;
-    }
-    const float4 cd    = LdP4< F16 >( P.cur[ ap.srcD ], W, H, x, y );
-    const v3     cs    = xyz( LdP4< F16 >( P.cur[ ap.srcS ], W, H, x, y ) );
-    const v3     ci    = xyz( LdP4< F16 >( P.cur[ ap.srcI ], W, H, x, y ) );
-    v3           n;
-    float        depth;
-    LdGuide( P, W, H, x, y, n, depth );
-    if( depth < 0.0f || depth > MAX_RAY_LENGTH )
-    {
-        if( ap.dstD >= 0 )
+        else if( ap.dstD >= 0 )
         {
             StP4< F16 >( P.cur[ ap.dstD ], W, x, y, cd );
             StP4< F16 >( P.cur[ ap.dstS ], W, x, y, f4( cs, 0.0f ) );
@@ -959,15 +929,35 @@ __global__ __launch_bounds__( THREADS ) void k_atrousN( FbPtrs P, Dims d, Atrous
         }
         return;
     }
-    const float rough = Ld2( P.cur[ RG_EXT_PLANE_METALLIC_ROUGHNESS ], W, H, x, y ).y;
-    const float pvar  = LdP1< F16 >( P.cur[ RG_EXT_PLANE_ATROUS_FILTERED_VARIANCE ], W, H, x, y );
-    AtrousPixel< F16 >( P, d, x, y, k, 1 << k, ap, n, depth, Ld1( P.cur[ RG_EXT_PLANE_DEPTH_GRAD ], W, H, x, y ), rough, cd, cs, ci, pvar,
-                 [ & ]( int, int, int qx, int qy, v3& nq, float& dq, float& rq, float4& cq, v3& sq, v3& iq ) {
-                     LdGuide( P, W, H, qx, qy, nq, dq );
-                     rq = Ld2( P.cur[ RG_EXT_PLANE_METALLIC_ROUGHNESS ], W, H, qx, qy ).y;
-                     cq = LdP4< F16 >( P.cur[ ap.srcD ], W, H, qx, qy );
-                     sq = xyz( LdP4< F16 >( P.cur[ ap.srcS ], W, H, qx, qy ) );
-                     iq = xyz( LdP4< F16 >( P.cur[ ap.srcI ], W, H, qx, qy ) );
+    float pvar;
+    if( FIRST )
+    {
+        float r = 0.0f;
+#pragma unroll
+        for( int yy = -1; yy <= 1; yy++ )
+        {
+#pragma unroll
+            for( int xx = -1; xx <= 1; xx++ )
+            {
+                r += s_diff[ c + yy * TW + xx ].w * ( ( xx == 0 ? 0.5f : 0.25f ) * ( yy == 0 ? 0.5f : 0.25f ) );
+            }
+        }
+        pvar = sqrtf( fmaxf( r, 0.0f ) );
+        StP1< F16 >( P.cur[ RG_EXT_PLANE_ATROUS_FILTERED_VARIANCE ], W, x, y, pvar );
+    }
+    else
+    {
+        pvar = LdP1< F16 >( P.cur[ RG_EXT_PLANE_ATROUS_FILTERED_VARIANCE ], W, H, x, y );
+    }
+    AtrousPixel< F16 >( P, d, x, y, k, step, ap, s_nrm[ c ], depth, Ld1( P.cur[ RG_EXT_PLANE_DEPTH_GRAD ], W, H, x, y ), s_rgh[ c ], cd, cs, ci, pvar,
+                 [ & ]( int xx, int yy, v3& nq, float& dq, float& rq, float4& cq, v3& sq, v3& iq ) {
+                     const int i = c + yy * TW + xx * step;
+                     nq          = s_nrm[ i ];
+                     dq          = s_dep[ i ];
+                     rq          = s_rgh[ i ];
+                     cq          = s_diff[ i ];
+                     sq          = s_spec[ i ];
+                     iq          = s_ind[ i ];
                  } );
 }
 
@@ -1058,29 +1048,32 @@ void DenoiseVariance( FramebufferSet& fb, const RgExtFrameParams& p, hipStream_t
 
 namespace
 {
-template< int TBX >
-void LaunchAtrousNTile( FramebufferSet& fb, const Dims& d, const AtrousPlanes& ap, uint32_t k, hipStream_t s )
+template< int TBX, bool FIRST >
+void LaunchAtrousTile( FramebufferSet& fb, const Dims& d, const AtrousPlanes& ap, uint32_t k, hipStream_t s )
 {
-    const dim3 grid( DivUp( d.W, TBX ), DivUp( d.H, THREADS / TBX ) );
+    // groups of THREADS / TBX lattice rows, each for the 2^k rows between
+    constexpr int ROWS = THREADS / TBX;
+    const dim3    grid( DivUp( d.W, TBX ), DivUp( d.H, ROWS << k ) << k );
+    const size_t  lds = size_t( TBX + ( 2 << k ) ) * ( ROWS + 2 ) * ATROUS_TEXEL;
     if( fb.Half() )
     {
-        k_atrousN< true, TBX ><<< grid, THREADS, 0, s >>>( fb.Ptrs(), d, ap, int( k ) );
+        k_atrous< true, TBX, FIRST ><<< grid, THREADS, lds, s >>>( fb.Ptrs(), d, ap, int( k ) );
     }
     else
     {
-        k_atrousN< false, TBX ><<< grid, THREADS, 0, s >>>( fb.Ptrs(), d, ap, int( k ) );
+        k_atrous< false, TBX, FIRST ><<< grid, THREADS, lds, s >>>( fb.Ptrs(), d, ap, int( k ) );
     }
-    CheckLaunch( "k_atrousN" );
+    CheckLaunch( "k_atrous" );
 }
 
 void LaunchAtrousN( FramebufferSet& fb, const Dims& d, const AtrousPlanes& ap, uint32_t k, uint32_t tileW, hipStream_t s )
 {
     switch( tileW )
     {
-        case 16: LaunchAtrousNTile< 16 >( fb, d, ap, k, s ); break;
-        case 64: LaunchAtrousNTile< 64 >( fb, d, ap, k, s ); break;
-        case 128: LaunchAtrousNTile< 128 >( fb, d, ap, k, s ); break;
-        default: LaunchAtrousNTile< 32 >( fb, d, ap, k, s ); break;
+        case 16: LaunchAtrousTile< 16, false >( fb, d, ap, k, s ); break;
+        case 64: LaunchAtrousTile< 64, false >( fb, d, ap, k, s ); break;
+        case 128: LaunchAtrousTile< 128, false >( fb, d, ap, k, s ); break;
+        default: LaunchAtrousTile< 32, false >( fb, d, ap, k, s ); break;
     }
 }
 } // namespace
@@ -1095,18 +1088,9 @@ void DenoiseAtrous( FramebufferSet& fb, const RgExtFrameParams& p, uint32_t k, h
     }
     const Dims         d  = GetDims( fb );
     const AtrousPlanes ap = GetAtrousPlanes( k, p.atrousIterations );
-    const dim3         grid( DivUp( d.W, BX ), DivUp( d.H, BY ) );
     if( k == 0 )
     {
-        if( fb.Half() )
-        {
-            k_atrous0< true ><<< grid, THREADS, 0, s >>>( fb.Ptrs(), d, ap );
-        }
-        else
-        {
-            k_atrous0< false ><<< grid, THREADS, 0, s >>>( fb.Ptrs(), d, ap );
-        }
-        CheckLaunch( "k_atrous0" );
+        LaunchAtrousTile< 64, true >( fb, d, ap, k, s );
     }
     else
     {

@@ -398,3 +398,22 @@ def test_gpu_atrous_tile_autotune(gpu):
     assert ms[(16, 32, 64, 128).index(chosen.value)] == min(ms)
     with pytest.raises(ffi.RgError):
         ffi.call("rgExtFramebuffersSetAtrousTile", g.h, 48)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W,H", [(2, 1), (62, 3), (66, 65), (130, 129), (66, 257)])
+@pytest.mark.parametrize("width", [64, 16])
+def test_gpu_atrous_lattice_edges(gpu, oracle, W, H, width):
+    """A workgroup of an a-trous pass takes every step-th row and stages a
+    halo: images smaller than a lattice group, cut in both directions and one
+    past its size, through temporal accumulation and five iterations, within
+    the bound of the chain.  (66 columns at 257 rows: at 34 the FP64 oracle's
+    own accumulated planes are not finite for these inputs.)"""
+    print(f"a-trous lattice edges {W}x{H}, {width} columns", flush=True)
+    g, o = _pair(oracle, W, H, seed=W * 31 + H)
+    ffi.call("rgExtFramebuffersSetAtrousTile", g.h, width)
+    p = frame_params(W, H)
+    p.atrousIterations = 5
+    ffi.call("rgExtDenoise", g.h, p, None)
+    o.run("", p)
+    _check(g, o, ["PRE_FINAL", "HISTOGRAM_INPUT", "DIFF_TEMPORARY", "ACCUM_HISTORY_LENGTH", "DIFF_PONG", "SPEC_PONG", "INDIR_PONG"])
