@@ -1958,18 +1958,46 @@ __global__ __launch_bounds__( THREADS ) void k_indirect_final( RgExtFrameParams 
     {
         const float radius  = mixf( 8.0f, 32.0f, clampf( float( H ) / 1080.0f, 0.0f, 1.0f ) );
         uint32_t    nobiasM = comb.M;
-        for( int k = 0; k < spatialCount; k++ )
-        {
+        // Neighbour k's pixel follows from the salt, which a neighbour that is
+        // taken moves by two and one that is not by one: the next record is
+        // asked for before this one is looked at, as if this one is taken, and
+        // asked for again where it was not (a chain of up to six fetches: 230
+        // -> 178 us at 1920x1080).
+        auto neighbour = [ & ]( uint32_t at, int* qx, int* qy ) __attribute__( ( always_inline ) ) {
             float r4[ 4 ];
-            rnd8_4( seed, salt++, r4 );
-            const int qx = x + int( ( r4[ 0 ] * 2.0f - 1.0f ) * radius );
-            const int qy = y + int( ( r4[ 1 ] * 2.0f - 1.0f ) * radius );
+            rnd8_4( seed, at, r4 );
+            *qx = x + int( ( r4[ 0 ] * 2.0f - 1.0f ) * radius );
+            *qy = y + int( ( r4[ 1 ] * 2.0f - 1.0f ) * radius );
             // the neighbour's GI_REUSE record (one cache line), at the pixel
             // clamped into the image; a pixel outside fails the reuse test
             // (its render-area check), so the clamped values are never used
-            const size_t  qi  = size_t( min( max( qy, 0 ), H - 1 ) ) * W + min( max( qx, 0 ), W - 1 );
-            const uint4*  rec = Plane< uint4 >( P, RG_EXT_PLANE_GI_REUSE ) + 4 * qi;
-            const uint4   r0 = rec[ 0 ], r1 = rec[ 1 ], r2 = rec[ 2 ], r3 = rec[ 3 ];
+            const size_t qi = size_t( min( max( *qy, 0 ), H - 1 ) ) * W + min( max( *qx, 0 ), W - 1 );
+            return Plane< uint4 >( P, RG_EXT_PLANE_GI_REUSE ) + 4 * qi;
+        };
+        uint4    n0, n1, n2, n3;
+        int      nx = 0, ny = 0;
+        uint32_t fetched = salt; // the salt of the record in n0..n3
+        if( spatialCount > 0 )
+        {
+            const uint4* rec = neighbour( fetched, &nx, &ny );
+            n0 = rec[ 0 ], n1 = rec[ 1 ], n2 = rec[ 2 ], n3 = rec[ 3 ];
+        }
+        for( int k = 0; k < spatialCount; k++ )
+        {
+            if( fetched != salt )
+            {
+                const uint4* rec = neighbour( salt, &nx, &ny );
+                n0 = rec[ 0 ], n1 = rec[ 1 ], n2 = rec[ 2 ], n3 = rec[ 3 ];
+            }
+            const uint4 r0 = n0, r1 = n1, r2 = n2, r3 = n3;
+            const int   qx = nx, qy = ny;
+            salt++;
+            fetched = salt + 1;
+            if( k + 1 < spatialCount )
+            {
+                const uint4* rec = neighbour( fetched, &nx, &ny );
+                n0 = rec[ 0 ], n1 = rec[ 1 ], n2 = rec[ 2 ], n3 = rec[ 3 ];
+            }
             auto          f  = []( uint32_t v ) { return __uint_as_float( v ); };
             const float4  x1q = make_float4( f( r0.x ), f( r0.y ), f( r0.z ), 0.0f );
             if( r1.w != 0u || !ReuseIndirOk( lo, hi, H, qx, qy, depthCur, f( r0.w ), s.normal, mk3( f( r1.x ), f( r1.y ), f( r1.z ) ) ) )
