@@ -12,12 +12,12 @@ geometry is uploaded once before the timed region and stays resident in HBM
 
 Prints one JSON line.  `roofline` prices the dominant kernel (the traversal
 kernel k_trace) by algorithmic bytes: 32 B ray in + 16 B hit out per ray,
-256 B per BVH8 node visit, 36 B per triangle test, divided by the kernel time
-measured with HIP events recorded on the instance stream around every launch.
+128 B per node visit, 36 B per triangle test, divided by the kernel time from
+the device clock (first block's start to last block's end of every launch).
 `cpu_baseline` times the CPU oracle on a bounded sample of the same frame.
 
 Beside the FP32 line (`value`), the same JSON object carries
-- `fp16`: the same frames with FP16 BVH nodes and FP16 storage of the
+- `fp16`: the same frames with both FP16 precision flags: FP16 storage of the
   denoiser's temporal and a-trous planes (frames/s, Mrays/s, and the last
   frame's denoised-radiance difference from the FP32 run);
 - `reflrefr`: the same frames with every third icosphere a mirror, glass or
@@ -50,7 +50,7 @@ METRIC = "Mrays/s & 1080p frames/s (FP16 vs FP32); p99 frame latency at 256 sess
 WIDTH, HEIGHT = 1920, 1080
 ORBIT_FRAMES = 60
 BYTES_PER_RAY = 32 + 16      # RgExtRay in, RgExtHit out
-BYTES_PER_NODE = 256         # one FP32 BVH8 node
+BYTES_PER_NODE = 128         # one traversal node
 BYTES_PER_TRI = 36           # three FP32 vertices
 HBM_PEAK_GBPS = 8000.0       # MI355X HBM3E
 TRAFFIC_FILE = REPO / "profiles" / "k_trace_traffic.json"
@@ -594,7 +594,7 @@ def main(argv=None) -> int:
             "launches": launches,
             "node_visits_per_ray": nodes / rays,
             "triangle_tests_per_ray": tris / rays,
-            # `achieved` counts every node fetch as 256 B although the node
+            # `achieved` counts every node fetch as 128 B although the node
             # array stays L2-resident: a work rate.  What the counters of
             # profiles/k_trace_traffic.json show for the same kernel:
             "measured": None if not prof else {
@@ -626,7 +626,7 @@ def main(argv=None) -> int:
         g, e = final16[..., :3].astype(np.float64), final32[..., :3].astype(np.float64)
         rel = (np.abs(g - e) / (np.abs(e) + 1e-3 * np.abs(e).mean())).max(axis=-1)
         out["fp16"] = {
-            "precision": "FP16 BVH nodes (144 B) + FP16 temporal/a-trous storage; FP32 arithmetic",
+            "precision": "FP16 temporal/a-trous storage (the traversal nodes are the same); FP32 arithmetic",
             "frames_per_s": n16 / wall16,
             "mrays_per_s": rays16 / wall16 / 1e6,
             "speedup_vs_fp32": (n16 / wall16) / (n / wall),

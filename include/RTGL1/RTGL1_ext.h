@@ -519,7 +519,8 @@ typedef struct RgExtDrawFramePathParams
 #define RG_EXT_PRECISION_FP16_NODES   2u
 
 /* Per-frame statistics of the last rgDrawFrame; GPU times from HIP events
- * recorded on the instance stream around each stage.  rgDrawFrame returns
+ * recorded on the instance stream around each stage, and of the traversal
+ * kernels from the device's clock inside them.  rgDrawFrame returns
  * once its frame is enqueued (at most two frames in flight, as the
  * reference's MAX_FRAMES_IN_FLIGHT, Source/Common.h:38), so
  * rgExtGetFrameStats waits for the last frame to finish. */
