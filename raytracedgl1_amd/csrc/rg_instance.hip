@@ -238,8 +238,8 @@ struct Instance
             ( changed || !dscene.bvhValid || bvh.nodeFormat != nodeFmt ||
               std::memcmp( dscene.builtClassTris, dscene.classTris, sizeof( dscene.classTris ) ) != 0 ) )
         {
-            // one triangle per leaf: measured fastest at 1M triangles (more
-            // nodes, fewer triangle tests per leaf visit)
+            // leafMax is that of the published nodes; frames walk the
+            // traversal tree, which has one triangle per leaf slot
             RgExtBvhBuildParams bp = { 1, nodeFmt };
             BuildFrameBvh( bvh, dscene.tris.as< float >(), dscene.classTris, GC_COUNT, bp, s );
             dscene.bvhValid      = true;

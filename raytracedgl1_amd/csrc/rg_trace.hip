@@ -45,9 +45,9 @@ constexpr uint32_t MAX_STEPS_PER_RAY = 1u << 22;
 constexpr uint32_t RAY_CHUNK_DEFAULT = 64; // rays per counter atomic
 // A wave refills its idle lanes once at least this many are idle (or none
 // is busy): the refill block (ballots, the chunk atomic, the ray set-up with
-// its six divisions) then runs for many lanes at once instead of for the
-// one or two lanes that finish in a typical iteration.  Measured on the
-// 1080p frame: 1 -> 3.77 ms of traversal, 8 -> 3.64, 16 -> 3.57, 32 -> 3.60.
+// its divisions) then runs for many lanes at once instead of for the one or
+// two lanes that finish in a typical iteration.  Camera rays at 1920x1080
+// with 8 / 16 / 24 / 32: 1.00 / 1.00 / 1.02 / 1.08 of the time.
 constexpr uint32_t REFILL_MIN_LANES = 16;
 constexpr uint32_t RAY_PARTITIONS    = 32;  // ray counters
 constexpr uint32_t COUNTER_STRIDE    = 64;  // u32 between counters (256 B)
