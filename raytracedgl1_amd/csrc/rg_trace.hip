@@ -374,7 +374,12 @@ __global__ __launch_bounds__( TR_THREADS, 4 ) void k_trace( TraceArgs a )
                 {
                     my = newBase + ( rank - left );
                 }
-                if( my < a.count )
+                if( grab && newBase < a.count && rank >= left + a.chunk )
+                {
+                    // past the chunk: rays of another wave; this lane takes its
+                    // ray from the next chunk
+                }
+                else if( my < a.count )
                 {
                     const RgExtRay r = a.rays[ my ];
                     rayId            = my;
@@ -739,7 +744,12 @@ __global__ __launch_bounds__( TR_THREADS ) void k_trace_view( TraceArgs a )
                 {
                     my = newBase + ( rank - left );
                 }
-                if( my < a.count )
+                if( grab && newBase < a.count && rank >= left + a.chunk )
+                {
+                    // past the chunk: rays of another wave; this lane takes its
+                    // ray from the next chunk
+                }
+                else if( my < a.count )
                 {
                     const RgExtRay r = a.rays[ my ];
                     rayId            = my;

@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 from raytracedgl1_amd import ffi, scenes
-from raytracedgl1_amd.ffi import HIT_DTYPE, RAY_DTYPE, RG_EXT_TRACE_ANY_HIT, Bvh, DeviceArray
+from raytracedgl1_amd.ffi import HIT_DTYPE, RAY_DTYPE, RG_EXT_TRACE_ANY_HIT, RG_EXT_TRACE_COLLECT_STATS, Bvh, DeviceArray
 
 pytestmark = pytest.mark.gpu
 
@@ -130,3 +130,24 @@ def test_autotune_keeps_results(gpu):
     # a batched BVH is traced only through the batched entry point
     with pytest.raises(ffi.RgError):
         bb.trace(dr, len(allrays), dh, 0)
+
+
+def test_visit_counts_do_not_depend_on_tuning(gpu):
+    """Every ray is traced, and counted, by one wave only, whatever number of
+    rays the tuning lets a wave take at a time: a wave has 64 lanes to fill
+    from a chunk of 32.  Tuned again and again, on few and on many rays (the
+    times are close, so each choice comes up), up to a chunk of 32."""
+    s = scenes.terrain_boxes_scene()
+    rays = _rays(300_000, 77, -30, 30)
+    b = Bvh()
+    b.build(DeviceArray.from_numpy(s.tris), len(s.tris), 1)
+    dr, dh = DeviceArray.from_numpy(rays), DeviceArray(len(rays), HIT_DTYPE)
+    before = {}
+    for k in range(13):
+        chunk = b.autotune(dr, (20_000, len(rays))[k % 2], dh).rayChunk if k else 64
+        print(f"visit counts, chunk {chunk}", flush=True)
+        for flags in (RG_EXT_TRACE_COLLECT_STATS, RG_EXT_TRACE_COLLECT_STATS | RG_EXT_TRACE_ANY_HIT):
+            b.trace(dr, len(rays), dh, flags)
+            assert b.trace_stats() == before.setdefault(flags, b.trace_stats()), (flags, chunk)
+        if chunk == 32:
+            break
