@@ -690,7 +690,8 @@ bool Slab( const Pre& r, const Node8& nd, int k, float tmin, float tmax, float* 
     const float ty0 = ( nd.lo_y[ k ] - r.o.y ) * r.inv.y, ty1 = ( nd.hi_y[ k ] - r.o.y ) * r.inv.y;
     const float tz0 = ( nd.lo_z[ k ] - r.o.z ) * r.inv.z, tz1 = ( nd.hi_z[ k ] - r.o.z ) * r.inv.z;
     const float tn = std::fmax( std::fmax( std::fmin( tx0, tx1 ), std::fmin( ty0, ty1 ) ), std::fmax( std::fmin( tz0, tz1 ), tmin ) );
-    const float tf = std::fmin( std::fmin( std::fmax( tx0, tx1 ), std::fmax( ty0, ty1 ) ), std::fmax( tz0, tz1 ) ) * 1.0000004f;
+    float       tf = std::fmin( std::fmin( std::fmax( tx0, tx1 ), std::fmax( ty0, ty1 ) ), std::fmax( tz0, tz1 ) );
+    tf *= tf < 0.0f ? 2.0f - 1.0000004f : 1.0000004f; // away from tn on either side of the origin
     *tnOut = tn;
     return tn <= std::fmin( tf, tmax );
 }

@@ -1308,9 +1308,9 @@ __device__ __forceinline__ AxisGrid MakeGrid( float lo, float hi )
     return g;
 }
 // The plane below lo or above hi.  The traversal evaluates
-// fma(q, 2^k / d, (origin - o) / d) with up to 2^-11 steps of rounding error
-// beyond a relative one of a few units in the last place; 2^-9 steps of
-// margin cover it.
+// fma(q, 2^k / d, (origin - o) / d) with up to 2^-10 steps of rounding error
+// beyond a relative one of its second term, which it covers itself; 2^-9 steps
+// of margin cover the steps.
 __device__ __forceinline__ uint16_t GridBits( double q )
 {
     return __builtin_bit_cast( uint16_t, _Float16( float( q ) ) ); // whole and at most 2047: exact

@@ -198,15 +198,28 @@ __device__ __forceinline__ void LoadHalfNode( const void* nodes, uint32_t node, 
     }
 }
 
-// Distances of a traversal node's planes are fma(q, scale / d, (origin - o) / d),
-// the far ones with both terms scaled by FAR_SLACK; against the exact
-// distance of the plane the rounding errors are at most 8 u |t| (u = 2^-24;
-// the hardware reciprocal's is in it) and 2^-11 grid steps.  The planes were
-// moved out by 2^-9 steps, and the relative part of both sides is covered by
-// the slack of the far distances, 33 u, and of the best hit so far: every box
-// that the exact ray meets before the best hit is visited.
+// Distances of a traversal node's planes are fma(q, scale / d, (origin - o) / d).
+// With u = 2^-24 and a hardware reciprocal off by up to 2 u, that is within
+// 5 u |(origin - o) / d| and 3 u * 2047 < 2^-10 grid steps of the plane's exact
+// distance.  The planes were moved out by 2^-9 steps, and the term (origin - o) / d
+// is moved by BOX_SLACK (16 u) of it, down for near planes and up for far ones,
+// so that each distance by itself is on the safe side, before and behind the
+// ray's origin: every box that the exact ray meets before the best hit is
+// visited.  Where the term overflows towards the side that would cull, moving
+// it gives inf - inf, and min / max leave that axis out.
+// FAR_SLACK is the relative slack of the entry roots' boxes, BEST_SLACK that of
+// the best hit so far.
+constexpr float BOX_SLACK  = 0x1p-20f;
 constexpr float FAR_SLACK  = 1.000002f;
 constexpr float BEST_SLACK = 1e-6f;
+
+// 1 / d for box distances: GuardDir's least |d|, raised with |o| so that a
+// box's distance from a far origin does not overflow.
+__device__ __forceinline__ float BoxRcp( float d, float o )
+{
+    const float least = fmaxf( 1e-20f, fabsf( o ) * 0x1p-126f );
+    return __builtin_amdgcn_rcpf( fabsf( d ) >= least ? d : ( d < 0.0f ? -least : least ) );
+}
 
 __device__ __forceinline__ void CmpSwap32( uint32_t& a, uint32_t& b )
 {
@@ -387,14 +400,15 @@ __global__ __launch_bounds__( TR_THREADS, 4 ) void k_trace( TraceArgs a )
                                                    mk3( r.direction[ 0 ], r.direction[ 1 ], r.direction[ 2 ] ) );
                     // the reciprocals only place boxes: a unit in the last place
                     // is inside the slack
-                    ray.invd         = mk3( __builtin_amdgcn_rcpf( GuardDir( ray.d.x ) ), __builtin_amdgcn_rcpf( GuardDir( ray.d.y ) ),
-                                            __builtin_amdgcn_rcpf( GuardDir( ray.d.z ) ) );
+                    ray.invd         = mk3( BoxRcp( ray.d.x, ray.o.x ), BoxRcp( ray.d.y, ray.o.y ), BoxRcp( ray.d.z, ray.o.z ) );
                     sgn              = ( ray.invd.x < 0.0f ? 1u : 0u ) | ( ray.invd.y < 0.0f ? 2u : 0u ) | ( ray.invd.z < 0.0f ? 4u : 0u );
                     tmin             = r.tmin;
                     bestT            = r.tmax;
                     bestU = bestV = 0.0f;
                     bestPrim      = RG_EXT_MISS;
-                    bestBox       = r.tmax + fabsf( r.tmax ) * BEST_SLACK;
+                    // (from an infinite origin no triangle is hit: no box is either)
+                    bestBox       = fmaxf( fmaxf( fabsf( ray.o.x ), fabsf( ray.o.y ) ), fabsf( ray.o.z ) ) == INFINITY
+                                        ? -INFINITY : r.tmax + fabsf( r.tmax ) * BEST_SLACK;
                     base          = 0; // the root
                     kids          = 1;
                     list          = 0;
@@ -522,21 +536,26 @@ __global__ __launch_bounds__( TR_THREADS, 4 ) void k_trace( TraceArgs a )
                     const half8    qny = LoadHalves( np + 3 + ny ), qfy = LoadHalves( np + 4 - ny );
                     const half8    qnz = LoadHalves( np + 5 + nz ), qfz = LoadHalves( np + 6 - nz );
                     const uint2    r7 = *reinterpret_cast< const uint2* >( np + 7 );
+                    // all eight are asked for before the first is waited for: left
+                    // to itself the compiler puts three behind the first use (+4%)
+                    __builtin_amdgcn_sched_barrier( 0 );
                     list >>= 3;
                     kids--;
-                    // per axis: scale / d and (origin - o) / d
+                    // per axis: scale / d, and (origin - o) / d moved back and on
                     const float sx = __uint_as_float( ( r0.w & 0xFFu ) << 23 ) * ray.invd.x, bx = ( __uint_as_float( r0.x ) - ray.o.x ) * ray.invd.x;
                     const float sy = __uint_as_float( ( r0.w & 0xFF00u ) << 15 ) * ray.invd.y, by = ( __uint_as_float( r0.y ) - ray.o.y ) * ray.invd.y;
                     const float sz = __uint_as_float( ( r0.w & 0xFF0000u ) << 7 ) * ray.invd.z, bz = ( __uint_as_float( r0.z ) - ray.o.z ) * ray.invd.z;
-                    const float fsx = sx * FAR_SLACK, fbx = bx * FAR_SLACK, fsy = sy * FAR_SLACK, fby = by * FAR_SLACK, fsz = sz * FAR_SLACK, fbz = bz * FAR_SLACK;
+                    const float nbx = __builtin_fmaf( fabsf( bx ), -BOX_SLACK, bx ), fbx = __builtin_fmaf( fabsf( bx ), BOX_SLACK, bx );
+                    const float nby = __builtin_fmaf( fabsf( by ), -BOX_SLACK, by ), fby = __builtin_fmaf( fabsf( by ), BOX_SLACK, by );
+                    const float nbz = __builtin_fmaf( fabsf( bz ), -BOX_SLACK, bz ), fbz = __builtin_fmaf( fabsf( bz ), BOX_SLACK, bz );
                     const uint32_t inner = ( r0.w >> 24 ) & 15u, leaf = r0.w >> 28;
                     uint32_t       key[ 8 ], hits = 0u;
 #pragma unroll
                     for( int k = 0; k < 8; k++ )
                     {
-                        const float tx0 = __builtin_fmaf( float( qnx[ k ] ), sx, bx ), tx1 = __builtin_fmaf( float( qfx[ k ] ), fsx, fbx );
-                        const float ty0 = __builtin_fmaf( float( qny[ k ] ), sy, by ), ty1 = __builtin_fmaf( float( qfy[ k ] ), fsy, fby );
-                        const float tz0 = __builtin_fmaf( float( qnz[ k ] ), sz, bz ), tz1 = __builtin_fmaf( float( qfz[ k ] ), fsz, fbz );
+                        const float tx0 = __builtin_fmaf( float( qnx[ k ] ), sx, nbx ), tx1 = __builtin_fmaf( float( qfx[ k ] ), sx, fbx );
+                        const float ty0 = __builtin_fmaf( float( qny[ k ] ), sy, nby ), ty1 = __builtin_fmaf( float( qfy[ k ] ), sy, fby );
+                        const float tz0 = __builtin_fmaf( float( qnz[ k ] ), sz, nbz ), tz1 = __builtin_fmaf( float( qfz[ k ] ), sz, fbz );
                         const float tn  = fmaxf( fmaxf( fmaxf( tx0, ty0 ), tz0 ), tmin );
                         const float tf  = fminf( fminf( fminf( tx1, ty1 ), tz1 ), bestBox );
                         const bool  h   = tn <= tf;

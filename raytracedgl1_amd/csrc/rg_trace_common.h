@@ -59,9 +59,16 @@ __host__ __device__ __forceinline__ RayPre MakeRayPre( v3 o, v3 d )
     return r;
 }
 
+// The far distance of a box moved away from the near one by a relative slack
+// (given as 1 + slack), whichever side of the origin the box is on.
+__host__ __device__ __forceinline__ float FarOut( float t, float slack )
+{
+    return t * ( t < 0.0f ? 2.0f - slack : slack );
+}
+
 // Robust slab test (Ize, "Robust BVH Ray Traversal", JCGT 2(2), 2013): the far
-// distance is scaled by 1 + 2*gamma(3) so rounding never culls a box that the
-// exact ray touches.
+// distance is moved out by 2*gamma(3) of it so that rounding never culls a box
+// that the exact ray touches.
 __host__ __device__ __forceinline__ bool SlabTest( const RayPre& r,
                                                    float lx, float ly, float lz,
                                                    float hx, float hy, float hz,
@@ -71,7 +78,7 @@ __host__ __device__ __forceinline__ bool SlabTest( const RayPre& r,
     const float ty0 = ( ly - r.o.y ) * r.invd.y, ty1 = ( hy - r.o.y ) * r.invd.y;
     const float tz0 = ( lz - r.o.z ) * r.invd.z, tz1 = ( hz - r.o.z ) * r.invd.z;
     const float tn  = fmaxf( fmaxf( fminf( tx0, tx1 ), fminf( ty0, ty1 ) ), fmaxf( fminf( tz0, tz1 ), tmin ) );
-    const float tf  = fminf( fminf( fmaxf( tx0, tx1 ), fmaxf( ty0, ty1 ) ), fmaxf( tz0, tz1 ) ) * farSlack;
+    const float tf  = FarOut( fminf( fminf( fmaxf( tx0, tx1 ), fmaxf( ty0, ty1 ) ), fmaxf( tz0, tz1 ) ), farSlack );
     *tnearOut       = tn;
     return tn <= fminf( tf, tmax );
 }
@@ -92,7 +99,7 @@ __host__ __device__ __forceinline__ bool SlabTestOrdered( const RayPre& r,
     const float ty0 = ( ny - r.o.y ) * r.invd.y, ty1 = ( fy - r.o.y ) * r.invd.y;
     const float tz0 = ( nz - r.o.z ) * r.invd.z, tz1 = ( fz - r.o.z ) * r.invd.z;
     const float tn  = fmaxf( fmaxf( tx0, ty0 ), fmaxf( tz0, tmin ) );
-    const float tf  = fminf( fminf( tx1, ty1 ), tz1 ) * 1.0000004f;
+    const float tf  = FarOut( fminf( fminf( tx1, ty1 ), tz1 ), 1.0000004f );
     *tnearOut       = tn;
     return tn <= fminf( tf, tmax );
 }

@@ -266,6 +266,65 @@ def test_traversal_nodes_at_their_limits(gpu, kind):
     assert np.array_equal(occ, g["prim"] != RG_EXT_MISS)
 
 
+def _grid_wall():
+    """3200 triangles side by side in the plane x = 0."""
+    y, z = np.meshgrid(np.arange(40.0) - 20.0, np.arange(40.0) - 20.0, indexing="ij")
+    p = [np.stack([np.zeros(1600), y.ravel() + a, z.ravel() + b], 1) for a, b in ((0, 0), (1, 0), (0, 1), (1, 1))]
+    return np.concatenate([np.concatenate([p[0], p[1], p[2]], 1), np.concatenate([p[3], p[2], p[1]], 1)]).astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", ["wall", "soup", "axis"])
+def test_boxes_behind_the_origin_and_beyond_the_range(gpu, oracle, kind):
+    """Hits of both walks against an FP64 loop over all triangles: at negative
+    distances (tmin < 0), where a slack on the far planes must not move them
+    nearer, down to boxes without thickness; and along rays parallel to an axis
+    on which the boxes reach out to 1e19, where distances overflow."""
+    print(f"boxes {kind}", flush=True)
+    r = np.random.default_rng(23)
+    n = 20000
+    rays = np.zeros(n, RAY_DTYPE)
+    if kind == "axis":
+        far = np.zeros((8, 3, 3))
+        far[np.arange(8), :, np.arange(8) % 2] = np.repeat([1e19, -1e19], 4)[:, None]
+        far += r.uniform(-1e13, 1e13, far.shape)
+        tris = np.concatenate([_random_tris(300, 4, spread=4.0), far.reshape(8, 9).astype(np.float32)])
+        rays["origin"] = r.uniform(-5, 5, (n, 3))
+        rays["origin"][:50, 0] = 1e25  # outside, and nowhere
+        rays["origin"][50:100, 1] = -np.inf
+        rays["direction"] = r.choice([0.0, -0.0, 1e-30, -1e-30], (n, 3))
+        rays["direction"][:, 2] = r.choice([-1.0, 1.0], n)
+        rays["tmax"] = 1000.0
+    else:
+        tris = _grid_wall() if kind == "wall" else _random_tris(3000, 5, size=0.2)
+        t = tris[r.integers(0, len(tris), n)].reshape(n, 3, 3).astype(np.float64)
+        d = r.normal(size=(n, 3)) + np.array([4.0, 0.0, 0.0])
+        d /= np.linalg.norm(d, axis=1, keepdims=True)
+        dist = -(10.0 ** r.uniform(0, 5 if kind == "wall" else 3, n))
+        rays["origin"] = (t * r.dirichlet([4, 4, 4], n)[..., None]).sum(1) - d * dist[:, None]
+        rays["direction"] = d
+        rays["tmin"] = dist * 1.5
+        rays["tmax"] = np.where(r.random(n) < 0.5, 0.0, 100.0)
+    b, _ = _gpu_bvh(tris, 1)
+    tb, _, _, p = oracle.bruteforce(tris, rays)
+    hit = p != RG_EXT_MISS
+    v = tris[np.where(hit, p, 0)].reshape(n, 3, 3).astype(np.float64)
+    nrm = np.cross(v[:, 1] - v[:, 0], v[:, 2] - v[:, 0])
+    cos = np.abs((nrm * rays["direction"]).sum(1)) / np.linalg.norm(nrm, axis=1)
+    assert hit.mean() > 0.3
+    for flags in (0, RG_EXT_TRACE_COLLECT_STATS):
+        g = _trace_gpu(b, rays, flags)
+        same = g["prim"] == p
+        # the FP32 triangle test and the FP64 one part at edges and ties only:
+        # a ray is placed within some 1e-7 of its distance, of triangles of 1 (wall) and 0.2
+        assert same.mean() >= 0.98, (flags, same.mean())
+        assert (hit & (g["prim"] == RG_EXT_MISS)).mean() <= 5e-3, flags
+        # that error (16 roundings of the distance bound it) across the plane,
+        # along the ray: over the cosine of incidence
+        assert (np.abs(g["t"] - tb) * cos <= 16 * 2.0 ** -24 * np.abs(tb) + 1e-6)[same & hit].all(), flags
+    occ = _trace_gpu(b, rays, RG_EXT_TRACE_ANY_HIT)["prim"] != RG_EXT_MISS
+    assert np.array_equal(occ, _trace_gpu(b, rays, 0)["prim"] != RG_EXT_MISS)
+
+
 @pytest.mark.parametrize("n", [1, 5, 4097, 16383, 16385, 65537, 131073, 262145, 300001])
 def test_launch_widths(gpu, n):
     """Ray counts about the change between the lanes per wave that take rays
