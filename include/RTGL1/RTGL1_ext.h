@@ -215,7 +215,10 @@ typedef struct RgExtTraceTuning
 
 /* Times every stack depth x ray chunk on the given rays (rayOffsets for a
  * batched BVH, else rayCount) and keeps the fastest for this BVH object's
- * later traces; results do not depend on the choice.  Synchronises the
+ * later traces; results do not depend on the choice.  Fewer rays than half the
+ * resident lanes (131,072 with 1024 blocks) are not taken by the chunk: then
+ * the stack depths alone are timed, and the chunk is the default.
+ * RG_EXT_TRACE_COLLECT_STATS is left out of the timed traces.  Synchronises the
  * stream.  No counterpart in the reference (the driver schedules its own
  * traversal). */
 RGAPI RgResult RGCONV rgExtTraceAutotune( RgExtBvh          bvh,

@@ -1489,6 +1489,9 @@ void AutotuneTrace( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
                     uint32_t flags, hipStream_t stream, RgExtTraceTuning* out )
 {
     RG_REQUIRE( count > 0 || rayOffsets, RG_RESULT_WRONG_FUNCTION_ARGUMENT, "no rays to tune on" );
+    InitGrids( s );
+    flags &= ~RG_EXT_TRACE_COLLECT_STATS; // what is tuned is the traversal, not the counting walk
+    const uint32_t total = rayOffsets ? rayOffsets[ bvh.sceneCount ] : count;
     static const uint32_t chunks[ 3 ] = { 32, 64, 128 };
     hipEvent_t            e0, e1;
     RG_HIP_CHECK( hipEventCreate( &e0 ) );
@@ -1513,6 +1516,10 @@ void AutotuneTrace( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
     {
         for( uint32_t c : chunks )
         {
+            if( c != RAY_CHUNK_DEFAULT && LanesPerWave( total, s.grid[ v ] ) < 64u )
+            {
+                continue; // so few rays are not taken by the chunk
+            }
             s.stackVariant = v;
             s.rayChunk     = c;
             run(); // warm

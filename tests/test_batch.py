@@ -132,6 +132,27 @@ def test_autotune_keeps_results(gpu):
         bb.trace(dr, len(allrays), dh, 0)
 
 
+def test_autotune_times_the_chunk_only_where_it_is_used(gpu):
+    """A launch of fewer rays than half the resident lanes takes them by lane
+    counts of its own: such rays tell nothing about the chunk, which stays at
+    its default whatever the noise of the times.  More rays, at every tuning:
+    the same hits, with the tuned chunk above and below a launch's rays per wave."""
+    s = scenes.terrain_boxes_scene()
+    rays = _rays(600_000, 78, -30, 30)
+    b = Bvh()
+    b.build(DeviceArray.from_numpy(s.tris), len(s.tris), 1)
+    dr, dh = DeviceArray.from_numpy(rays), DeviceArray(len(rays), HIT_DTYPE)
+    before = [_trace(b, rays[:n], 0) for n in (len(rays), 300_000)]
+    for k in range(6):
+        few = b.autotune(dr, 60_000 + 10_000 * k, dh, k % 2 * RG_EXT_TRACE_COLLECT_STATS)
+        print(f"autotune on few rays: stack {few.stackLdsEntries}, chunk {few.rayChunk}", flush=True)
+        assert few.rayChunk == 64 and 0 < few.msPerLaunch <= few.msDefault
+        many = b.autotune(dr, len(rays), dh, 0)
+        print(f"autotune on many rays: stack {many.stackLdsEntries}, chunk {many.rayChunk}", flush=True)
+        for want in before:
+            assert np.array_equal(_trace(b, rays[:len(want)], 0), want)
+
+
 def test_visit_counts_do_not_depend_on_tuning(gpu):
     """Every ray is traced, and counted, by one wave only, whatever number of
     rays the tuning lets a wave take at a time: a wave has 64 lanes to fill
