@@ -1265,6 +1265,14 @@ void TraceRaysImpl( const BvhObject& bvh, TraceContext& s, const RgExtRay* d_ray
     }
     a.lanes         = lanes;
     a.chunk         = lanes < 64u ? lanes : ( s.rayChunk >= 16 && s.rayChunk <= 1024 ? s.rayChunk : RAY_CHUNK_DEFAULT );
+    // A tuned chunk above the default leaves waves without rays where it is more
+    // than a wave's share: 300,000 rays over 10,592 triangles take 61 us with
+    // chunks of 128 and 56 with 64 (60 with the share itself, 74, which a wave
+    // takes in two goes); from one chunk per wave on, 600,000 rays, both take 67.
+    if( a.chunk > RAY_CHUNK_DEFAULT && uint64_t( blocks ) * ( TR_THREADS / 64 ) * a.chunk > count )
+    {
+        a.chunk = RAY_CHUNK_DEFAULT;
+    }
     a.alpha         = alpha && tex ? alpha : nullptr;
     a.tex           = tex ? *tex : TexView{};
     if( accum )
