@@ -237,7 +237,7 @@ def run_frames(a, scene, precision: int, flags=None, planes=("PRE_FINAL",)):
         width, ms = C.c_uint32(0), (C.c_float * 4)()
         ffi.call("rgExtDenoiseAutotune", r.framebuffers().h, r.frame_params(), None, C.byref(width), ms)
         tune = {"tile_width": width.value, "tile": f"{width.value}x{256 // width.value}",
-                "iteration1_ms": {f"{w}x{256 // w}": round(float(m), 4) for w, m in zip((16, 32, 64, 128), ms)}}
+                "iteration_ms": {f"{w}x{256 // w}": round(float(m), 4) for w, m in zip((16, 32, 64, 128), ms)}}
         if precision == 0:
             a.atrous_tune = tune
         print(f"a-trous tile autotune (precision flags {precision}): {tune}", file=sys.stderr, flush=True)

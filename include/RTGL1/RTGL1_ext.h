@@ -471,11 +471,11 @@ RGAPI RgResult RGCONV rgExtDenoise( RgExtFramebuffers fb, const RgExtFrameParams
  * the workgroup tile of a-trous iterations >= 1, 256 pixels of tileWidth
  * 16, 32, 64 (the default: the fastest at 1080p) or 128 columns.  Results
  * do not depend on it.
- * rgExtDenoiseAutotune times iteration 1 on the set's current planes with
- * each width (it writes that iteration's outputs and synchronises the
- * stream), keeps the fastest for later a-trous calls on the set and returns
- * it; pMs (optional) receives the four times in milliseconds, in width
- * order. */
+ * rgExtDenoiseAutotune times the steps of iterations 1 .. atrousIterations - 1
+ * on the set's current planes with each width (it writes iteration 1's
+ * outputs and synchronises the stream), keeps the fastest for later a-trous
+ * calls on the set and returns it; pMs (optional) receives the four mean times
+ * of an iteration in milliseconds, in width order. */
 RGAPI RgResult RGCONV rgExtFramebuffersSetAtrousTile( RgExtFramebuffers fb, uint32_t tileWidth );
 RGAPI RgResult RGCONV rgExtDenoiseAutotune( RgExtFramebuffers fb, const RgExtFrameParams* p, void* stream, uint32_t* pTileWidth, float* pMs );
 /* Final compose: CmCheckerboard.comp:49-76 and CmPrepareFinal.comp:148-176

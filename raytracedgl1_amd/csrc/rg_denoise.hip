@@ -864,8 +864,9 @@ __device__ void AtrousPixel( const FbPtrs& P, const Dims& d, int x, int y, int k
 // and one lattice row) and read there eight times.  Gathered from memory, the
 // taps of steps 2 to 16 were bound by the L1, which passed every texel nine
 // times: 122 us an iteration over 1920x1080 dense pixels, 85 staged (58 and 36
-// with half storage).  64 columns: fewer make more halo, and 128 leave two
-// rows to share the halo rows.
+// with half storage).  64 columns: over steps 2 to 16 they stage 1.6 to 2.25
+// texels a pixel, 32 columns 1.4 to 2.5 and 128 columns 2.1 to 2.5; an iteration
+// of that chain takes 73, 75 and 77 us, and 90 with 16 columns.
 // FIRST: iteration 0 also filters the variance (a 3x3 Gaussian over its own
 // footprint) and keeps its root (CmSVGFAtrous_Iter0.comp:96-163).
 constexpr int ATROUS_TEXEL = 16 + 3 * 12 + 2 * 4; // bytes staged per texel
@@ -1115,6 +1116,14 @@ uint32_t AutotuneAtrous( FramebufferSet& fb, const RgExtFrameParams& p, hipStrea
     WriteGuide( fb, s );
     const Dims         d  = GetDims( fb );
     const AtrousPlanes ap = GetAtrousPlanes( 1, p.atrousIterations );
+    // every step that the width serves: its halo is a step wide, so the best
+    // width of one step is not that of the chain
+    auto chain = [ & ]( uint32_t width ) {
+        for( uint32_t k = 1; k < p.atrousIterations; k++ )
+        {
+            LaunchAtrousN( fb, d, ap, k, width, s );
+        }
+    };
     hipEvent_t         e0, e1;
     RG_HIP_CHECK( hipEventCreate( &e0 ) );
     RG_HIP_CHECK( hipEventCreate( &e1 ) );
@@ -1125,17 +1134,17 @@ uint32_t AutotuneAtrous( FramebufferSet& fb, const RgExtFrameParams& p, hipStrea
         for( uint32_t i = 0; i < 4; i++ )
         {
             const uint32_t w = ATROUS_TILE_WIDTHS[ i ];
-            LaunchAtrousN( fb, d, ap, 1, w, s ); // warm-up
+            chain( w ); // warm-up
             float ms = 1e30f;
             for( int r = 0; r < 3; r++ )
             {
                 RG_HIP_CHECK( hipEventRecord( e0, s ) );
-                LaunchAtrousN( fb, d, ap, 1, w, s );
+                chain( w );
                 RG_HIP_CHECK( hipEventRecord( e1, s ) );
                 RG_HIP_CHECK( hipEventSynchronize( e1 ) );
                 float t = 0.0f;
                 RG_HIP_CHECK( hipEventElapsedTime( &t, e0, e1 ) );
-                ms = std::min( ms, t );
+                ms = std::min( ms, t / float( p.atrousIterations - 1 ) );
             }
             if( msOut )
             {

@@ -393,11 +393,46 @@ def test_gpu_atrous_tile_autotune(gpu):
             assert np.array_equal(a, outs[width][name]), (width, name)
     chosen, ms = ctypes.c_uint32(0), (ctypes.c_float * 4)()
     ffi.call("rgExtDenoiseAutotune", g.h, p, None, ctypes.byref(chosen), ms)
-    print(f"  iteration-1 ms for widths 16/32/64/128: {[round(m, 4) for m in ms]}, kept {chosen.value}", flush=True)
+    print(f"  ms an iteration for widths 16/32/64/128: {[round(m, 4) for m in ms]}, kept {chosen.value}", flush=True)
     assert chosen.value in (16, 32, 64, 128) and all(m > 0.0 for m in ms)
     assert ms[(16, 32, 64, 128).index(chosen.value)] == min(ms)
     with pytest.raises(ffi.RgError):
         ffi.call("rgExtFramebuffersSetAtrousTile", g.h, 48)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("iterations", [4, 5])
+def test_gpu_atrous_autotune_times_every_step(gpu, iterations):
+    """The width is chosen by all iterations that use it.  Against the same
+    chain timed here, call by call, the tuner's times are less by what the calls
+    do beside (the guide, the last one's composition), the same for every width
+    up to 12% of the chain; those of step 2 alone differ by 24% of it, and the
+    width they choose for five iterations is 5% slower than the best."""
+    print(f"a-trous autotune over {iterations} iterations", flush=True)
+    W, H = 1920, 1080
+    p = frame_params(W, H)
+    p.atrousIterations = iterations
+    cur, prev = make_gbuffer(W, H, 17)
+    g = FramebufferSet(W, H)
+    fill_planes(cur, prev, g, None)
+    ffi.call("rgExtDenoise", g.h, p, None)
+    t, timed = ffi.Timer(), {}
+    for width in (16, 32, 64, 128):
+        ffi.call("rgExtFramebuffersSetAtrousTile", g.h, width)
+        runs = []
+        for _ in range(6):
+            t.start()
+            for k in range(1, iterations):
+                ffi.call("rgExtDenoiseAtrous", g.h, p, k, None)
+            t.stop()
+            runs.append(t.elapsed_ms() / (iterations - 1))
+        timed[width] = min(runs)
+    chosen, ms = ctypes.c_uint32(0), (ctypes.c_float * 4)()
+    ffi.call("rgExtDenoiseAutotune", g.h, p, None, ctypes.byref(chosen), ms)
+    print(f"  ms an iteration: {[round(m, 4) for m in ms]}, timed {timed}, kept {chosen.value}", flush=True)
+    beside = [timed[w] - m for w, m in zip((16, 32, 64, 128), ms)]
+    assert max(beside) - min(beside) <= 0.12 * min(timed.values()), beside
+    assert timed[chosen.value] <= 1.05 * min(timed.values())
 
 
 @pytest.mark.gpu
