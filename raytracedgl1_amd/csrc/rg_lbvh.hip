@@ -797,8 +797,9 @@ __global__ __launch_bounds__( THREADS ) void k_tree( TreeSets sets )
             float          la = lo ? ( left ? areaOwn : areaSib ) : -1.0f, ra = ro ? ( left ? areaSib : areaOwn ) : -1.0f;
             if( a.sizes )
             {
-                la = lo ? __uint_as_float( ( __float_as_uint( la ) & ~15u ) | min( ll - lf + 1u, 15u ) ) : la;
-                ra = ro ? __uint_as_float( ( __float_as_uint( ra ) & ~15u ) | min( rl - rf + 1u, 15u ) ) : ra;
+                // (an infinite area with these bits would be a NaN, which is never opened)
+                la = lo ? __uint_as_float( ( __float_as_uint( fminf( la, FLT_MAX ) ) & ~15u ) | min( ll - lf + 1u, 15u ) ) : la;
+                ra = ro ? __uint_as_float( ( __float_as_uint( fminf( ra, FLT_MAX ) ) & ~15u ) | min( rl - rf + 1u, 15u ) ) : ra;
             }
 #pragma unroll
             for( int k = 0; k < 3; k++ )

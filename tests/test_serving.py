@@ -377,3 +377,20 @@ def test_newest_first_and_expiry():
     assert len(res) == 4 and all(x in (serving.RG_EXT_FRAME_DONE, serving.RG_EXT_FRAME_EXPIRED) for x in status)
     assert status.count(serving.RG_EXT_FRAME_EXPIRED) >= 1
     assert st.framesDropped == status.count(serving.RG_EXT_FRAME_EXPIRED)
+
+
+def test_scene_nodes_at_infinite_areas(gpu):
+    """Boxes whose areas overflow FP32 are collapsed into 8-wide nodes as
+    others are, not left in pairs: the nodes of a scene, by the bytes that the
+    server counts (128 a node beside 160 a triangle), at coordinates of 3e22."""
+    a, _ = _scenes()
+    nodes = []
+    for scale in (1.0, 2.0 ** 70):
+        srv = serving.Server(64, 64)
+        try:
+            srv.scene(scenes.Scene(a.tris * np.float32(scale), a.normals, a.colors, a.objects, a.lights))
+            nodes.append((srv.stats().sceneBytes - len(a.tris) * 160) // 128)
+        finally:
+            srv.close()
+    print(f"nodes {nodes} of {len(a.tris)} triangles", flush=True)
+    assert 0 < nodes[1] <= 1.25 * nodes[0] < len(a.tris) / 2
