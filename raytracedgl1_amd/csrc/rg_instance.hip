@@ -194,7 +194,6 @@ struct Instance
         RG_REQUIRE( ( prec & ~( RG_EXT_PRECISION_FP16_STORAGE | RG_EXT_PRECISION_FP16_NODES ) ) == 0, RG_RESULT_WRONG_FUNCTION_ARGUMENT,
                     "unknown precisionFlags bits" );
         const uint32_t storage  = ( prec & RG_EXT_PRECISION_FP16_STORAGE ) ? RG_EXT_STORAGE_FP16 : RG_EXT_STORAGE_FP32;
-        const uint32_t nodeFmt  = ( prec & RG_EXT_PRECISION_FP16_NODES ) ? RG_EXT_BVH_NODE_FP16 : RG_EXT_BVH_NODE_FP32;
         // at most two frames in flight: the frame two back has finished
         const uint32_t slot = framesDrawn % 2u;
         RG_HIP_CHECK( hipEventSynchronize( frameDone[ slot ] ) );
@@ -235,12 +234,11 @@ struct Instance
         RG_HIP_CHECK( hipEventRecord( ev[ ST_ASSEMBLED ], s ) );
         uint32_t rebuilt = 0;
         if( dscene.triCount > 0 &&
-            ( changed || !dscene.bvhValid || bvh.nodeFormat != nodeFmt ||
-              std::memcmp( dscene.builtClassTris, dscene.classTris, sizeof( dscene.classTris ) ) != 0 ) )
+            ( changed || !dscene.bvhValid || std::memcmp( dscene.builtClassTris, dscene.classTris, sizeof( dscene.classTris ) ) != 0 ) )
         {
-            // leafMax is that of the published nodes; frames walk the
-            // traversal tree, which has one triangle per leaf slot
-            RgExtBvhBuildParams bp = { 1, nodeFmt };
+            // both are of published nodes; frames walk the traversal's tree,
+            // which has one triangle per leaf slot and one node format
+            RgExtBvhBuildParams bp = { 1, RG_EXT_BVH_NODE_FP32 };
             BuildFrameBvh( bvh, dscene.tris.as< float >(), dscene.classTris, GC_COUNT, bp, s );
             dscene.bvhValid      = true;
             dscene.builtTriCount = dscene.triCount;

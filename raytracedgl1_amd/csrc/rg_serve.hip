@@ -225,7 +225,6 @@ struct StreamCtx
 struct RgExtServer_T
 {
     RgExtServerCreateInfo                       info{};
-    uint32_t                                    nodeFormat = RG_EXT_BVH_NODE_FP32;
     uint32_t                                    batchCapacity = 1; // within-frame plane sets per stream
     uint32_t                                    activeStreams = 1; // streams that take an idle session's next launch
     uint32_t                                    storage    = RG_EXT_STORAGE_FP32;
@@ -625,7 +624,6 @@ RgResult rgExtServerCreate( const RgExtServerCreateInfo* pInfo, RgExtServer* pOu
         srv->batchCapacity = ci.batchFrames;
         srv->activeStreams = ci.streamCount;
         srv->storage    = ( ci.precisionFlags & RG_EXT_PRECISION_FP16_STORAGE ) ? RG_EXT_STORAGE_FP16 : RG_EXT_STORAGE_FP32;
-        srv->nodeFormat = ( ci.precisionFlags & RG_EXT_PRECISION_FP16_NODES ) ? RG_EXT_BVH_NODE_FP16 : RG_EXT_BVH_NODE_FP32;
         RG_HIP_CHECK( hipStreamCreateWithFlags( &srv->setup, hipStreamNonBlocking ) );
         const size_t capPx = size_t( ci.maxRenderWidth ) * ci.maxRenderHeight;
         for( uint32_t i = 0; i < ci.streamCount; i++ )
@@ -736,7 +734,7 @@ RgResult rgExtSceneBuild( RgExtScene scene )
         AssembleScene( scene->ds, s.setup );
         if( scene->ds.triCount > 0 )
         {
-            RgExtBvhBuildParams bp = { 1, s.nodeFormat };
+            RgExtBvhBuildParams bp = { 1, RG_EXT_BVH_NODE_FP32 };
             BuildFrameBvh( scene->bvh, scene->ds.tris.as< float >(), scene->ds.classTris, GC_COUNT, bp, s.setup );
             scene->ds.bvhValid      = true;
             scene->ds.builtTriCount = scene->ds.triCount;
@@ -821,7 +819,7 @@ RgResult rgExtSceneGroupCreate( RgExtServer server, const RgExtScene* pScenes, u
                 RG_HIP_CHECK( hipMemcpyAsync( tris.as< float >() + size_t( offsets[ k ] ) * 9, grp->members[ k ]->ds.tris.ptr,
                                               size_t( grp->members[ k ]->ds.triCount ) * 9 * sizeof( float ), hipMemcpyDeviceToDevice, s.setup ) );
             }
-            const RgExtBvhBuildParams bp = { 1, s.nodeFormat };
+            const RgExtBvhBuildParams bp = { 1, RG_EXT_BVH_NODE_FP32 };
             BuildBvhBatch( grp->bvh, tris.as< float >(), offsets.data(), sceneCount, bp, s.setup, false );
             RG_HIP_CHECK( hipStreamSynchronize( s.setup ) );
         }

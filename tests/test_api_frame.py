@@ -303,6 +303,21 @@ def test_lightstyles_scale_lights_one_frame_late(boxes):
     assert np.array_equal(out_of_range[1]["UNFILTERED_DIRECT"], full[1]["UNFILTERED_DIRECT"])
 
 
+def test_node_precision_flag_rebuilds_nothing(boxes):
+    """Frames walk one kind of node: the flag, on and off over unchanged
+    geometry, builds no BVH again."""
+    _, up = boxes
+    r = rtgl.Renderer(W1, H1)
+    try:
+        rebuilt = []
+        for prec in (0, ffi.RG_EXT_PRECISION_FP16_NODES, 0, ffi.RG_EXT_PRECISION_FP16_NODES):
+            r.path.precisionFlags = prec
+            rebuilt.append(r.frame(up, scenes.terrain_boxes_camera()).bvhRebuilt)
+    finally:
+        r.close()
+    assert rebuilt == [1, 0, 0, 0]
+
+
 def test_fp16_precision_form(boxes):
     """FP16 nodes change only the order boxes are visited in, so frames are
     bit-identical to the FP32 path's; FP16 storage of the denoiser planes
