@@ -1520,7 +1520,11 @@ struct Carver
     }
 };
 
-// Scratch of the traversal's tree.
+// Scratch of the traversal's tree.  What the nodes' launch (k_pack_nodes) no
+// longer reads lies in its output buffer, nodeTris, and with a published tree
+// the boxes lie in sortedTris, which is written last: 63 bytes a triangle are
+// left of 155, and a published BVH of 1M triangles with 3 a leaf takes 390 in
+// all, not 482.
 struct TreeScratch
 {
     uint64_t *keys0, *keys1;
@@ -1535,30 +1539,33 @@ struct TreeScratch
     uint32_t* roots;
     float*    boxes;
     uint32_t* levels; // per set: nodes of each level, then its first node; one more word for the triangle count
-    size_t    bytes;
+    size_t    bytes;      // of base
+    size_t    earlyBytes; // of nodeTris, which its own contents may exceed
 
-    TreeScratch( char* base, uint32_t n, uint32_t sceneCount )
+    TreeScratch( char* base, char* nodeTris, float* sortedTris, bool view, uint32_t n, uint32_t sceneCount )
     {
-        Carver       c{ base };
         const size_t slots = n > 1 ? n - 1 : 1;
-        keys0     = c.Take< uint64_t >( n );
-        keys1     = c.Take< uint64_t >( n );
-        vals0     = c.Take< uint32_t >( n );
-        vals1     = c.Take< uint32_t >( n );
-        hist      = c.Take< uint32_t >( size_t( 256 ) * ( DivUp( n, RS_TILE ) + 1 ) );
-        children  = c.Take< uint2 >( slots );
-        rf        = c.Take< uint32_t >( slots );
-        rl        = c.Take< uint32_t >( slots );
-        bounds    = c.Take< float >( ( 2 * size_t( n ) - 1 ) * 6 );
-        info      = c.Take< uint4 >( slots );
-        lists     = c.Take< uint2 >( TreeListBytes( n ) / sizeof( uint2 ) + 1 );
-        expansion = c.Take< uint32_t >( ( slots + sceneCount ) * 8 ); // one-triangle scenes have nodes of their own
-        queue     = c.Take< uint32_t >( slots + sceneCount );
-        nodeBase  = c.Take< uint2 >( slots + sceneCount );
-        roots     = c.Take< uint32_t >( sceneCount + 1 );
-        boxes     = c.Take< float >( size_t( sceneCount + 1 ) * 8 );
-        levels    = c.Take< uint32_t >( LEVEL_WORDS * 2 + 1 );
-        bytes     = c.used;
+        Carver       e{ nodeTris };
+        keys0      = e.Take< uint64_t >( n );
+        keys1      = e.Take< uint64_t >( n );
+        vals1      = e.Take< uint32_t >( n );
+        rf         = e.Take< uint32_t >( slots );
+        rl         = e.Take< uint32_t >( slots );
+        info       = e.Take< uint4 >( slots );
+        earlyBytes = e.used;
+        Carver c{ base };
+        vals0      = c.Take< uint32_t >( n );
+        hist       = c.Take< uint32_t >( size_t( 256 ) * ( DivUp( n, RS_TILE ) + 1 ) );
+        children   = c.Take< uint2 >( slots );
+        bounds     = view ? sortedTris : c.Take< float >( ( 2 * size_t( n ) - 1 ) * 6 ); // 48 n - 24 bytes
+        lists      = c.Take< uint2 >( TreeListBytes( n ) / sizeof( uint2 ) + 1 );
+        expansion  = c.Take< uint32_t >( ( slots + sceneCount ) * 8 ); // one-triangle scenes have nodes of their own
+        queue      = c.Take< uint32_t >( slots + sceneCount );
+        nodeBase   = c.Take< uint2 >( slots + sceneCount );
+        roots      = c.Take< uint32_t >( sceneCount + 1 );
+        boxes      = c.Take< float >( size_t( sceneCount + 1 ) * 8 );
+        levels     = c.Take< uint32_t >( LEVEL_WORDS * 2 + 1 );
+        bytes      = c.used;
     }
     static constexpr uint32_t LEVEL_WORDS = ( BVH_MAX_LEVELS + 1 ) * 2;
 };
@@ -1592,9 +1599,14 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
     const uint32_t sets      = view ? 2 : 1; // set 0: the traversal's tree, set 1: the published one
     const uint32_t S         = batched ? sceneCount : 0u;
 
-    bvh.scratch.Reserve( TreeScratch( nullptr, n, S ).bytes );
-    const TreeScratch ts( bvh.scratch.as< char >(), n, S );
-    bvh.nodeTris.Reserve( size_t( n ) * 48 );
+    const TreeScratch size( nullptr, nullptr, nullptr, view, n, S );
+    bvh.scratch.Reserve( size.bytes );
+    bvh.nodeTris.Reserve( std::max( size_t( n ) * 48, size.earlyBytes ) );
+    if( view )
+    {
+        bvh.sortedTris.Reserve( size_t( n ) * 48 );
+    }
+    const TreeScratch ts( bvh.scratch.as< char >(), bvh.nodeTris.as< char >(), bvh.sortedTris.as< float >(), view, n, S );
     bvh.boundsPartials.Reserve( size_t( bndBlocks + 1 ) * 6 * 8 );
     if( !bvh.hostLevels )
     {
@@ -1602,7 +1614,6 @@ void BuildBvhImpl( BvhObject& bvh, const float* d_tris, uint32_t n, const RgExtB
     }
     if( view )
     {
-        bvh.sortedTris.Reserve( size_t( n ) * 48 );
         bvh.codes.Reserve( size_t( n ) * 8 );
         bvh.keysA.Reserve( size_t( n ) * 8 );
         bvh.keysB.Reserve( size_t( n ) * 8 );

@@ -6,6 +6,8 @@ references, primitive ids, histogram bins) must be bit-exact; FP32 outputs of
 the same IEEE operation sequence (boxes, hit t/u/v, average luminance) must be
 equal as floats.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -343,6 +345,28 @@ def test_launch_widths(gpu, n):
     for _ in range(2):  # the second launch finds the counters of the first
         _assert_same_hits(_trace_gpu(b, rays, 0), v)
         _assert_same_hits(_trace_gpu(b, rays, RG_EXT_TRACE_ANY_HIT), v, any_hit=True)
+
+
+def _free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL("libamdhip64.so.7").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_published_bvh_memory(gpu):
+    """What a published BVH keeps, per triangle: its own arrays, the
+    traversal's tree (48 and some 25 bytes) and both builds' scratch, that of
+    the traversal's tree mostly inside the arrays that are written last."""
+    n = 1_000_000
+    d = DeviceArray.from_numpy(_random_tris(n, 3, spread=300.0, size=0.5))
+    _gpu_bvh(_random_tris(4, 1))
+    b = Bvh()
+    before = _free_bytes()
+    for _ in range(2):  # a second build takes nothing more
+        b.build(d, n, 3)
+        per = (before - _free_bytes()) / n
+        print(f"published BVH: {per:.0f} bytes a triangle", flush=True)
+        assert 200 < per <= 410
 
 
 def test_histogram_bit_exact(gpu, oracle):
