@@ -107,6 +107,16 @@ struct BvhObject
 
     const uint32_t* sortedIdx = nullptr; // the published sorted order
 
+    // Gives back what only builds use, once the last one has run (a BVH that
+    // is not built again); every other member stays as it is.
+    void ReleaseBuildScratch()
+    {
+        scratch.Release();
+        boundsPartials.Release();
+        scenePartials.Release();
+        sceneBounds.Release();
+    }
+
     ~BvhObject()
     {
         if( hostLevels )

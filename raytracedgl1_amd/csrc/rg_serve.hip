@@ -742,6 +742,7 @@ RgResult rgExtSceneBuild( RgExtScene scene )
         RG_HIP_CHECK( hipStreamSynchronize( s.setup ) );
         sc.vertices.Free();
         sc.indices.Free();
+        scene->bvh.ReleaseBuildScratch(); // a scene is built once
         const size_t n = scene->ds.triCount;
         scene->bytes   = n * ( 9 + 9 + 1 + 9 ) * 4 + size_t( scene->bvh.nodeCountQ ) * sizeof( BvhNodeQ ) + n * 48;
         scene->built   = true;
@@ -822,6 +823,7 @@ RgResult rgExtSceneGroupCreate( RgExtServer server, const RgExtScene* pScenes, u
             const RgExtBvhBuildParams bp = { 1, RG_EXT_BVH_NODE_FP32 };
             BuildBvhBatch( grp->bvh, tris.as< float >(), offsets.data(), sceneCount, bp, s.setup, false );
             RG_HIP_CHECK( hipStreamSynchronize( s.setup ) );
+            grp->bvh.ReleaseBuildScratch();
         }
         catch( ... )
         {

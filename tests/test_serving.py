@@ -394,3 +394,34 @@ def test_scene_nodes_at_infinite_areas(gpu):
             srv.close()
     print(f"nodes {nodes} of {len(a.tris)} triangles", flush=True)
     assert 0 < nodes[1] <= 1.25 * nodes[0] < len(a.tris) / 2
+
+
+def _free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL("libamdhip64.so.7").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_static_scenes_keep_no_build_scratch(gpu):
+    """A scene and a scene group are built once: what they hold afterwards is
+    what the server counts (sceneBytes) and, for a scene, its vertices and
+    indices (up to 200 bytes a triangle here)."""
+    a, b = (serving.serving_scene(i, 300_000) for i in range(2))
+    n = len(a.tris) + len(b.tris)
+    srv = serving.Server(64, 64)
+    try:
+        free = [_free_bytes()]
+        handles = [srv.scene(a), srv.scene(b)]
+        free.append(_free_bytes())
+        counted = [srv.stats().sceneBytes]
+        srv.group(handles)
+        free.append(_free_bytes())
+        counted.append(srv.stats().sceneBytes - counted[0])
+    finally:
+        srv.close()
+    held = -np.diff(np.array(free, np.int64))
+    print(f"bytes a triangle: scenes {held[0] / n:.0f} ({counted[0] / n:.0f} counted), group {held[1] / n:.0f} "
+          f"({counted[1] / n:.0f} counted)", flush=True)
+    slack = 16 << 20  # allocations round up to 2 MiB
+    assert held[0] <= counted[0] + 200 * n + slack
+    assert held[1] <= counted[1] + slack
