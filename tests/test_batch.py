@@ -106,6 +106,38 @@ def test_batch_equals_single_scene_builds(gpu, fmt):
             assert (part["prim"][part["prim"] != ffi.RG_EXT_MISS] < len(t)).all()
 
 
+@pytest.mark.parametrize("fmt", [ffi.RG_EXT_BVH_NODE_FP32, ffi.RG_EXT_BVH_NODE_FP16])
+@pytest.mark.parametrize("any_hit", [0, RG_EXT_TRACE_ANY_HIT])
+def test_batch_counting_walk_equals_single_scene_builds(gpu, fmt, any_hit):
+    """With statistics a batch walks its published nodes, of either format,
+    each scene from its own root: the hits of the traversal and of the scenes'
+    own BVHs, and about the sum of their counts (a scene's Morton cells in a batch
+    are four times as long on each axis, which changes few nodes)."""
+    print(f"batched counting walk, node format {fmt}, any hit {any_hit}", flush=True)
+    sc = _scenes()
+    tris = np.concatenate([t for t, _ in sc])
+    offs = np.concatenate([[0], np.cumsum([len(t) for t, _ in sc])]).astype(np.uint32)
+    rays = [_rays(4000 + 700 * k, 50 + k, lo, hi) for k, (_, (lo, hi)) in enumerate(sc)]
+    roffs = np.concatenate([[0], np.cumsum([len(r) for r in rays])]).astype(np.uint32)
+    bb = Bvh()
+    bb.build_batch(DeviceArray.from_numpy(tris), offs, 1, fmt)
+    plain = _trace(bb, np.concatenate(rays), any_hit, roffs)
+    hits = _trace(bb, np.concatenate(rays), any_hit | RG_EXT_TRACE_COLLECT_STATS, roffs)
+    counts, single = np.array(bb.trace_stats()), np.zeros(2)
+    assert np.array_equal(hits["prim"] == ffi.RG_EXT_MISS, plain["prim"] == ffi.RG_EXT_MISS)
+    assert any_hit or np.array_equal(hits, plain)
+    for s, (t, _) in enumerate(sc):
+        b1 = Bvh()
+        b1.build(DeviceArray.from_numpy(t), len(t), 1, fmt)
+        h1 = _trace(b1, rays[s], any_hit | RG_EXT_TRACE_COLLECT_STATS)
+        single += b1.trace_stats()
+        part = hits[roffs[s]:roffs[s + 1]]
+        assert np.array_equal(part["prim"] == ffi.RG_EXT_MISS, h1["prim"] == ffi.RG_EXT_MISS), s
+        assert any_hit or np.array_equal(part, h1), s
+    print(f"  node visits and triangle tests {counts}, one by one {single}", flush=True)
+    assert (np.abs(counts - single) <= 0.02 * single).all()
+
+
 def test_autotune_keeps_results(gpu):
     print("trace autotune on a batch", flush=True)
     sc = _scenes()

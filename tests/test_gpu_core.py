@@ -209,7 +209,7 @@ def test_trace_terrain_spheres_1080p(gpu, oracle):
 
 
 def _edge_scene(kind, r):
-    """Triangles at the limits of the traversal nodes' byte grids, and their spread."""
+    """Triangles at the limits of the traversal nodes' grids, and their spread."""
     if kind.startswith("n"):  # leaves per node, and nodes of one child
         return _random_tris(int(kind[1:]), seed=int(kind[1:])), 10.0
     t = _random_tris(3000, seed=7)
@@ -230,7 +230,7 @@ def _edge_scene(kind, r):
 
 @pytest.mark.parametrize("kind", ["n1", "n2", "n7", "n8", "n9", "n15", "n57", "n500", "flat", "thin", "far", "huge", "broken"])
 def test_traversal_nodes_at_their_limits(gpu, kind):
-    """Hits through the traversal's byte-grid nodes against the walk of the
+    """Hits through the traversal's grid nodes against the walk of the
     published FP32 nodes: the same, or a hit that the FP32 boxes' rounding
     hid, nearer by rounding (1e-5 t bounds the triangle test's error) or as
     near with a lower id.  At most 1e-4 of the rays differ, but where all
@@ -266,6 +266,144 @@ def test_traversal_nodes_at_their_limits(gpu, kind):
     assert ((g["t"] < v["t"]) | ((g["t"] == v["t"]) & (g["prim"] < v["prim"])))[diff].all()
     occ = _trace_gpu(b, rays, RG_EXT_TRACE_ANY_HIT)["prim"] != RG_EXT_MISS
     assert np.array_equal(occ, g["prim"] != RG_EXT_MISS)
+
+
+def _nested_clusters():
+    """20 clusters of 64 triangles at halving distances from the origin, each
+    triangle as large as its cluster: boxes within boxes, and from the origin
+    outwards every cluster lies behind the ones nested in it."""
+    r = np.random.default_rng(3)
+    out = []
+    for k in range(20):
+        v = r.uniform(-1, 1, (64, 3, 3))
+        out.append((r.uniform(0.55, 0.95, (64, 1, 3)) + 0.4 * (v - v.mean(1, keepdims=True))) * 2.0 ** -k)
+    return np.concatenate(out).reshape(-1, 9).astype(np.float32)
+
+
+def _deepest_group_stack(b, tris, origin, direction):
+    """The traversal restated for one ray over the same keys (the scene is a
+    cube): the binary tree collapsed by area, subtrees of up to 8 triangles
+    last, and the most groups that wait on its stack."""
+    ch, bd, I = b["children"], b["bounds"], b["n"] - 1
+    size = np.ones(2 * I + 1, int)
+    order = [0]
+    for x in order:
+        order += [int(c) for c in ch[x] if c < I]
+    for x in reversed(order):
+        size[x] = size[ch[x]].sum()
+    d = bd[:, 3:] - bd[:, :3]
+    area = d[:, 0] * d[:, 1] + d[:, 1] * d[:, 2] + d[:, 2] * d[:, 0]
+
+    def children(x):
+        kids = [int(c) for c in ch[x]]
+        while True:
+            opens = [i for i, c in enumerate(kids) if c < I and size[c] > 8 and len(kids) < 8] or \
+                    [i for i, c in enumerate(kids) if c < I and size[c] - 1 <= 8 - len(kids)]
+            if not opens:
+                return kids
+            i = max(opens, key=lambda i: area[kids[i]])
+            kids[i:i + 1] = [int(c) for c in ch[kids[i]]]
+
+    best, stack, group, deepest = np.inf, [], [0], 0
+    while group or stack:
+        if not group:
+            group = stack.pop()
+        hit = []
+        for c in children(group.pop(0)):
+            t = (bd[c].reshape(2, 3) - origin) / direction
+            near, far = max(t.min(0).max(), 0.0), min(t.max(0).min(), best)
+            if near <= far and c < I:
+                hit.append((near, c))
+            elif near <= far:
+                p = tris[b["sorted_idx"][c - I]].reshape(3, 3).astype(np.float64)
+                m = np.stack([p[1] - p[0], p[2] - p[0], -direction], 1)
+                u, v, t = np.linalg.solve(m, origin - p[0])
+                best = t if u >= 0 and v >= 0 and u + v <= 1 and 0 <= t < best else best
+        if hit:
+            if group:
+                stack.append(group)
+                deepest = max(deepest, len(stack))
+            group = [c for _, c in sorted(hit)]
+    return deepest
+
+
+def test_traversal_stack_beyond_lds(gpu, oracle):
+    """Rays that leave more groups waiting than the stack has in LDS (8, 12 or
+    16 of them by the tuning, 12 of 32 in the variant without allocations):
+    the rest goes through global memory.  Against the oracle's walk, whose
+    stack has no end (these rays need up to 140 entries of one child each)."""
+    tris = _nested_clusters()
+    r = np.random.default_rng(1)
+    n = 40000
+    rays = np.zeros(n, RAY_DTYPE)
+    rays["origin"] = 1e-7
+    d = r.uniform(0.6, 1.4, (n, 3))
+    rays["direction"] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    rays["tmax"] = 100.0
+    o = oracle.bvh(tris, 1)
+    ob = o.download()
+    deep = [_deepest_group_stack(ob, tris, np.full(3, 1e-7), rays["direction"][k].astype(np.float64)) for k in range(20)]
+    print(f"groups on the stack: {min(deep)} to {max(deep)}", flush=True)
+    assert 17 <= max(deep) <= 32
+    b, _ = _gpu_bvh(tris, 1)
+    v = o.trace(rays, 0)
+    assert (v["prim"] != RG_EXT_MISS).mean() > 0.5
+    dr, dh = DeviceArray.from_numpy(rays), DeviceArray(n, HIT_DTYPE)
+    for _ in range(6):
+        _assert_same_hits(_trace_gpu(b, rays, 0), v)
+        _assert_same_hits(_trace_gpu(b, rays, RG_EXT_TRACE_ANY_HIT), v, any_hit=True)
+        for flags in (0, RG_EXT_TRACE_ANY_HIT):
+            ffi.call("rgExtTraceRaysNoAlloc", b.h, dr.ptr, n, dh.ptr, flags, None)
+            _assert_same_hits(dh.download(), v, any_hit=bool(flags))
+            assert b.trace_errors() == 0
+        print(f"  next: {b.autotune(dr, n, dh).stackLdsEntries} words in LDS", flush=True)
+
+
+@pytest.mark.parametrize("kind", ["n9", "n57", "n500", "flat", "thin", "far", "huge", "broken"])
+def test_traversal_nodes_against_a_loop_over_all_triangles(gpu, oracle, kind):
+    """The same scenes against the FP64 loop, with rays at the middle of a
+    triangle from outside the plane of flat scenes: a ray that hits a triangle
+    there hits it or a nearer one."""
+    print(f"loop over all triangles {kind}", flush=True)
+    r = np.random.default_rng(29)
+    tris, spread = _edge_scene(kind, r)
+    n = 5000
+    good = np.flatnonzero(np.isfinite(tris).all(1))
+    scale = max(1.0, np.abs(tris[good]).max() if kind == "huge" else spread)
+    t = tris[good[r.integers(0, len(good), n)]].reshape(n, 3, 3).astype(np.float64)
+    target = (t * r.dirichlet([8, 8, 8], n)[..., None]).sum(1)
+    nrm = np.cross(t[:, 1] - t[:, 0], t[:, 2] - t[:, 0])
+    nrm /= np.maximum(np.linalg.norm(nrm, axis=1, keepdims=True), 1e-300)
+    d = nrm * r.choice([-1.0, 1.0], (n, 1)) + r.normal(size=(n, 3)) * 0.3
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    rays = np.zeros(n, RAY_DTYPE)
+    rays["origin"] = target - d * (r.uniform(0.5, 3.0, (n, 1)) * scale)
+    rays["direction"] = d
+    rays["tmax"] = 100.0 * scale
+    tb, _, _, p = oracle.bruteforce(tris[good], rays)
+    hit = p != RG_EXT_MISS
+    p = np.where(hit, good[np.where(hit, p, 0)], RG_EXT_MISS)
+    assert hit.mean() > 0.9
+    v = tris[np.where(hit, p, good[0])].reshape(n, 3, 3).astype(np.float64)
+    nrm = np.cross(v[:, 1] - v[:, 0], v[:, 2] - v[:, 0])
+    cos = np.abs((nrm * d).sum(1)) / np.maximum(np.linalg.norm(nrm, axis=1), 1e-300)
+    b, _ = _gpu_bvh(tris, 1)
+    g = _trace_gpu(b, rays, 0)
+    same = g["prim"] == p
+    # One flat plane of overlapping triangles: any of those within rounding may
+    # be the nearest.  Else a ray meets another triangle only at an edge.
+    if kind not in ("flat", "thin"):
+        assert (g["prim"] == p).mean() >= 0.999
+    assert np.array_equal(g["prim"] != RG_EXT_MISS, hit)
+    # A ray is placed on the triangle within a few roundings of its distance or
+    # of the triangle's size, and the depth there by weights off by as much over the
+    # triangle's height: across the plane 8 roundings times the aspect, along the
+    # ray over the cosine.
+    edge = np.linalg.norm(v - np.roll(v, 1, 1), axis=2).max(1)
+    aspect = edge ** 2 / np.maximum(np.linalg.norm(np.cross(v[:, 1] - v[:, 0], v[:, 2] - v[:, 0]), axis=1), 1e-300)
+    err = (np.abs(g["t"] - tb) * cos / (np.maximum(np.abs(tb), edge) * aspect))[hit]
+    print(f"  error at most {err.max() * 2.0 ** 24:.1f} roundings", flush=True)
+    assert err.max() <= 8 * 2.0 ** -24
 
 
 def _grid_wall():

@@ -31,8 +31,8 @@ def test_no_alloc_trace_equals_trace(gpu, fmt):
     b = Bvh()
     b.build(DeviceArray.from_numpy(np.ascontiguousarray(s.tris, np.float32)), len(s.tris), 3, fmt)
     big, small = _rays()
-    for flags in (ffi.RG_EXT_TRACE_COLLECT_STATS, ffi.RG_EXT_TRACE_ANY_HIT | ffi.RG_EXT_TRACE_COLLECT_STATS,
-                  ffi.RG_EXT_TRACE_CULL_FRONT_FACE):
+    for flags in (0, ffi.RG_EXT_TRACE_ANY_HIT, ffi.RG_EXT_TRACE_COLLECT_STATS,
+                  ffi.RG_EXT_TRACE_ANY_HIT | ffi.RG_EXT_TRACE_COLLECT_STATS, ffi.RG_EXT_TRACE_CULL_FRONT_FACE):
         for rays in (big, small):  # the second call has fewer rays
             print(f"no-alloc trace: node format {fmt}, flags {flags}, {len(rays)} rays", flush=True)
             dr = DeviceArray.from_numpy(rays)
@@ -45,8 +45,9 @@ def test_no_alloc_trace_equals_trace(gpu, fmt):
             _no_alloc(b, dr, len(rays), got, flags)
             h = got.download()
             assert b.trace_errors() == 0
-            for f in ("prim", "t", "u", "v"):
+            for f in ("prim", "t", "u", "v") if flags != ffi.RG_EXT_TRACE_ANY_HIT else ():
                 assert np.array_equal(h[f], want[f]), (fmt, flags, len(rays), f)
+            assert np.array_equal(h["prim"] == ffi.RG_EXT_MISS, want["prim"] == ffi.RG_EXT_MISS)
             # front-face culling leaves the back faces only
             assert (h["prim"] != ffi.RG_EXT_MISS).mean() > (0.1 if flags & ffi.RG_EXT_TRACE_CULL_FRONT_FACE else 0.5)
             if want_stats is not None:
