@@ -239,6 +239,7 @@ struct Instance
             // both are of published nodes; frames walk the traversal's tree,
             // which has one triangle per leaf slot and one node format
             RgExtBvhBuildParams bp = { 1, RG_EXT_BVH_NODE_FP32 };
+            dscene.bvhValid = false; // a build that throws is tried again by the next frame
             BuildFrameBvh( bvh, dscene.tris.as< float >(), dscene.classTris, GC_COUNT, bp, s );
             dscene.bvhValid      = true;
             dscene.builtTriCount = dscene.triCount;
