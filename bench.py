@@ -588,6 +588,8 @@ def main(argv=None) -> int:
             "peak": HBM_PEAK_GBPS,
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBPS,
+            "frac_of": "algorithmic work rate over the HBM peak (most node reads hit L2); the HBM traffic's share is "
+                       "measured.hbm_frac, the limiter measured.valu_issue",
             "traffic": traffic,
             "algorithmic_bytes_per_launch": alg_bytes / launches,
             "avg_launch_ms": trav_ms / launches,

@@ -45,7 +45,8 @@ static_assert( sizeof( BvhNode8H ) == 144, "node size" );
 
 // The traversal's node, one 128-byte cache line: eight child boxes as whole
 // numbers on a grid of the node's own (origin + q * 2^k per axis, rounded
-// outward), child nodes in the first slots (slot s is node childBase + s),
+// outward; the idea of Ylitie, Karras, Laine, "Efficient Incoherent Ray
+// Traversal on GPUs Through Compressed Wide BVHs", HPG 2017), child nodes in the first slots (slot s is node childBase + s),
 // then leaves of one triangle each (slot s is triangle triBase + s), so that
 // neither a sort key nor the stack needs a child reference.  The numbers are
 // halves (exact to 2048): a plane's distance is then one mixed-precision

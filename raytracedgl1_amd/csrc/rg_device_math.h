@@ -302,5 +302,4 @@ RG_HD float rgExp2( float x )
     std::memcpy( &s2, &b2, 4 );
     return ( p * s1 ) * s2;
 }
-
 } // namespace rg

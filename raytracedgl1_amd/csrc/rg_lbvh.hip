@@ -315,10 +315,6 @@ __global__ __launch_bounds__( THREADS ) void k_scene_roots( uint32_t internal, c
     }
 }
 
-// Seeds a collapse with every scene root.  A one-triangle scene (frame
-// segments only) has no internal node: the published tree leaves it out, the
-// traversal's tree gives it a node of one leaf, so that scene s's root is
-// its node s.  With boxes: each root's box (lo xyz, hi xyz, 2 unused).
 // The words a build starts from: the collapse's level counts at 0, the node
 // flags at 0 and the scene roots at none; one launch for what were up to
 // four memsets of two kernels each.
@@ -346,6 +342,10 @@ __global__ __launch_bounds__( THREADS ) void k_build_init( uint32_t* levels, uin
     }
 }
 
+// Seeds a collapse with every scene root.  A one-triangle scene (frame
+// segments only) has no internal node: the published tree leaves it out, the
+// traversal's tree gives it a node of one leaf, so that scene s's root is
+// its node s.  With boxes: each root's box (lo xyz, hi xyz, 2 unused).
 __global__ void k_seed_frontier_seg( const uint32_t* roots, uint32_t S, const uint32_t* offsets, uint32_t internal, bool leaves, uint32_t* queue,
                                      uint32_t* counts, const float* bounds, float* boxes )
 {

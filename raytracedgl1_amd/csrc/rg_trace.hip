@@ -14,7 +14,9 @@
 //
 // k_trace walks the traversal's tree (BvhNodeQ): a node visit is eight
 // loads of one cache line, eight boxes of one multiply-add per plane, and a
-// sort of 32-bit keys whose low bits are the child's slot.  A node's hit
+// sort of 32-bit keys whose low bits are the child's slot (distances behind
+// the ray's origin, which only a negative tmin lets in, come last and in
+// reverse: an order, not the result).  A node's hit
 // leaves are tested before its child nodes; the child nodes left over are one
 // group of two words on a stack that is short in LDS (12 groups by default,
 // interleaved by lane) and goes on in global memory.
