@@ -318,7 +318,7 @@ def serving_run(a) -> dict:
             "sessions_requested": a.serving_sessions, "sessions_admitted": len(sessions), "sessions_refused": refused,
             "scenes": len(handles), "scene_triangles": [int(c) for c in counts], "mean_mpix_per_session": mpx,
             "memory_budget_gib": 200, "session_gib": st.sessionBytes / 2**30, "shared_gib": st.sharedBytes / 2**30,
-            "scene_gib": st.sceneBytes / 2**30, "streams": st.streams, "precision": "fp16 storage + fp16 nodes",
+            "scene_gib": st.sceneBytes / 2**30, "streams": st.streams, "precision": "fp16 storage (the node flag set too: no effect)",
             "readback": "FINAL as RGBA8 (sRGB) to pinned host memory; latency ends when the copy is done",
             "request_rate_hz_per_session": 30.0, **runs, "sustainable_load": light,
         }
